@@ -139,7 +139,9 @@ inline PatchLayout patch_layout(uint32_t vmax, uint32_t imax, uint32_t cmax)
 	L.off = take((vmax + 2) * 2);
 	L.adj = take(imax * 4);
 	// the sort's ping-pong half and digit counts (64 offsets + 64 counts per wavefront)
-	L.sortbuf = take(align16(cmax * 2) + (1 + kBatchWaves) * 64 * 4);
+	// (commit keeps a 64-bit lane mask per vertex there; the sort needs as much in nearly every layout)
+	const uint32_t sort_bytes = align16(cmax * 2) + (1 + kBatchWaves) * 64 * 4;
+	L.sortbuf = take(sort_bytes > vmax * 8 ? sort_bytes : vmax * 8);
 	// one region for uses whose lifetimes do not overlap: the candidate arrays (pick to commit)
 	// and the scratch of setup (position hash, wedge maxima), of build_adjacency (cursor, corner
 	// ids; the ordered welded corners live on through the quadrics) and of the edge-loop update
@@ -213,6 +215,13 @@ __device__ __forceinline__ Quad QL(const PatchSmem& s, uint32_t v)
 __device__ __forceinline__ void QS(const PatchSmem& s, uint32_t v, const Quad& q)
 {
 	store_quad(s.gq, v, q);
+}
+
+// orders the wavefront's own LDS accesses before it against those after it
+__device__ __forceinline__ void wave_fence()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
 }
 
 // exclusive scan of one value per thread across the workgroup; `part` holds kBatchThreads/64 words
@@ -1163,45 +1172,46 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 		}
 
 		PROFILE_PHASE(6);
-		// greedy commit (src/simplifier.cpp:1498-1636) on wavefront 0, 64 ranks at a time: every
-		// lane loads one candidate and evaluates its lock state, its commit targets and its flip
-		// test against the collapse_remap of the chunk start; the lanes are then resolved in rank
-		// order with scalar state, exactly as the sequential loop decides them.  A lane's flip
-		// result can only change if an earlier commit of the same chunk moved one of the welded
-		// neighbours its test reads (the source class of that commit); each lane keeps its first
-		// kNearSlots adjacency entries in registers to detect this exactly, and re-runs the test
-		// on the current collapse_remap only then.
+		// greedy commit (src/simplifier.cpp:1498-1636) on wavefront 0, 64 ranks at a time, one per
+		// lane.  What a rank decides hangs on the lower ranks of its chunk that share an endpoint
+		// class with it (the lock test) or whose source class its flip test reads (a commit moves its
+		// source and nothing else); those of earlier chunks are decided.  Each lane collects the two
+		// as lane masks through a per-vertex word of LDS, and the chunk is then decided in rounds:
+		// every lane with no undecided lane in its masks takes its flip test on the current
+		// collapse_remap and commits or rejects.  The lowest undecided lane always can, and both
+		// relations are symmetric (a lane waits for every lower one that could see its move), so each
+		// lane sees exactly what the sequential loop shows it.  The loop's breaks are tested on the
+		// decided chunk with prefix counts, and the commits past the first break are taken back (they
+		// wrote their own source classes only).
+		//
+		// Bound by the latency of one wavefront's LDS and ballot chains; a chunk takes 4-8 rounds
+		// where one rank at a time took 15-20 decisions.  4096 patches of 64-512 triangles: @COMMIT@.
+		uint64_t* const tab = (uint64_t*)s.sortbuf; // the sort's half: one word per vertex, zero between chunks
 		for (uint32_t v = tid; v < V; v += kBatchThreads)
 		{
 			s.cremap[v] = (uint16_t)v;
 			s.lock[v] = 0;
+			tab[v] = 0;
 		}
 		__syncthreads();
 		if (tid < 64)
 		{
 			constexpr int kNearSlots = 8;
 			const uint32_t lane = tid;
+			const uint64_t bit = 1ull << lane, below = bit - 1;
 			const uint32_t goal = (result_count - target) / 3;
 			uint32_t edge_goal = goal / 2;
-			// cerr of the sorted candidates edge_goal .. edge_goal + 63, one per lane: the error
-			// goal follows edge_goal one step per rejection and is read from this window
-			uint32_t gbase = edge_goal;
-			float gwin = gbase + lane < C ? s.cerr[s.order[gbase + lane]] : 0.f;
-			float error_goal = edge_goal < C ? 1.5f * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gwin), 0)) : FLT_MAX;
 			uint32_t tri_collapses = 0, committed = 0, evaluated = 0;
+			uint32_t best = 0; // bits of the largest error among this lane's commits
 			bool stop = false;
 			for (uint32_t base = 0; base < C && !stop; base += 64)
 			{
 				PROFILE_PHASE(15);
 				PROFILE_COUNT(24, 1);
 				const uint32_t k = base + lane;
-				uint32_t i0 = 0, i1 = 0, r0 = kNone16, r1 = kNone16, s0 = kNone16, s1 = 0, ab = 0, ae = 0;
+				uint32_t i0 = 0, i1 = 0, r0 = 0, r1 = 0, s0 = kNone16, s1 = 0, ab = 0, ae = 0;
 				float err = 0.f;
-				bool locked = true, flips = false, border = false, complex = false;
-				uint32_t near[kNearSlots];
-#pragma unroll
-				for (int q = 0; q < kNearSlots; ++q)
-					near[q] = 0xffffffffu; // 0xffff never equals a vertex id
+				bool open = false, border = false, complex = false;
 				if (k < C)
 				{
 					const uint32_t c = s.order[k];
@@ -1210,11 +1220,11 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 					err = s.cerr[c];
 					r0 = s.remap[i0];
 					r1 = s.remap[i1];
-					locked = (s.lock[r0] | s.lock[r1]) != 0;
+					open = (s.lock[r0] | s.lock[r1]) == 0;
 					const uint8_t kd = s.kind[i0];
 					border = kd == kBorder;
 					complex = kd == kComplex;
-					if (kd == kSeam)
+					if (open && kd == kSeam)
 					{
 						s0 = s.wedge[i0];
 						uint32_t t = s.loop[i0] == i1 ? s.loopback[s0] : s.loop[s0];
@@ -1222,104 +1232,88 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 					}
 					ab = s.off[r0];
 					ae = s.off[r0 + 1];
-					if (!locked)
-					{
-						// hasTriangleFlips (src/simplifier.cpp:1200-1232); a boolean OR over the
-						// corners, evaluated without early exit so the loads overlap
-						const V3 v0 = P(s, r0), v1 = P(s, r1);
+				}
+				// flip: the lower lanes whose source the flip test reads; share: those that share an
+				// endpoint class
+				uint64_t flip = 0, share = 0;
+				if (open)
+					atomicOr((unsigned long long*)&tab[r0], (unsigned long long)bit);
+				wave_fence();
+				if (open)
+				{
 #pragma unroll
-						for (int q = 0; q < kNearSlots; ++q)
+					for (int q = 0; q < kNearSlots; ++q)
+						if (ab + q < ae)
 						{
-							if (ab + q < ae)
-							{
-								const uint32_t ad = s.adj[ab + q];
-								near[q] = ad;
-								const uint32_t a2 = s.cremap[ad & 0xffffu], b2 = s.cremap[ad >> 16];
-								if (!(a2 == r1 || b2 == r1 || a2 == b2))
-									flips |= triangle_flips(P(s, a2), P(s, b2), v0, v1);
-							}
+							const uint32_t ad = s.adj[ab + q];
+							flip |= tab[ad & 0xffffu] | tab[ad >> 16];
 						}
-						for (uint32_t p = ab + kNearSlots; p < ae; ++p)
-						{
-							const uint32_t ad = s.adj[p];
-							const uint32_t a2 = s.cremap[ad & 0xffffu], b2 = s.cremap[ad >> 16];
-							if (!(a2 == r1 || b2 == r1 || a2 == b2))
-								flips |= triangle_flips(P(s, a2), P(s, b2), v0, v1);
-						}
+					for (uint32_t p = ab + kNearSlots; p < ae; ++p)
+					{
+						const uint32_t ad = s.adj[p];
+						flip |= tab[ad & 0xffffu] | tab[ad >> 16];
 					}
 				}
-				uint64_t lock_mask = __ballot(locked);
-				const uint64_t flip_mask = __ballot(flips);
-				// lanes whose corners do not all fit the register slots count as stale after any commit
-				const uint64_t wide_mask = __ballot(ae - ab > (uint32_t)kNearSlots);
-				uint64_t stale_mask = 0;
-				const uint32_t n = C - base < 64 ? C - base : 64;
-				const uint64_t valid = n == 64 ? ~0ull : (1ull << n) - 1;
-				PROFILE_PHASE(14);
-				// the stop test of every lane at the current scalar state; that state changes only on
-				// a rejection or a commit, so the locked candidates between two such events are
-				// passed over by one scan of the masks (they change nothing but the evaluated count)
-				uint64_t stop_mask = __ballot(err > error_limit || tri_collapses >= goal || (err > error_goal && err > result_error && tri_collapses > goal / 6));
-				for (uint32_t j = 0; j < n; ++j)
+				wave_fence();
+				if (open)
+					atomicOr((unsigned long long*)&tab[r1], (unsigned long long)bit);
+				wave_fence();
+				if (open)
+					share = (tab[r0] | tab[r1]) & below;
+				wave_fence();
+				if (open)
 				{
-					const uint64_t events = (stop_mask | ~lock_mask) & valid & (~0ull << j);
-					if (!events)
+					tab[r0] = 0;
+					tab[r1] = 0;
+				}
+				const uint64_t deps = (flip & below) | share;
+				const uint32_t ends = r0 | (r1 << 16), span = ab | (ae << 16);
+				uint64_t undecided = __ballot(open), commits = 0, rejects = 0;
+				PROFILE_PHASE(14);
+				while (undecided)
+				{
+					undecided &= ~__ballot((share & commits) != 0);
+					const uint64_t ready = undecided & __ballot((deps & undecided) == 0);
+					uint64_t flips = 0;
+					// flip tests (hasTriangleFlips, src/simplifier.cpp:1200-1232) of eight lanes at a
+					// time, eight adjacency entries of each
+					for (uint64_t left = ready; left;)
 					{
-						evaluated += n - j;
-						break;
-					}
-					const uint32_t jn = (uint32_t)__builtin_ctzll(events);
-					evaluated += jn - j + 1;
-					j = jn;
-					if ((stop_mask >> j) & 1)
-					{
-						stop = true;
-						break;
-					}
-					const float ej = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(err), j));
-					const uint32_t r0j = __builtin_amdgcn_readlane(r0, j), r1j = __builtin_amdgcn_readlane(r1, j);
-					bool fj = (flip_mask >> j) & 1;
-					if ((stale_mask >> j) & 1)
-					{
-						// re-run on the current collapse_remap, one adjacency entry per lane
 						PROFILE_COUNT(25, 1);
-						PROFILE_PHASE(15);
-						fj = false;
-						const uint32_t b = __builtin_amdgcn_readlane(ab, j), e = __builtin_amdgcn_readlane(ae, j);
-						const V3 v0 = P(s, r0j), v1 = P(s, r1j);
-						for (uint32_t p0 = b; p0 < e; p0 += 64)
+						const uint32_t slot = (uint32_t)__popcll(left & below); // this lane's place among those left
+						uint64_t rest = left;
+						uint32_t from = 64;
+#pragma unroll
+						for (uint32_t q = 0; q < 8; ++q)
+							if (rest)
+							{
+								const uint32_t l = (uint32_t)__builtin_ctzll(rest);
+								from = (lane >> 3) == q ? l : from;
+								rest &= rest - 1;
+							}
+						const uint32_t fe = __shfl(ends, (int)(from & 63), 64), fs = __shfl(span, (int)(from & 63), 64);
+						const uint32_t q1 = fe >> 16, e = from < 64 ? fs >> 16 : 0;
+						uint32_t p = (fs & 0xffffu) + (lane & 7);
+						const V3 v0 = P(s, fe & 0xffffu), v1 = P(s, q1);
+						bool f = false;
+						while (__ballot(p < e))
 						{
-							const uint32_t p = p0 + lane;
-							bool f = false;
 							if (p < e)
 							{
 								const uint32_t ad = s.adj[p];
 								const uint32_t a2 = s.cremap[ad & 0xffffu], b2 = s.cremap[ad >> 16];
-								if (!(a2 == r1j || b2 == r1j || a2 == b2))
-									f = triangle_flips(P(s, a2), P(s, b2), v0, v1);
+								if (!(a2 == q1 || b2 == q1 || a2 == b2))
+									f |= triangle_flips(P(s, a2), P(s, b2), v0, v1);
 							}
-							if (__ballot(f))
-							{
-								fj = true;
-								break;
-							}
+							p += 8;
 						}
-						PROFILE_PHASE(16);
+						const uint64_t found = __ballot(f);
+						flips |= __ballot((left & bit) != 0 && slot < 8 && ((found >> (8 * (slot & 7))) & 0xffu) != 0);
+						left = rest;
 					}
-					if (fj)
-					{
-						edge_goal++;
-						if (edge_goal - gbase >= 64)
-						{
-							gbase = edge_goal;
-							gwin = gbase + lane < C ? s.cerr[s.order[gbase + lane]] : 0.f;
-						}
-						error_goal = edge_goal < C ? 1.5f * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(gwin), edge_goal - gbase)) : FLT_MAX;
-						stop_mask = __ballot(err > error_limit || tri_collapses >= goal || (err > error_goal && err > result_error && tri_collapses > goal / 6));
-						continue;
-					}
-					// commit (src/simplifier.cpp:1573-1611) from the candidate's own lane
-					if (lane == j)
+					// commits (src/simplifier.cpp:1573-1611) from the candidates' own lanes
+					const uint64_t now = ready & ~flips;
+					if (now & bit)
 					{
 						if (complex)
 						{
@@ -1339,21 +1333,86 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 						s.lock[r0] = 1;
 						s.lock[r1] = 1;
 					}
-					// the writes are read by later stale re-runs and by the next chunk's loads
-					__builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-					__builtin_amdgcn_wave_barrier();
-					lock_mask |= __ballot(r0 == r0j || r0 == r1j || r1 == r0j || r1 == r1j);
-					bool moved = false;
-#pragma unroll
-					for (int q = 0; q < kNearSlots; ++q)
-						moved |= (near[q] & 0xffffu) == r0j || (near[q] >> 16) == r0j;
-					stale_mask |= __ballot(moved) | wide_mask;
-					tri_collapses += __builtin_amdgcn_readlane((int)border, j) ? 1 : 2;
-					committed++;
-					result_error = result_error < ej ? ej : result_error;
-					stop_mask = __ballot(err > error_limit || tri_collapses >= goal || (err > error_goal && err > result_error && tri_collapses > goal / 6));
+					wave_fence();
+					commits |= now;
+					rejects |= flips;
+					undecided &= ~ready;
 				}
+				PROFILE_PHASE(16);
+				// the breaks (src/simplifier.cpp:1517-1539), each rank against the state before it
+				const uint64_t borders = __ballot(border);
+				const uint32_t tri = tri_collapses + 2 * (uint32_t)__popcll(commits & below) - (uint32_t)__popcll(commits & borders & below);
+				const uint32_t eg = edge_goal + (uint32_t)__popcll(rejects & below);
+				const float error_goal = eg < C ? 1.5f * s.cerr[s.order[eg]] : FLT_MAX;
+				const bool plain_break = k < C && (err > error_limit || tri >= goal);
+				bool goal_break = k < C && err > error_goal && err > result_error && tri > goal / 6;
+				if (__ballot(goal_break))
+				{
+					// against the largest error committed below: the earlier chunks' and this one's
+					uint32_t x = best;
+#pragma unroll
+					for (int o = 32; o > 0; o >>= 1)
+					{
+						const uint32_t t = __shfl_xor(x, o, 64);
+						x = t > x ? t : x;
+					}
+					uint32_t m = (commits & bit) && err == err ? __float_as_uint(err) : 0u;
+#pragma unroll
+					for (int o = 1; o < 64; o <<= 1)
+					{
+						const uint32_t t = __shfl_up(m, o, 64);
+						m = lane >= (uint32_t)o && t > m ? t : m;
+					}
+					const uint32_t prev = __shfl_up(m, 1, 64);
+					x = lane && prev > x ? prev : x;
+					goal_break = goal_break && err > __uint_as_float(x);
+				}
+				const uint64_t stops = __ballot(plain_break || goal_break);
+				uint64_t kept = ~0ull;
+				if (stops)
+				{
+					const uint32_t at = (uint32_t)__builtin_ctzll(stops);
+					stop = true;
+					evaluated += at + 1;
+					kept = (1ull << at) - 1;
+					if (commits & ~kept & bit)
+					{
+						if (complex)
+						{
+							uint32_t v = i0;
+							do
+							{
+								s.cremap[v] = (uint16_t)v;
+								v = s.wedge[v];
+							} while (v != i0);
+						}
+						else
+						{
+							s.cremap[i0] = (uint16_t)i0;
+							if (s0 != kNone16)
+								s.cremap[s0] = (uint16_t)s0;
+						}
+					}
+				}
+				else
+					evaluated += C - base < 64 ? C - base : 64;
+				commits &= kept;
+				if ((commits & bit) && err == err)
+				{
+					const uint32_t e = __float_as_uint(err);
+					best = e > best ? e : best;
+				}
+				tri_collapses += 2 * (uint32_t)__popcll(commits) - (uint32_t)__popcll(commits & borders);
+				edge_goal += (uint32_t)__popcll(rejects);
+				committed += (uint32_t)__popcll(commits);
 			}
+#pragma unroll
+			for (int o = 32; o > 0; o >>= 1)
+			{
+				const uint32_t t = __shfl_xor(best, o, 64);
+				best = t > best ? t : best;
+			}
+			result_error = result_error < __uint_as_float(best) ? __uint_as_float(best) : result_error;
 			if (lane == 0)
 			{
 				sh[4] = evaluated;

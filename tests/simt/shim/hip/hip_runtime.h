@@ -106,6 +106,7 @@ inline T readlane(T v, unsigned int j, int line)
 #define __syncthreads() ::simt::block_barrier(__LINE__)
 #define __shfl_up(v, d, w) ::simt::shfl_up((v), (d), __LINE__)
 #define __shfl_xor(v, m, w) ::simt::shfl_xor((v), (m), __LINE__)
+#define __shfl(v, j, w) ::simt::readlane((v), (unsigned int)(j), __LINE__)
 #define __ballot(p) ::simt::ballot((p), __LINE__)
 #define __builtin_amdgcn_readlane(v, j) ::simt::readlane((v), (j), __LINE__)
 // every fiber of the wavefront must reach it (all lanes are active in this model: lane 0 is first)
@@ -128,5 +129,6 @@ inline unsigned int atomicOr(unsigned int* p, unsigned int v) { unsigned int o =
 inline unsigned int atomicMax(unsigned int* p, unsigned int v) { unsigned int o = *p; *p = o > v ? o : v; return o; }
 inline unsigned int atomicMin(unsigned int* p, unsigned int v) { unsigned int o = *p; *p = o < v ? o : v; return o; }
 inline unsigned int atomicCAS(unsigned int* p, unsigned int cmp, unsigned int v) { unsigned int o = *p; if (o == cmp) *p = v; return o; }
+inline unsigned long long atomicOr(unsigned long long* p, unsigned long long v) { unsigned long long o = *p; *p = o | v; return o; }
 inline unsigned long long atomicMax(unsigned long long* p, unsigned long long v) { unsigned long long o = *p; *p = o > v ? o : v; return o; }
 inline unsigned long long atomicMin(unsigned long long* p, unsigned long long v) { unsigned long long o = *p; *p = o < v ? o : v; return o; }
