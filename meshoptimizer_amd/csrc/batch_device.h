@@ -97,7 +97,7 @@ __device__ unsigned long long g_batch_profile[32];
 struct PatchLayout
 {
 	uint32_t vmax, imax, cmax;
-	uint32_t ib, px, py, pz, remap, wedge, loop, loopback, cremap, kind, lock, off, adj, sortbuf, region, cv0, cv1, order, cerr, total;
+	uint32_t ib, pos, remap, wedge, loop, loopback, cremap, kind, lock, off, adj, sortbuf, region, cv0, cv1, order, cerr, total;
 };
 
 inline uint32_t align16(uint32_t x)
@@ -126,9 +126,7 @@ inline PatchLayout patch_layout(uint32_t vmax, uint32_t imax, uint32_t cmax)
 		return at;
 	};
 	L.ib = take(imax * 2);
-	L.px = take(vmax * 4);
-	L.py = take(vmax * 4);
-	L.pz = take(vmax * 4);
+	L.pos = take(vmax * 12);
 	L.remap = take(vmax * 2);
 	L.wedge = take(vmax * 2);
 	L.loop = take(vmax * 2);
@@ -165,7 +163,8 @@ inline PatchLayout patch_layout(uint32_t vmax, uint32_t imax, uint32_t cmax)
 struct PatchSmem
 {
 	uint16_t *ib, *remap, *wedge, *loop, *loopback, *cremap, *off, *cv0, *cv1, *order, *sortbuf;
-	float *px, *py, *pz, *cerr;
+	float* cerr;
+	V3* pos;
 	Quad* gq; // the mesh's vertex quadrics in global memory (read and written by this workgroup only)
 	uint8_t *kind, *lock;
 	uint32_t* adj; // next | prev << 16
@@ -177,9 +176,7 @@ __device__ __forceinline__ PatchSmem bind(uint8_t* base, const PatchLayout& L)
 {
 	PatchSmem s;
 	s.ib = (uint16_t*)(base + L.ib);
-	s.px = (float*)(base + L.px);
-	s.py = (float*)(base + L.py);
-	s.pz = (float*)(base + L.pz);
+	s.pos = (V3*)(base + L.pos);
 	s.remap = (uint16_t*)(base + L.remap);
 	s.wedge = (uint16_t*)(base + L.wedge);
 	s.loop = (uint16_t*)(base + L.loop);
@@ -204,7 +201,7 @@ __device__ __forceinline__ PatchSmem bind(uint8_t* base, const PatchLayout& L)
 
 __device__ __forceinline__ V3 P(const PatchSmem& s, uint32_t i)
 {
-	return V3{s.px[i], s.py[i], s.pz[i]};
+	return s.pos[i];
 }
 
 __device__ __forceinline__ Quad QL(const PatchSmem& s, uint32_t v)
@@ -215,6 +212,18 @@ __device__ __forceinline__ Quad QL(const PatchSmem& s, uint32_t v)
 __device__ __forceinline__ void QS(const PatchSmem& s, uint32_t v, const Quad& q)
 {
 	store_quad(s.gq, v, q);
+}
+
+// the thread's id as a value that the compiler cannot see through: what is computed from it stays
+// where it is used instead of being hoisted out of the pass loop, where a dozen such addresses
+// took registers that spilled to scratch
+__device__ __forceinline__ int thread_id()
+{
+	int t = (int)threadIdx.x;
+#ifdef __HIP_DEVICE_COMPILE__
+	asm volatile("" : "+v"(t));
+#endif
+	return t;
 }
 
 // orders the wavefront's own LDS accesses before it against those after it
@@ -261,17 +270,18 @@ template <typename KeyOf>
 __device__ void segment_items(uint16_t* off, uint16_t* items, uint32_t n, uint32_t count, KeyOf key_of, uint32_t* cursor, uint32_t* part,
                               bool ordered)
 {
-	for (uint32_t v = threadIdx.x; v <= n; v += kBatchThreads)
+	const uint32_t tid = (uint32_t)thread_id();
+	for (uint32_t v = tid; v <= n; v += kBatchThreads)
 		cursor[v] = 0;
 	__syncthreads();
-	for (uint32_t i = threadIdx.x; i < count; i += kBatchThreads)
+	for (uint32_t i = tid; i < count; i += kBatchThreads)
 		atomicAdd(&cursor[key_of(i)], 1u);
 	__syncthreads();
 	// exclusive scan of cursor[0..n) (n <= a few thousand): chunks of kBatchThreads
 	uint32_t carry = 0;
 	for (uint32_t base = 0; base < n; base += kBatchThreads)
 	{
-		uint32_t v = base + threadIdx.x;
+		uint32_t v = base + tid;
 		uint32_t c = v < n ? cursor[v] : 0;
 		uint32_t tot;
 		uint32_t ex = wg_scan(c, part, tot);
@@ -280,19 +290,19 @@ __device__ void segment_items(uint16_t* off, uint16_t* items, uint32_t n, uint32
 		carry += tot;
 		__syncthreads();
 	}
-	if (threadIdx.x == 0)
+	if (tid == 0)
 		off[n] = (uint16_t)carry;
 	__syncthreads();
-	for (uint32_t v = threadIdx.x; v < n; v += kBatchThreads)
+	for (uint32_t v = tid; v < n; v += kBatchThreads)
 		cursor[v] = off[v];
 	__syncthreads();
-	for (uint32_t i = threadIdx.x; i < count; i += kBatchThreads)
+	for (uint32_t i = tid; i < count; i += kBatchThreads)
 		items[atomicAdd(&cursor[key_of(i)], 1u)] = (uint16_t)i;
 	__syncthreads();
 	if (!ordered)
 		return;
 	// ascending item order inside each segment (segments are short)
-	for (uint32_t v = threadIdx.x; v < n; v += kBatchThreads)
+	for (uint32_t v = tid; v < n; v += kBatchThreads)
 	{
 		uint32_t b = off[v], e = off[v + 1];
 		for (uint32_t x = b + 1; x < e; ++x)
@@ -362,7 +372,7 @@ __device__ void build_adjacency(const PatchSmem& s, const uint16_t* ib, uint32_t
 		return welded ? s.remap[v] : v;
 	};
 	segment_items(s.off, corners, vcount, icount, key_of, cursor, part, ordered);
-	for (uint32_t p = threadIdx.x; p < icount; p += kBatchThreads)
+	for (uint32_t p = (uint32_t)thread_id(); p < icount; p += kBatchThreads)
 	{
 		uint32_t j = corners[p];
 		uint32_t t = j / 3, c = j - t * 3;
@@ -451,7 +461,7 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 	const uint32_t V = vb_end - vb_begin;
 	const uint32_t target = a.target_index_counts[patch];
 	const uint32_t options = a.options;
-	const int tid = threadIdx.x;
+	const int tid = thread_id();
 
 	if (V > L.vmax || I > L.imax || V >= kNone16)
 	{
@@ -504,9 +514,7 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 				const uint32_t i = i0 + u * kBatchThreads;
 				if (i < V)
 				{
-					s.px[i] = x[u];
-					s.py[i] = y[u];
-					s.pz[i] = z[u];
+					s.pos[i] = V3{x[u], y[u], z[u]};
 				}
 			}
 		}
@@ -554,7 +562,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 		__syncthreads();
 		for (uint32_t i = tid; i < V; i += kBatchThreads)
 		{
-			float x = s.px[i], y = s.py[i], z = s.pz[i];
+			const V3 p = P(s, i);
+			const float x = p.x, y = p.y, z = p.z;
 			if (x != x || y != y || z != z)
 				continue;
 			uint64_t h = (uint64_t)canon_bits(x) * 0x9E3779B97F4A7C15ull ^ (uint64_t)canon_bits(y) * 0xC2B2AE3D27D4EB4Full ^
@@ -565,7 +574,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 				uint32_t old = atomicCAS(&table[slot], kNone, i);
 				if (old == kNone)
 					break;
-				if (s.px[old] == x && s.py[old] == y && s.pz[old] == z)
+				const V3 o = P(s, old);
+				if (o.x == x && o.y == y && o.z == z)
 				{
 					atomicMin(&table[slot], i);
 					break;
@@ -576,7 +586,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 		__syncthreads();
 		for (uint32_t i = tid; i < V; i += kBatchThreads)
 		{
-			float x = s.px[i], y = s.py[i], z = s.pz[i];
+			const V3 p = P(s, i);
+			const float x = p.x, y = p.y, z = p.z;
 			uint32_t r = i;
 			if (!(x != x || y != y || z != z))
 			{
@@ -588,7 +599,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 					uint32_t e = table[slot];
 					if (e == kNone)
 						break;
-					if (s.px[e] == x && s.py[e] == y && s.pz[e] == z)
+					const V3 o = P(s, e);
+					if (o.x == x && o.y == y && o.z == z)
 					{
 						r = e;
 						break;
@@ -750,7 +762,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 		uint64_t mn[3] = {~0ull, ~0ull, ~0ull}, mx[3] = {0, 0, 0};
 		for (uint32_t i = tid; i < V; i += kBatchThreads)
 		{
-			float c[3] = {s.px[i], s.py[i], s.pz[i]};
+			const V3 p = P(s, i);
+			const float c[3] = {p.x, p.y, p.z};
 			for (int k = 0; k < 3; ++k)
 			{
 				if (c[k] != c[k])
@@ -778,19 +791,20 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 	if (tid == 0)
 	{
 		float lo[3], hi[3];
-		const float* comp[3] = {s.px, s.py, s.pz};
 		for (int k = 0; k < 3; ++k)
 		{
 			lo[k] = FLT_MAX;
 			hi[k] = -FLT_MAX;
 			if (box[k] != ~0ull)
 			{
-				float v = comp[k][(uint32_t)box[k]];
+				const V3 p = P(s, (uint32_t)box[k]);
+				const float v = k == 0 ? p.x : (k == 1 ? p.y : p.z);
 				lo[k] = FLT_MAX > v ? v : FLT_MAX;
 			}
 			if (box[3 + k] != 0ull)
 			{
-				float v = comp[k][0xffffffffu - (uint32_t)box[3 + k]];
+				const V3 p = P(s, 0xffffffffu - (uint32_t)box[3 + k]);
+				const float v = k == 0 ? p.x : (k == 1 ? p.y : p.z);
 				hi[k] = -FLT_MAX < v ? v : -FLT_MAX;
 			}
 		}
@@ -808,9 +822,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 	for (uint32_t i = tid; i < V; i += kBatchThreads)
 	{
 		float sc = shf[3];
-		s.px[i] = (s.px[i] - shf[0]) * sc;
-		s.py[i] = (s.py[i] - shf[1]) * sc;
-		s.pz[i] = (s.pz[i] - shf[2]) * sc;
+		const V3 p = P(s, i);
+		s.pos[i] = V3{(p.x - shf[0]) * sc, (p.y - shf[1]) * sc, (p.z - shf[2]) * sc};
 	}
 	const float extent = shf[4];
 	__syncthreads();
@@ -959,6 +972,7 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 			break;
 		}
 		const uint32_t T = result_count / 3;
+		const int tid = thread_id();
 		build_adjacency(s, ib, result_count, V, true, false, corners, cursor, part);
 		PROFILE_PHASE(3);
 
@@ -1185,7 +1199,8 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 		// wrote their own source classes only).
 		//
 		// Bound by the latency of one wavefront's LDS and ballot chains; a chunk takes 4-8 rounds
-		// where one rank at a time took 15-20 decisions.  4096 patches of 64-512 triangles: @COMMIT@.
+		// where one rank at a time took 15-20 decisions.  4096 patches of 64-512 triangles:
+		// 541 to 466 us a call; 1156 groups of 1810 triangles: 2.58 to 1.43 ms.
 		uint64_t* const tab = (uint64_t*)s.sortbuf; // the sort's half: one word per vertex, zero between chunks
 		for (uint32_t v = tid; v < V; v += kBatchThreads)
 		{
