@@ -93,8 +93,7 @@ struct CallScalars
 	float scale;          // 1 / extent (0 for a flat mesh)
 	float extent;         // largest bounding box side
 	float result_error;   // squared error so far (prefix max of committed collapses)
-	float vertex_error;   // squared positional error (attribute path)
-	uint32_t vertex_error_bits; // atomicMax target for vertex_error (non-negative floats order as uints)
+	uint32_t vertex_error_bits; // squared positional error (attribute path): an atomicMax of float bits
 	uint64_t box_min[3];  // (ordered key << 32 | index) reductions for the bounding box
 	uint64_t box_max[3];
 	uint32_t candidates;  // C_p of the current pass
@@ -106,7 +105,6 @@ struct CallScalars
 	uint32_t stop_reason; // 0 out of collapses, 1 error limit, 2 count limit, 3 error goal
 	uint32_t skipped;
 	uint32_t rejected;
-	uint32_t tri_collapses;
 	uint32_t list_count[3][kListSegments]; // undecided work-list counters of the rounds (rotating), per segment
 	uint32_t list_off[kListSegments];      // where each segment starts in the list buffers
 	uint32_t window_count[kListSegments];  // ranks per segment of the window being opened (zero otherwise)
@@ -121,7 +119,9 @@ struct CallScalars
 	uint32_t x_launches;
 	uint32_t round;         // the commit rounds' base of the pass (list buffers rotate with the round number)
 	uint32_t epoch;         // the round tag before the base round (round minima are tagged, monotonic over the call)
-	uint32_t extended;      // 1 when the pass's window was extended on the device to the whole list
+	uint32_t extend;        // 1 when the pass's first window held no break and the list goes on
+	uint32_t split;         // 1 when a pass took wedges of one class to different classes
+	uint32_t stop_done;     // workgroups of the stop scan that have left their record (0 between scans)
 	uint32_t pick_capacity; // boundEdgeCollapses (src/simplifier.cpp:1292-1308): pick stops before exceeding it
 	uint32_t work[8];     // small counters of setup kernels
 };

@@ -485,11 +485,17 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	{
 		m.pend[k] = a.take<uint64_t>(2 * Vp);
 	}
+	for (int k = 0; k < 2; ++k)
+	{
+		m.adj_range[k] = a.take<uint2>(Vp);
+		m.adj[k] = a.take<uint2>(I + 4);
+	}
+	m.new_class = a.take<uint32_t>(Vp);
 	m.adj_off = a.take<uint32_t>(Vp + 1);
-	m.adj = a.take<uint2>(I + 4);
 
-	m.tri_cnt = a.take<uint32_t>(T);
-	m.tri_off = a.take<uint32_t>(T);
+	m.tile_sums = a.take<uint2>(2 * tile_sum_words(std::max(V, T)));
+	m.tri_cnt = prune ? a.take<uint32_t>(T) : nullptr;
+	m.tri_off = prune ? a.take<uint32_t>(T) : nullptr;
 
 	m.c_v0 = a.take<uint32_t>(cap);
 	m.c_v1 = a.take<uint32_t>(cap);
@@ -508,7 +514,7 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	m.status = a.take<uint8_t>(cap);
 	m.list[0] = a.take<uint4>(cap);
 	m.list[1] = a.take<uint4>(cap);
-	m.stop_tile = a.take<uint32_t>(3 * (cap / kScanTile + 2));
+	m.stop_tile = a.take<uint32_t>(stop_scan_words(cap));
 
 	// setup-only buffers alias the candidate arrays (not live at the same time)
 	p.table_size = pow2_at_least(2 * V + 2);
@@ -575,7 +581,6 @@ __global__ void __launch_bounds__(256) k_count_kinds(const uint32_t* remap, cons
 __global__ void k_scalars_init(CallScalars* sc)
 {
 	sc->result_error = 0.f;
-	sc->vertex_error = 0.f;
 	sc->vertex_error_bits = 0u;
 	sc->candidates = 0;
 	sc->dual_count = 0;
@@ -610,8 +615,7 @@ static std::atomic<int> g_deep_heads{kDeepHeads}, g_deep_from_head{kDeepFromHead
 // process: the rounds a list needs grow with its length, and the contexts of concurrent calls and
 // serving slots see calls of very different sizes (0: not seen yet)
 static std::atomic<int> g_head_rounds[33];
-// the same for the extension window [W, C) of a pass, learned only from extensions that opened
-// (most never do: each head of an extension that does not open is an empty launch)
+// the same for the extension window [W, C) of a pass
 static std::atomic<int> g_ext_head_rounds[33];
 
 static int size_bucket(size_t n)
@@ -713,6 +717,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		m.timer = nullptr;
 	m.ib_cur = 0;
 	m.loop_cur = 0;
+	m.adj_cur = 0;
 	m.epoch = 0;
 
 	t_read_backs = 0;
@@ -778,13 +783,10 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		HIP_CHECK(hipMemsetAsync(m.pend[b], 0xff, 2 * (V + 1) * sizeof(uint64_t), s));
 	}
 
-	// the first pass's adjacency and pick go before the set-up read-back, which returns their count
+	// the first pass's candidates go before the set-up read-back, which returns their count
 	launch_pick_capacity(s, m, I);
-	if (!prune && I)
-	{
-		launch_adjacency(s, m, I / 3);
+	if (I)
 		launch_pick(s, m, I / 3);
-	}
 
 	sync_scalars(ctx, m);
 	const CallScalars& h = *ctx.sc_host;
@@ -808,25 +810,17 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	// Prune: smallest component error still present (src/simplifier.cpp:2466-2470)
 	float prune_next = prune ? host_float_bits(h.prune_min_bits) : 0.f;
 
-	// Outside Prune a pass makes one read-back: when the stop scan of the first rank window finds
-	// no break, the window is extended on the device to the whole list (its rounds and stop scan
-	// are enqueued and leave at once otherwise), and the next pass's adjacency and pick follow the
-	// index remap, reading the new triangle count on the device.  Prune reads the pass's error back
-	// before its component pruning, and picks after it.
-	bool picked = !prune;
+	// A pass makes one read-back.  It enqueues the rounds of its first rank window, the stop scan and
+	// what follows the stop, the next pass's candidates among it; when the window holds no break and
+	// the list goes on, all that follows the scan leaves at once, and after the read-back the rest of
+	// the list is decided and the steps are enqueued again.  Prune, when it drops components after
+	// the pass, picks again from the triangles that are left.
 	// set once a window of this call needed more rounds than the cheap ones drain (long chains of
 	// dependent ranks, as on regular grids): later windows of the call run deep rounds
 	bool long_chains = false;
 	while (result_count > c.target_index_count)
 	{
 		size_t T = result_count / 3;
-		if (!picked)
-		{
-			launch_adjacency(s, m, T);
-			launch_pick(s, m, T);
-			sync_scalars(ctx, m);
-		}
-		picked = false;
 		size_t C = h.candidates;
 		if (C == 0)
 			break;
@@ -851,16 +845,14 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		launch_perform_init(s, m, C, deep);
 		// head rounds with one thread per rank of the window (the list only shrinks; workgroups
 		// past its current length leave at once, while a grid smaller than the list would make
-		// each thread walk several ranks' dependent gathers in turn), then the tail and the
-		// flip-failure resolution; their grid strides over any list length, so a grid capped at
+		// each thread walk several ranks' dependent gathers in turn), then the tail; their grid strides over any list length, so a grid capped at
 		// `max_threads` stays correct
 		auto window_rounds = [&](size_t lo, size_t hi, int head_base, int head_count, size_t max_threads) {
 			for (int hd = 0; hd < head_count; ++hd)
 				launch_round(s, m, std::min(hi - lo, max_threads), head_base + hd, hd, deep && hd >= deep_from);
 			launch_round_tail(s, m, head_count, (uint32_t)(hi - lo + 2), deep);
-			launch_resolve(s, m, lo, hi);
 		};
-		launch_window_extend(s, m, 0, W, false);
+		launch_window_open(s, m, 0, W);
 		int heads_run = heads;
 		bool switched_deep = false;
 		if (!learned && W > kWholeWindow && heads)
@@ -890,33 +882,25 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 			}
 			heads_run = done;
 			launch_round_tail(s, m, done, (uint32_t)(W + 2), deep);
-			launch_resolve(s, m, 0, W);
 		}
 		else
 			window_rounds(0, W, 0, heads, (size_t)-1);
-		launch_stop_scan(s, m, W, C, goal, error_limit, false);
+		launch_stop_scan(s, m, W, C, goal, error_limit);
+		launch_apply(s, m, W, T);
+		sync_scalars(ctx, m);
 		const int ext_bucket = size_bucket(C - W);
 		const int ext_learned = g_ext_head_rounds[ext_bucket].load(std::memory_order_relaxed);
 		const int ext_heads = std::max(2, std::min(ext_learned ? ext_learned : 2, kHeadSizeSlots - heads_run));
-		if (W < C)
+		const bool extended = h.extend != 0;
+		if (extended)
 		{
-			// the rest of the list, decided only when the window held no break (otherwise every
-			// kernel below leaves at once: a few small grids)
-			launch_window_extend(s, m, W, C, true);
-			window_rounds(W, C, heads_run, ext_heads, (size_t)64 * 1024);
-			launch_stop_scan(s, m, C, C, goal, error_limit, true);
+			// the rest of the list
+			launch_window_open(s, m, W, C);
+			window_rounds(W, C, heads_run, ext_heads, (size_t)-1);
+			launch_stop_scan(s, m, C, C, goal, error_limit);
+			launch_apply(s, m, C, T);
+			sync_scalars(ctx, m);
 		}
-		launch_stop_commit(s, m, C, goal, error_limit);
-		// a pass without commits changes nothing below: the loop then ends on the read-back
-		launch_apply(s, m, C);
-		launch_remap_triangles(s, m, T);
-		if (!prune)
-		{
-			launch_adjacency(s, m, T, &m.sc->next_triangles);
-			launch_pick(s, m, T, &m.sc->next_triangles);
-			picked = true;
-		}
-		sync_scalars(ctx, m);
 		if (h.work[3])
 			throw std::runtime_error("priority rounds did not converge (internal error)");
 
@@ -947,13 +931,8 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		};
 		if (heads_run)
 			g_head_rounds[bucket].store(learn_heads(0, heads_run), std::memory_order_relaxed);
-		if (W < C)
-		{
-			if (h.extended)
-				g_ext_head_rounds[ext_bucket].store(learn_heads(heads_run, ext_heads), std::memory_order_relaxed);
-			else if (ext_learned > 2)
-				g_ext_head_rounds[ext_bucket].store(ext_learned - ext_learned / 8, std::memory_order_relaxed);
-		}
+		if (extended)
+			g_ext_head_rounds[ext_bucket].store(learn_heads(heads_run, ext_heads), std::memory_order_relaxed);
 		long_chains |= switched_deep || (heads_run >= deep_heads && h.head_sizes[heads_run - 1] >= kTailList);
 		ctx.window_fraction = std::min(1.0, (double)(h.stop + 1) / (double)C);
 
@@ -968,23 +947,25 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		ps.rounds = h.round;
 		ps.tail_rounds = h.tail_rounds;
 		t_passes.push_back(ps);
-		t_call.device_extensions += h.extended;
+		t_call.device_extensions += extended;
 
+		// without a commit the reference stops before the index remap and the loop update
+		// (src/simplifier.cpp:2523-2524): the buffers of this pass stay the current ones
 		if (h.committed == 0)
-		{
-			// the index remap and loop update ran before the read-back; without a commit the
-			// reference stops before them (src/simplifier.cpp:2523-2524), and the buffers they read
-			// are untouched (both are double-buffered), so those stay current
-			m.ib_cur ^= 1;
-			m.loop_cur ^= 1;
 			break;
-		}
+		m.ib_cur ^= 1;
+		m.loop_cur ^= 1;
+		m.adj_cur ^= 1;
 		result_count = (size_t)h.next_triangles * 3;
+		if (h.split)
+			launch_adjacency_ranges(s, m, h.next_triangles);
 
 		// components whose error fell under the pass's error (src/simplifier.cpp:2539-2541)
-		if (prune && result_count > c.target_index_count && prune_next <= h.vertex_error)
+		const float vertex_error = A ? host_float_bits(h.vertex_error_bits) : h.result_error;
+		if (prune && result_count > c.target_index_count && prune_next <= vertex_error)
 		{
-			launch_prune_triangles(s, m, result_count / 3, plan.comp, plan.cerr, h.vertex_error);
+			launch_prune_triangles(s, m, result_count / 3, plan.comp, plan.cerr, vertex_error);
+			launch_pick(s, m, result_count / 3, &m.sc->next_triangles);
 			sync_scalars(ctx, m);
 			result_count = (size_t)h.next_triangles * 3;
 			prune_next = host_float_bits(h.prune_min_bits);
@@ -993,7 +974,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 
 	// the last read-back (every pass ends with one, after its stop scan) holds the result error
 	result_error_sq = h.result_error;
-	float vertex_error_sq = h.vertex_error;
+	float vertex_error_sq = A ? host_float_bits(h.vertex_error_bits) : h.result_error;
 
 	// remaining components up to the error limit (src/simplifier.cpp:2545-2569)
 	bool prune_stale = true;

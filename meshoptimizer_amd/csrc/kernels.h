@@ -48,13 +48,17 @@ struct Mesh
 	                         // over ranks whose source is the class, and whose target is
 	uint32_t epoch;
 
-	uint32_t* adj_off;       // V + 1: welded corner CSR offsets of the current pass
-	uint2* adj;              // I: (next, prev) per corner
+	uint2* adj_range[2];     // V: a class's entries (begin, end) of adj, of the current pass and the next
+	uint2* adj[2];           // I: (next, prev) classes per corner
+	int adj_cur;
+	uint32_t* new_class;     // V: the class a primary's class belongs to after the pass
+	uint32_t* adj_off;       // V + 1: offsets of an adjacency built from scratch
 
 	uint32_t* ib[2];         // index buffer ping-pong
 	int ib_cur;
 
-	uint32_t* tri_cnt;       // per-triangle counts (pick / remap compaction)
+	uint2* tile_sums;        // per-tile sums of the blocked compactions
+	uint32_t* tri_cnt;       // per-triangle flags and offsets (Prune only)
 	uint32_t* tri_off;
 
 	uint32_t* c_v0;          // candidates in pick order
@@ -72,7 +76,7 @@ struct Mesh
 	float* r_err;
 	uint8_t* status;
 	uint4* list[2];          // undecided work lists: (rank, source class, target class, 0)
-	uint32_t* stop_tile;     // per-tile aggregates of the stop scan (3 words each)
+	uint32_t* stop_tile;     // per-tile sums and records of the stop scan
 
 	uint32_t* temp;          // scan / sort temporaries
 	CallScalars* sc;
@@ -99,10 +103,14 @@ void launch_attribute_quadrics(hipStream_t s, Mesh& m, const uint32_t* raw_off, 
 void launch_dual_count(hipStream_t s, Mesh& m, const uint32_t* raw_off);
 
 // ---------------------------------------------------------------- passes (pass.hip)
-// tri_count sizes the grids; `live`, when given, is a device word holding the actual count (at
-// most tri_count), so a pass can be enqueued before the host has read it
-void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live = nullptr);
+// the candidates of the current triangles; tri_count sizes the grids, `live`, when given, is a
+// device word holding the actual count (at most tri_count)
 void launch_pick(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live = nullptr);
+// welded adjacency of the current triangles from scratch, as offsets (m.adj_off, m.adj[m.adj_cur]),
+// and as the ranges the passes read
+void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count);
+void launch_adjacency_ranges(hipStream_t s, Mesh& m, size_t tri_count);
+size_t tile_sum_words(size_t n); // entries of one m.tile_sums array (there are two)
 void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count);
 // commit state of a pass; with source_lists, also the candidate ranks grouped by source class
 // that deep rounds read
@@ -111,12 +119,14 @@ void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count);
 void launch_pick_capacity(hipStream_t s, Mesh& m, size_t index_count);
 void launch_round(hipStream_t s, Mesh& m, size_t list_bound, int head_index, int rel, bool deep);
 void launch_round_tail(hipStream_t s, Mesh& m, int rel, uint32_t max_rounds, bool deep);
-void launch_window_extend(hipStream_t s, Mesh& m, size_t lo, size_t hi, bool if_no_stop);
-void launch_resolve(hipStream_t s, Mesh& m, size_t lo, size_t hi);
-void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, uint32_t goal, float error_limit, bool conditional);
-void launch_stop_commit(hipStream_t s, Mesh& m, size_t window, uint32_t goal, float error_limit);
-void launch_apply(hipStream_t s, Mesh& m, size_t cand_count);
-void launch_remap_triangles(hipStream_t s, Mesh& m, size_t tri_count);
+void launch_window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi);
+void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, uint32_t goal, float error_limit);
+size_t stop_scan_words(size_t cand_count); // words of m.stop_tile
+// what follows the stop of a pass whose window was [0, window), into the other set of loop, index
+// and adjacency buffers: commits at or past the stop taken back, quadrics, edge loops, the index
+// remap with the next pass's candidates, the next adjacency.  Nothing runs when the list goes on
+// past the window (sc->extend)
+void launch_apply(hipStream_t s, Mesh& m, size_t window, size_t tri_count);
 void launch_debug_bits(hipStream_t s, Mesh& m, size_t index_count);
 void launch_sparse_backmap(hipStream_t s, uint32_t* ib, size_t index_count, const uint32_t* sparse_remap);
 

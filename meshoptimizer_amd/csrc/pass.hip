@@ -33,33 +33,22 @@ __constant__ uint8_t c_has_opposite[5][5] = {
 };
 
 // ------------------------------------------------------------------------------------------
-// welded corner CSR for this pass (src/simplifier.cpp:52-109).  Segment order is free: every
-// consumer (open-edge tests, flip tests, neighbourhood scans) is a count or an any().  One atomic
-// pass counts the corners per class and hands each corner its slot in the class's segment; after
-// the scan the fill places the corners without atomics.
+// welded corner CSR of the current index buffer (src/simplifier.cpp:52-109), from scratch: for the
+// vertex solve, over the result, and after a pass that split a class.  Segment order is free: every consumer is a count or an any().
+// One atomic pass counts the corners per class and hands each corner its slot in the class's
+// segment; after the scan the fill places the corners without atomics.
 
-// the live triangle count: the host's when `live` is null, else the device word (at most the
-// host's, which sizes the grid)
-__device__ __forceinline__ size_t live_tris(size_t tris_max, const uint32_t* live)
-{
-	if (!live)
-		return tris_max;
-	size_t n = *live;
-	return n < tris_max ? n : tris_max;
-}
-
-__global__ void k_adj_count(const uint32_t* ib, size_t tris_max, const uint32_t* live, const uint32_t* remap, uint32_t* counts, uint32_t* slot)
+__global__ void k_adj_count(const uint32_t* ib, size_t corners, const uint32_t* remap, uint32_t* counts, uint32_t* slot)
 {
 	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (j < 3 * live_tris(tris_max, live))
+	if (j < corners)
 		slot[j] = atomicAdd(&counts[remap[ib[j]]], 1u);
 }
 
-__global__ void k_adj_fill(const uint32_t* ib, size_t tris_max, const uint32_t* live, const uint32_t* remap, const uint32_t* off, const uint32_t* slot,
-                           uint2* adj)
+__global__ void k_adj_fill(const uint32_t* ib, size_t tris, const uint32_t* remap, const uint32_t* off, const uint32_t* slot, uint2* adj)
 {
 	size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= live_tris(tris_max, live))
+	if (t >= tris)
 		return;
 	uint32_t a = remap[ib[t * 3 + 0]], b = remap[ib[t * 3 + 1]], c = remap[ib[t * 3 + 2]];
 	adj[off[a] + slot[t * 3 + 0]] = make_uint2(b, c);
@@ -67,109 +56,324 @@ __global__ void k_adj_fill(const uint32_t* ib, size_t tris_max, const uint32_t* 
 	adj[off[c] + slot[t * 3 + 2]] = make_uint2(a, b);
 }
 
-// the corner slots go to m.keys, free whenever the adjacency is rebuilt (before pick, after the
-// pass loop)
-void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live)
+__global__ void k_adj_ranges(const uint32_t* off, size_t n, uint2* range)
+{
+	size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (v < n)
+		range[v] = make_uint2(off[v], off[v + 1]);
+}
+
+// the corner slots go to m.keys, free between the passes and after them
+void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count)
 {
 	size_t n = m.vertex_count;
 	fill_u32(s, m.adj_off, 0, n + 1);
 	if (tri_count)
-		k_adj_count<<<grid_for(tri_count * 3), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, live, m.remap, m.adj_off, m.keys);
+		k_adj_count<<<grid_for(tri_count * 3), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count * 3, m.remap, m.adj_off, m.keys);
 	scan_exclusive(s, m.adj_off, m.adj_off, n, nullptr, m.adj_off + n, m.temp);
 	if (tri_count)
-		k_adj_fill<<<grid_for(tri_count), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, live, m.remap, m.adj_off, m.keys, m.adj);
+		k_adj_fill<<<grid_for(tri_count), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, m.remap, m.adj_off, m.keys, m.adj[m.adj_cur]);
+}
+
+void launch_adjacency_ranges(hipStream_t s, Mesh& m, size_t tri_count)
+{
+	launch_adjacency(s, m, tri_count);
+	k_adj_ranges<<<grid_for(m.vertex_count), kThreads, 0, s>>>(m.adj_off, m.vertex_count, m.adj_range[m.adj_cur]);
 }
 
 // ------------------------------------------------------------------------------------------
-// pickEdgeCollapses, src/simplifier.cpp:1310-1372: candidates of one triangle in edge order
+// Blocked compaction: a count kernel leaves one sum per tile, and the workgroup that writes a tile
+// adds the sums before its own and scans its items; no per-item counts or offsets go through
+// memory and no scan kernels run in between.  At most kMaxTiles tiles, so that the sums before a
+// tile stay a few reads per thread.
 
-__device__ __forceinline__ int pick_triangle(const uint32_t* ib, size_t t, const uint32_t* remap, const uint8_t* kind, const uint32_t* loop,
-                                             const uint32_t* loopback, uint32_t v0[3], uint32_t v1[3], uint32_t bidi[3])
+constexpr size_t kMaxTiles = 1024;
+
+static inline uint32_t tile_items(size_t n)
 {
-	uint32_t tri[3] = {ib[t * 3 + 0], ib[t * 3 + 1], ib[t * 3 + 2]};
-	int count = 0;
+	return div_up(n ? n : 1, (size_t)kThreads * kMaxTiles);
+}
+
+size_t tile_sum_words(size_t)
+{
+	return kMaxTiles + 1;
+}
+
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
+{
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1)
+		v += __shfl_xor(v, o, 64);
+	return v;
+}
+
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+#pragma unroll
+	for (int o = 32; o > 0; o >>= 1)
+	{
+		const uint32_t t = __shfl_xor(v, o, 64);
+		v = t > v ? t : v;
+	}
+	return v;
+}
+
+// sums over the workgroup, in every thread; red: one word per wavefront and value
+__device__ __forceinline__ uint2 block_sum2(uint2 v, uint2* red)
+{
+	const uint32_t x = wave_sum(v.x), y = wave_sum(v.y);
+	if (__lane_id() == 0)
+		red[threadIdx.x >> 6] = make_uint2(x, y);
+	__syncthreads();
+	uint2 t = make_uint2(0, 0);
+#pragma unroll
+	for (int w = 0; w < kThreads / 64; ++w)
+	{
+		t.x += red[w].x;
+		t.y += red[w].y;
+	}
+	__syncthreads();
+	return t;
+}
+
+__device__ __forceinline__ uint2 sums_before(const uint2* sums, uint32_t tile, uint2* red)
+{
+	uint2 v = make_uint2(0, 0);
+	for (uint32_t b = threadIdx.x; b < tile; b += kThreads)
+	{
+		v.x += sums[b].x;
+		v.y += sums[b].y;
+	}
+	return block_sum2(v, red);
+}
+
+// exclusive scan of one word per thread across the workgroup
+__device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* red, uint32_t& total)
+{
+	uint32_t x = v;
+	const int lane = __lane_id(), wave = threadIdx.x >> 6;
+#pragma unroll
+	for (int o = 1; o < 64; o <<= 1)
+	{
+		const uint32_t t = __shfl_up(x, o, 64);
+		x += lane >= o ? t : 0u;
+	}
+	if (lane == 63)
+		red[wave] = x;
+	__syncthreads();
+	uint32_t before = 0, all = 0;
+#pragma unroll
+	for (int w = 0; w < kThreads / 64; ++w)
+	{
+		before += w < wave ? red[w] : 0u;
+		all += red[w];
+	}
+	__syncthreads();
+	total = all;
+	return before + x - v;
+}
+
+// ------------------------------------------------------------------------------------------
+// remapIndexBuffer (src/simplifier.cpp:1811-1843) and the next pass's pickEdgeCollapses
+// (1310-1372) in one sweep of two kernels: each triangle is taken through collapse_remap and kept
+// when its primaries stay distinct, in order, and a kept triangle's candidates are listed in edge
+// order.  kCompact false: the triangles as they are, candidates only (the first pass, and the
+// triangles that Prune left).
+
+struct TriArgs
+{
+	const uint32_t* in;
+	uint32_t* out;
+	const uint32_t* live; // device word bounding the triangle count (null: the host's)
+	const uint32_t* cremap;
+	const uint32_t* remap;
+	const uint8_t* kind;
+	const uint32_t* loop;
+	const uint32_t* loopback;
+	uint2* sums; // (kept triangles, candidates) per tile
+	uint32_t* c_v0;
+	uint32_t* c_v1;
+	float* c_err;
+	CallScalars* sc;
+	uint32_t tris;
+	uint32_t items;
+};
+
+__device__ __forceinline__ uint32_t live_tris(const TriArgs& a)
+{
+	if (!a.live)
+		return a.tris;
+	const uint32_t n = *a.live;
+	return n < a.tris ? n : a.tris;
+}
+
+template <bool kCompact>
+__device__ __forceinline__ bool load_triangle(const TriArgs& a, uint32_t t, uint32_t v[3], uint32_t r[3])
+{
+#pragma unroll
+	for (int q = 0; q < 3; ++q)
+	{
+		const uint32_t i = a.in[(size_t)t * 3 + q];
+		v[q] = kCompact ? a.cremap[i] : i;
+	}
+#pragma unroll
+	for (int q = 0; q < 3; ++q)
+		r[q] = a.remap[v[q]];
+	return !kCompact || (r[0] != r[1] && r[0] != r[2] && r[1] != r[2]);
+}
+
+// the candidates of one triangle, pickEdgeCollapses (src/simplifier.cpp:1310-1372), in edge order
+__device__ __forceinline__ uint32_t pick_triangle(const TriArgs& a, const uint32_t v[3], const uint32_t r[3], uint32_t v0[3], uint32_t v1[3], bool bidi[3])
+{
+	const uint8_t kd[3] = {a.kind[v[0]], a.kind[v[1]], a.kind[v[2]]};
+	uint32_t count = 0;
 #pragma unroll
 	for (int e = 0; e < 3; ++e)
 	{
-		uint32_t i0 = tri[e];
-		uint32_t i1 = tri[e == 2 ? 0 : e + 1];
-		uint32_t r0 = remap[i0], r1 = remap[i1];
-		if (r0 == r1)
+		const int f = e == 2 ? 0 : e + 1;
+		const uint32_t i0 = v[e], i1 = v[f];
+		if (r[e] == r[f])
 			continue;
-		uint8_t k0 = kind[i0], k1 = kind[i1];
-		uint8_t c01 = c_can_collapse[k0][k1], c10 = c_can_collapse[k1][k0];
+		const uint8_t k0 = kd[e], k1 = kd[f];
+		const uint8_t c01 = c_can_collapse[k0][k1], c10 = c_can_collapse[k1][k0];
 		if (!(c01 | c10))
 			continue;
-		if (c_has_opposite[k0][k1] && r1 > r0)
+		if (c_has_opposite[k0][k1] && r[f] > r[e])
 			continue;
-		if ((k0 == kBorder || k0 == kSeam) && k1 != kManifold && loop[i0] != i1)
+		if ((k0 == kBorder || k0 == kSeam) && k1 != kManifold && a.loop[i0] != i1)
 			continue;
-		if ((k1 == kBorder || k1 == kSeam) && k0 != kManifold && loopback[i1] != i0)
+		if ((k1 == kBorder || k1 == kSeam) && k0 != kManifold && a.loopback[i1] != i0)
 			continue;
-		if (c01 & c10)
-		{
-			v0[count] = i0;
-			v1[count] = i1;
-			bidi[count] = 1;
-		}
-		else
-		{
-			v0[count] = c01 ? i0 : i1;
-			v1[count] = c01 ? i1 : i0;
-			bidi[count] = 0;
-		}
+		const bool both = c01 & c10, fwd = both || c01;
+		// at a compile-time place, so that the arrays stay in registers
+#pragma unroll
+		for (uint32_t q = 0; q < 3; ++q)
+			if (q == count)
+			{
+				v0[q] = fwd ? i0 : i1;
+				v1[q] = fwd ? i1 : i0;
+				bidi[q] = both;
+			}
 		count++;
 	}
 	return count;
 }
 
-__global__ void k_pick_count(const uint32_t* ib, size_t tris_max, const uint32_t* live, const uint32_t* remap, const uint8_t* kind, const uint32_t* loop,
-                             const uint32_t* loopback, uint32_t* counts)
+template <bool kCompact>
+__global__ void __launch_bounds__(kThreads) k_tri_count(TriArgs a)
 {
-	size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= live_tris(tris_max, live))
+	__shared__ uint2 red[kThreads / 64];
+	if (kCompact && a.sc->extend)
 		return;
-	uint32_t v0[3], v1[3], bd[3];
-	counts[t] = (uint32_t)pick_triangle(ib, t, remap, kind, loop, loopback, v0, v1, bd);
+	const uint32_t tris = live_tris(a), base = blockIdx.x * kThreads * a.items;
+	uint2 n = make_uint2(0, 0);
+	for (uint32_t j = 0; j < a.items; ++j)
+	{
+		const uint32_t t = base + j * kThreads + threadIdx.x;
+		if (t >= tris)
+			break;
+		uint32_t v[3], r[3], v0[3], v1[3];
+		bool bd[3];
+		if (load_triangle<kCompact>(a, t, v, r))
+		{
+			n.x++;
+			n.y += pick_triangle(a, v, r, v0, v1, bd);
+		}
+	}
+	n = block_sum2(n, red);
+	if (threadIdx.x == 0)
+	{
+		a.sums[blockIdx.x] = n;
+		if (blockIdx.x == 0)
+			a.sc->candidates = 0;
+	}
 }
 
-// triangles are taken while `written + 3 <= capacity` (src/simplifier.cpp:1318-1320)
-__global__ void k_pick_write(const uint32_t* ib, size_t tris_max, const uint32_t* live, const uint32_t* remap, const uint8_t* kind, const uint32_t* loop,
-                             const uint32_t* loopback, const uint32_t* offsets, const uint32_t* capacity_word, uint32_t* c_v0, uint32_t* c_v1,
-                             float* c_err, uint32_t* out_count)
+// Candidates are taken while `written + 3 <= capacity` (src/simplifier.cpp:1318-1320): the taken
+// triangles form a prefix.
+template <bool kCompact>
+__global__ void __launch_bounds__(kThreads) k_tri_write(TriArgs a)
 {
-	size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	const size_t tris = live_tris(tris_max, live);
-	if (t >= tris)
+	__shared__ uint2 red2[kThreads / 64];
+	__shared__ uint32_t red[kThreads / 64];
+	if (kCompact && a.sc->extend)
 		return;
-	const uint32_t capacity = *capacity_word;
-	uint32_t base = offsets[t];
-	if ((uint64_t)base + 3 > capacity)
-		return;
-	uint32_t v0[3], v1[3], bd[3];
-	int count = pick_triangle(ib, t, remap, kind, loop, loopback, v0, v1, bd);
-	for (int k = 0; k < count; ++k)
+	const uint32_t tris = live_tris(a), base = blockIdx.x * kThreads * a.items;
+	const uint64_t capacity = a.sc->pick_capacity;
+	uint2 at = sums_before(a.sums, blockIdx.x, red2);
+	for (uint32_t j = 0; j < a.items; ++j)
 	{
-		c_v0[base + k] = v0[k];
-		c_v1[base + k] = v1[k];
-		c_err[base + k] = __uint_as_float(bd[k]); // the bidirectional flag until ranked
+		const uint32_t t = base + j * kThreads + threadIdx.x;
+		uint32_t v[3], r[3], v0[3], v1[3];
+		bool bd[3];
+		const bool keep = t < tris && load_triangle<kCompact>(a, t, v, r);
+		const uint32_t count = keep ? pick_triangle(a, v, r, v0, v1, bd) : 0;
+		uint32_t total;
+		const uint32_t ex = block_scan((keep ? 0x10000u : 0u) + count, red, total);
+		if (keep)
+		{
+			if (kCompact)
+			{
+				uint32_t* out = a.out + (size_t)(at.x + (ex >> 16)) * 3;
+				out[0] = v[0];
+				out[1] = v[1];
+				out[2] = v[2];
+			}
+			const uint32_t c = at.y + (ex & 0xffffu);
+			if ((uint64_t)c + 3 <= capacity)
+			{
+#pragma unroll
+				for (uint32_t q = 0; q < 3; ++q)
+					if (q < count)
+					{
+						a.c_v0[c + q] = v0[q];
+						a.c_v1[c + q] = v1[q];
+						a.c_err[c + q] = __uint_as_float(bd[q] ? 1u : 0u); // the two-way flag until ranked
+					}
+				// the taken triangle after which the next does not fit ends the list
+				if ((uint64_t)c + count + 3 > capacity)
+					a.sc->candidates = c + count;
+			}
+		}
+		at.x += total >> 16;
+		at.y += total & 0xffffu;
 	}
-	// offsets are non-decreasing, so the processed triangles form a prefix; its last one writes C
-	if (t + 1 == tris || (uint64_t)offsets[t + 1] + 3 > capacity)
-		*out_count = base + (uint32_t)count;
+	if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0)
+	{
+		if (kCompact)
+			a.sc->next_triangles = at.x;
+		if ((uint64_t)at.y + 3 <= capacity)
+			a.sc->candidates = at.y;
+	}
+}
+
+static TriArgs tri_args(Mesh& m, size_t tri_count, const uint32_t* live, int loop_set)
+{
+	TriArgs a;
+	a.in = m.ib[m.ib_cur];
+	a.out = m.ib[m.ib_cur ^ 1];
+	a.live = live;
+	a.cremap = m.cremap;
+	a.remap = m.remap;
+	a.kind = m.kind;
+	a.loop = m.loop[loop_set];
+	a.loopback = m.loopback[loop_set];
+	a.sums = m.tile_sums;
+	a.c_v0 = m.c_v0;
+	a.c_v1 = m.c_v1;
+	a.c_err = m.c_err;
+	a.sc = m.sc;
+	a.tris = (uint32_t)tri_count;
+	a.items = tile_items(tri_count);
+	return a;
 }
 
 void launch_pick(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live)
 {
-	uint32_t* loop = m.loop[m.loop_cur];
-	uint32_t* loopback = m.loopback[m.loop_cur];
-	HIP_CHECK(hipMemsetAsync(&m.sc->candidates, 0, sizeof(uint32_t), s));
-	if (!tri_count)
-		return;
-	k_pick_count<<<grid_for(tri_count), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, live, m.remap, m.kind, loop, loopback, m.tri_cnt);
-	scan_exclusive(s, m.tri_cnt, m.tri_off, tri_count, live, nullptr, m.temp);
-	k_pick_write<<<grid_for(tri_count), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, live, m.remap, m.kind, loop, loopback, m.tri_off,
-	                                                      &m.sc->pick_capacity, m.c_v0, m.c_v1, m.c_err, &m.sc->candidates);
+	const TriArgs a = tri_args(m, tri_count, live, m.loop_cur);
+	const unsigned int tiles = div_up(tri_count ? tri_count : 1, (size_t)kThreads * a.items);
+	k_tri_count<false><<<tiles, kThreads, 0, s>>>(a);
+	k_tri_write<false><<<tiles, kThreads, 0, s>>>(a);
 }
 
 // boundEdgeCollapses (src/simplifier.cpp:1292-1308) from the dual count on the device:
@@ -323,30 +527,25 @@ void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count)
 // the minimum over both roles is the smaller of the pair.
 // Ranks that decide in one round never touch each other's state.
 
+enum : uint8_t
+{
+	kFlipPass = 4,        // flip test passes, now and for good; commits once lowest at its endpoints
+	kFlipFail = 5,        // flip test fails for good; resolved as skipped or rejected at the end
+	kCommittedBorder = 6, // committed, the source a border vertex (one triangle, not two)
+};
+
+__device__ __forceinline__ bool is_commit(uint8_t st)
+{
+	return st == kCommitted || st == kCommittedBorder;
+}
+
 __device__ __forceinline__ uint64_t round_key(uint32_t epoch, uint32_t k)
 {
 	return ((uint64_t)(~epoch) << 32) | k;
 }
 
-// hasTriangleFlips, src/simplifier.cpp:1200-1232
-__device__ __forceinline__ bool collapse_flips(const uint32_t* off, const uint2* adj, const float4* pos, const uint32_t* cremap, uint32_t i0, uint32_t i1)
-{
-	V3 v0 = load_pos(pos, i0), v1 = load_pos(pos, i1);
-	for (uint32_t p = off[i0], e = off[i0 + 1]; p < e; ++p)
-	{
-		uint2 nb = adj[p];
-		uint32_t a = cremap[nb.x];
-		uint32_t b = cremap[nb.y];
-		if (a == i1 || b == i1 || a == b)
-			continue;
-		if (triangle_flips(load_pos(pos, a), load_pos(pos, b), v0, v1))
-			return true;
-	}
-	return false;
-}
-
-// commit writes of one collapse, src/simplifier.cpp:1573-1611
-__device__ __forceinline__ void commit_collapse(uint32_t* cremap, uint32_t i0, uint32_t i1, const uint8_t* kind, const uint32_t* wedge,
+// commit writes of one collapse, src/simplifier.cpp:1573-1611; returns the status that records it
+__device__ __forceinline__ uint8_t commit_collapse(uint32_t* cremap, uint32_t i0, uint32_t i1, const uint8_t* kind, const uint32_t* wedge,
                                                 const uint32_t* remap, const uint32_t* loop, const uint32_t* loopback)
 {
 	uint8_t k = kind[i0];
@@ -369,19 +568,14 @@ __device__ __forceinline__ void commit_collapse(uint32_t* cremap, uint32_t i0, u
 	}
 	else
 		cremap[i0] = i1;
+	return k == kBorder ? kCommittedBorder : kCommitted;
 }
-
-enum : uint8_t
-{
-	kFlipPass = 4, // flip test passes, now and for good; commits once lowest at its endpoints
-	kFlipFail = 5, // flip test fails for good; resolved as skipped or rejected at the end
-};
 
 struct RoundState
 {
 	const uint32_t* r_v0;
 	const uint32_t* r_v1;
-	const uint32_t* adj_off;
+	const uint2* adj_range; // a class's entries of adj: (begin, end)
 	const uint2* adj;
 	const float4* pos;
 	const uint8_t* kind;
@@ -635,7 +829,7 @@ __device__ __forceinline__ bool round_x(const RoundState& a, uint4 w, uint32_t e
 	const uint32_t l0 = a.lock_rank[r0], l1 = a.lock_rank[r1];
 	const ulonglong2 q0 = prev[r0], q1 = prev[r1];
 	const uint64_t p0 = q0.x < q0.y ? q0.x : q0.y, p1 = q1.x < q1.y ? q1.x : q1.y;
-	const uint32_t begin = a.adj_off[r0], end = a.adj_off[r0 + 1];
+	const uint2 range = a.adj_range[r0];
 	const V3 v0 = load_pos(a.pos, r0), v1 = load_pos(a.pos, r1);
 	if (st != kUndecided && st != kFlipPass)
 		return false;
@@ -651,7 +845,7 @@ __device__ __forceinline__ bool round_x(const RoundState& a, uint4 w, uint32_t e
 	uint8_t now = st;
 	if (st == kUndecided && (low0 || low1))
 	{
-		int o = flip_outcome<kDeep>(a, r1, k, epoch, begin, end, v0, v1);
+		int o = flip_outcome<kDeep>(a, r1, k, epoch, range.x, range.y, v0, v1);
 		if (o == 2)
 		{
 			a.status[k] = kFlipFail;
@@ -662,10 +856,9 @@ __device__ __forceinline__ bool round_x(const RoundState& a, uint4 w, uint32_t e
 	}
 	if (now == kFlipPass && low0 && low1)
 	{
-		commit_collapse(a.cremap, a.r_v0[k], a.r_v1[k], a.kind, a.wedge, a.remap, a.loop, a.loopback);
+		a.status[k] = commit_collapse(a.cremap, a.r_v0[k], a.r_v1[k], a.kind, a.wedge, a.remap, a.loop, a.loopback);
 		a.lock_rank[r0] = k;
 		a.lock_rank[r1] = k;
-		a.status[k] = kCommitted;
 		return false;
 	}
 	if (now != st)
@@ -708,7 +901,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(k
 {
 	CallScalars* sc = a.sc;
 	// rounds are numbered from a base on the device (the tail leaves it past its last round), so
-	// rounds can follow a tail or a device-side window extension without a read-back; `rel` counts
+	// rounds can follow a tail without a read-back; `rel` counts
 	// the head rounds launched since the base was set
 	const uint32_t round = sc->round + rel, epoch = sc->epoch + 1 + rel;
 	const uint32_t seg = blockIdx.x % kListSegments;
@@ -838,10 +1031,8 @@ __global__ void k_perform_init_scalars(CallScalars* sc)
 		sc->list_off[q] = 0;
 		sc->window_count[q] = 0;
 	}
-	sc->stop_reason = 0;
 	sc->tail_rounds = 0;
 	sc->round = 0;
-	sc->extended = 0;
 }
 
 // candidate ranks grouped by source class (order inside a group is irrelevant): one atomic pass
@@ -870,8 +1061,8 @@ static RoundState round_state(Mesh& m)
 	RoundState a;
 	a.r_v0 = m.r_v0;
 	a.r_v1 = m.r_v1;
-	a.adj_off = m.adj_off;
-	a.adj = m.adj;
+	a.adj_range = m.adj_range[m.adj_cur];
+	a.adj = m.adj[m.adj_cur];
 	a.pos = m.pos;
 	a.kind = m.kind;
 	a.wedge = m.wedge;
@@ -918,23 +1109,14 @@ void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count)
 		k_src_fill<<<grid_for(cand_count), kThreads, 0, s>>>(round_state(m), m.r_r0, cand_count, m.keys, m.src_rank, m.src_val);
 }
 
-// ranks [lo, hi) become the list of the next round (sc->round), in segments by source class.
-// With `if_no_stop` the window opens only when the stop scan of [0, lo) found no break
-// (sc->stop == lo) and the list goes on: the rest of the list is then decided in the same pass
-// without a read-back (sc->extended = 1); otherwise the list stays empty and the rounds that
-// follow do nothing.  Two kernels: the count of each segment (into sc->window_count, zero since
-// the previous window's tail), then the placement, each segment at the sum of the counts before it.
-__device__ __forceinline__ bool window_opens(const CallScalars* sc, uint32_t lo, uint32_t hi, bool if_no_stop)
-{
-	return !if_no_stop || (sc->stop >= lo && hi > lo);
-}
-
-__global__ void __launch_bounds__(kThreads) k_window_count(RoundState a, uint32_t lo, uint32_t hi, const uint32_t* r_r0, bool if_no_stop)
+// ranks [lo, hi) become the list of the next round (sc->round), in segments by source class.  Two
+// kernels: the count of each segment (into sc->window_count, zero since the previous window's
+// tail), then the placement, each segment at the sum of the counts before it.
+__global__ void __launch_bounds__(kThreads) k_window_count(RoundState a, uint32_t lo, uint32_t hi, const uint32_t* r_r0)
 {
 	__shared__ uint32_t s_cnt[kListSegments];
 	CallScalars* sc = a.sc;
 	const uint32_t round = sc->round;
-	const bool open = window_opens(sc, lo, hi, if_no_stop);
 	if (threadIdx.x < kListSegments)
 	{
 		s_cnt[threadIdx.x] = 0;
@@ -946,19 +1128,18 @@ __global__ void __launch_bounds__(kThreads) k_window_count(RoundState a, uint32_
 	}
 	__syncthreads();
 	const uint32_t k = lo + blockIdx.x * blockDim.x + threadIdx.x;
-	if (open && k < hi)
+	if (k < hi)
 		atomicAdd(&s_cnt[list_segment(a, r_r0[k])], 1u);
 	__syncthreads();
 	if (threadIdx.x < kListSegments && s_cnt[threadIdx.x])
 		atomicAdd(&sc->window_count[threadIdx.x], s_cnt[threadIdx.x]);
 }
 
-__global__ void __launch_bounds__(kThreads) k_window_open(RoundState a, uint32_t lo, uint32_t hi, const uint32_t* r_r0, const uint32_t* r_r1, bool if_no_stop)
+__global__ void __launch_bounds__(kThreads) k_window_open(RoundState a, uint32_t lo, uint32_t hi, const uint32_t* r_r0, const uint32_t* r_r1)
 {
 	__shared__ uint32_t s_off[kListSegments], s_cnt[kListSegments], s_base[kListSegments];
 	CallScalars* sc = a.sc;
 	const uint32_t round = sc->round;
-	const bool open = window_opens(sc, lo, hi, if_no_stop);
 	if (threadIdx.x < kListSegments)
 	{
 		uint32_t off = 0;
@@ -969,11 +1150,9 @@ __global__ void __launch_bounds__(kThreads) k_window_open(RoundState a, uint32_t
 		if (blockIdx.x == 0)
 			sc->list_off[threadIdx.x] = off;
 	}
-	if (if_no_stop && blockIdx.x == 0 && threadIdx.x == 0)
-		sc->extended = open ? 1u : 0u;
 	__syncthreads();
 	const uint32_t k = lo + blockIdx.x * blockDim.x + threadIdx.x;
-	const bool in = open && k < hi;
+	const bool in = k < hi;
 	const uint32_t r0 = in ? r_r0[k] : 0;
 	const uint32_t seg = list_segment(a, r0);
 	uint32_t local = 0;
@@ -987,12 +1166,12 @@ __global__ void __launch_bounds__(kThreads) k_window_open(RoundState a, uint32_t
 		a.list[round & 1][s_off[seg] + s_base[seg] + local] = make_uint4(k, r0, r_r1[k], 0);
 }
 
-void launch_window_extend(hipStream_t s, Mesh& m, size_t lo, size_t hi, bool if_no_stop)
+void launch_window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi)
 {
 	const unsigned int grid = grid_for(hi > lo ? hi - lo : 1);
 	const RoundState a = round_state(m);
-	k_window_count<<<grid, kThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_r0, if_no_stop);
-	k_window_open<<<grid, kThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_r0, m.r_r1, if_no_stop);
+	k_window_count<<<grid, kThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_r0);
+	k_window_open<<<grid, kThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_r0, m.r_r1);
 }
 
 // list_estimate sizes the grid (one rank per thread); the kernels stay correct for any length
@@ -1020,331 +1199,325 @@ void launch_round_tail(hipStream_t s, Mesh& m, int rel, uint32_t max_rounds, boo
 	k_round_tail<<<1, kTailThreads, 0, s>>>(round_state(m), (uint32_t)rel, max_rounds, deep);
 }
 
-// a failed flip test is a rejection unless a lower commit locked an endpoint first
-__global__ void k_resolve_flip_fail(uint8_t* status, const uint32_t* r_r0, const uint32_t* r_r1, const uint32_t* lock_rank, uint32_t lo, uint32_t hi)
-{
-	uint32_t k = lo + blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= hi || status[k] != kFlipFail)
-		return;
-	uint32_t l0 = lock_rank[r_r0[k]], l1 = lock_rank[r_r1[k]];
-	status[k] = ((l0 != kNone && l0 < k) || (l1 != kNone && l1 < k)) ? kSkipped : kRejected;
-}
-
-void launch_resolve(hipStream_t s, Mesh& m, size_t lo, size_t hi)
-{
-	if (hi > lo)
-		k_resolve_flip_fail<<<grid_for(hi - lo), kThreads, 0, s>>>(m.status, m.r_r0, m.r_r1, m.lock_rank, (uint32_t)lo, (uint32_t)hi);
-}
-
 // ------------------------------------------------------------------------------------------
 // stop scan: the first rank where the sequential loop breaks (src/simplifier.cpp:1517-1539)
 //   S1 err > error_limit
 //   S2 tri_collapses >= goal
 //   S3 err > 1.5 * err[goal/2 + rejects] && err > result_error && tri_collapses > goal/6
-// with tri_collapses, rejects and result_error the exclusive prefix sums / max of the
-// decided ranks.  Tiles of 4096 ranks: reduce, scan the tile aggregates, then test.
+// with tri_collapses, rejects and result_error the exclusive prefix sums / max of the decided
+// ranks.  Two kernels over tiles of ranks, each thread owning consecutive ones: the first settles
+// the failed flip tests and adds up its tile; in the second each workgroup adds the tiles before
+// its own, tests its ranks and leaves a record, and the workgroup that finishes last takes the
+// first record with a break.  14 us a pass at 200 k candidates, where settling, tile scan, totals and
+// finish as kernels of their own, with one block scan per 256 ranks, took 61.
 
 struct StopAgg
 {
-	uint32_t tri, rej, err;
+	uint32_t commit; // committed | border << 16
+	uint32_t other;  // rejected | skipped << 16
+	uint32_t err;    // bits of the largest committed error; a NaN stays out (its `<` test fails)
 };
 
-__device__ __forceinline__ StopAgg stop_item(uint8_t st, uint8_t k0, float err)
+constexpr int kStopWords = 5; // of a tile: committed, border, rejected, skipped, largest error
+
+__device__ __forceinline__ void stop_add(StopAgg& a, uint8_t st, float err)
 {
-	StopAgg a;
-	a.tri = st == kCommitted ? (k0 == kBorder ? 1u : 2u) : 0u;
-	a.rej = st == kRejected ? 1u : 0u;
-	// result_error keeps a NaN error out (its `<` test fails); errors are >= 0 otherwise
-	a.err = (st == kCommitted && err == err) ? __float_as_uint(err) : 0u;
-	return a;
+	a.commit += is_commit(st) ? (st == kCommittedBorder ? 0x10001u : 1u) : 0u;
+	a.other += st == kRejected ? 1u : (st == kSkipped ? 0x10000u : 0u);
+	const uint32_t e = is_commit(st) && err == err ? __float_as_uint(err) : 0u;
+	a.err = e > a.err ? e : a.err;
 }
 
-template <bool Max>
-__device__ __forceinline__ uint32_t wave_incl(uint32_t v)
+// a failed flip test is a rejection unless a lower commit locked an endpoint first
+__device__ __forceinline__ uint8_t settle(uint8_t st, uint32_t k, const uint32_t* r_r0, const uint32_t* r_r1, const uint32_t* lock_rank)
 {
-	const int lane = __lane_id();
+	if (st != kFlipFail)
+		return st;
+	const uint32_t l0 = lock_rank[r_r0[k]], l1 = lock_rank[r_r1[k]];
+	return ((l0 != kNone && l0 < k) || (l1 != kNone && l1 < k)) ? kSkipped : kRejected;
+}
+
+// thread t owns ranks [base, base + kItems): the status bytes of a full run as words
+template <int kItems>
+__device__ __forceinline__ void load_status(const uint8_t* status, uint32_t base, uint32_t count, uint8_t st[kItems])
+{
+	if (base + kItems <= count)
+	{
+#pragma unroll
+		for (int q = 0; q < kItems / 4; ++q)
+		{
+			const uint32_t w = reinterpret_cast<const uint32_t*>(status + base)[q];
+#pragma unroll
+			for (int b = 0; b < 4; ++b)
+				st[4 * q + b] = (uint8_t)(w >> (8 * b));
+		}
+	}
+	else
+	{
+#pragma unroll
+		for (int q = 0; q < kItems; ++q)
+			st[q] = base + q < count ? status[base + q] : (uint8_t)kUndecided;
+	}
+}
+
+template <int kItems>
+__global__ void __launch_bounds__(kThreads) k_stop_reduce(uint8_t* status, const float* r_err, const uint32_t* r_r0, const uint32_t* r_r1,
+                                                          const uint32_t* lock_rank, uint32_t count, uint32_t* tiles)
+{
+	__shared__ uint32_t red[kStopWords][kThreads / 64];
+	const uint32_t base = (blockIdx.x * kThreads + threadIdx.x) * kItems;
+	uint8_t st[kItems];
+	load_status<kItems>(status, base, count, st);
+	StopAgg acc{0, 0, 0};
+#pragma unroll
+	for (int q = 0; q < kItems; ++q)
+		if (base + q < count)
+		{
+			const uint8_t now = settle(st[q], base + q, r_r0, r_r1, lock_rank);
+			if (now != st[q])
+				status[base + q] = now;
+			stop_add(acc, now, r_err[base + q]);
+		}
+	const uint32_t v[kStopWords] = {acc.commit & 0xffffu, acc.commit >> 16, acc.other & 0xffffu, acc.other >> 16, acc.err};
+	const int wave = threadIdx.x >> 6;
+#pragma unroll
+	for (int q = 0; q < kStopWords; ++q)
+	{
+		const uint32_t x = q < 4 ? wave_sum(v[q]) : wave_max(v[q]);
+		if (__lane_id() == 0)
+			red[q][wave] = x;
+	}
+	__syncthreads();
+	if (threadIdx.x < kStopWords)
+	{
+		uint32_t x = 0;
+		for (int w = 0; w < kThreads / 64; ++w)
+		{
+			const uint32_t t = red[threadIdx.x][w];
+			x = threadIdx.x < 4 ? x + t : (t > x ? t : x);
+		}
+		tiles[(size_t)blockIdx.x * kStopWords + threadIdx.x] = x;
+	}
+}
+
+// words of a tile's record: the first stopping rank (kNone: none), then the totals below it (below
+// the tile's end when there is none) and the reason
+enum
+{
+	kRecRank,
+	kRecCommitted,
+	kRecBorder,
+	kRecRejected,
+	kRecSkipped,
+	kRecError,
+	kRecReason,
+	kRecWords
+};
+
+template <int kItems>
+__global__ void __launch_bounds__(kThreads) k_stop_find(const uint8_t* status, const float* r_err, uint32_t count, uint32_t cand_count, const uint32_t* tiles,
+                                                        uint32_t* records, uint32_t goal, float error_limit, CallScalars* sc)
+{
+	__shared__ uint32_t red[kStopWords][kThreads / 64];
+	__shared__ uint32_t before[kStopWords];
+	__shared__ uint32_t s_first, s_last;
+	const int wave = threadIdx.x >> 6, lane = __lane_id();
+	// the tiles before this one
+	{
+		uint32_t v[kStopWords] = {0, 0, 0, 0, 0};
+		for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kThreads)
+		{
+#pragma unroll
+			for (int q = 0; q < kStopWords; ++q)
+			{
+				const uint32_t t = tiles[(size_t)b * kStopWords + q];
+				v[q] = q < 4 ? v[q] + t : (t > v[q] ? t : v[q]);
+			}
+		}
+#pragma unroll
+		for (int q = 0; q < kStopWords; ++q)
+		{
+			const uint32_t x = q < 4 ? wave_sum(v[q]) : wave_max(v[q]);
+			if (lane == 0)
+				red[q][wave] = x;
+		}
+		if (threadIdx.x == 0)
+			s_first = kNone;
+		__syncthreads();
+		if (threadIdx.x < kStopWords)
+		{
+			uint32_t x = threadIdx.x < 4 ? 0u : __float_as_uint(sc->result_error);
+			for (int w = 0; w < kThreads / 64; ++w)
+			{
+				const uint32_t t = red[threadIdx.x][w];
+				x = threadIdx.x < 4 ? x + t : (t > x ? t : x);
+			}
+			before[threadIdx.x] = x;
+		}
+		__syncthreads();
+	}
+	// the ranks before this thread's inside the tile
+	const uint32_t base = (blockIdx.x * kThreads + threadIdx.x) * kItems;
+	uint8_t st[kItems];
+	float err[kItems];
+	load_status<kItems>(status, base, count, st);
+	StopAgg own{0, 0, 0};
+#pragma unroll
+	for (int q = 0; q < kItems; ++q)
+	{
+		err[q] = base + q < count ? r_err[base + q] : 0.f;
+		if (base + q < count)
+			stop_add(own, st[q], err[q]);
+	}
+	StopAgg in = own;
 #pragma unroll
 	for (int o = 1; o < 64; o <<= 1)
 	{
-		uint32_t t = __shfl_up(v, o, 64);
+		const uint32_t c = __shfl_up(in.commit, o, 64), r = __shfl_up(in.other, o, 64), e = __shfl_up(in.err, o, 64);
 		if (lane >= o)
-			v = Max ? (t > v ? t : v) : v + t;
+		{
+			in.commit += c;
+			in.other += r;
+			in.err = e > in.err ? e : in.err;
+		}
 	}
-	return v;
-}
-
-// exclusive block scan of three values (sum, sum, max) for 256 threads
-__device__ __forceinline__ StopAgg block_scan3(StopAgg v, StopAgg& total)
-{
-	__shared__ uint32_t lds[3][4];
-	uint32_t it = wave_incl<false>(v.tri);
-	uint32_t ir = wave_incl<false>(v.rej);
-	uint32_t ie = wave_incl<true>(v.err);
-	const int wave = threadIdx.x >> 6;
-	if (__lane_id() == 63)
+	if (lane == 63)
 	{
-		lds[0][wave] = it;
-		lds[1][wave] = ir;
-		lds[2][wave] = ie;
+		red[0][wave] = in.commit;
+		red[1][wave] = in.other;
+		red[2][wave] = in.err;
 	}
 	__syncthreads();
-	uint32_t bt = 0, br = 0, be = 0, at = 0, ar = 0, ae = 0;
+	uint32_t up = __shfl_up(in.err, 1, 64);
+	up = lane ? up : 0u;
+	uint32_t wc = 0, wo = 0, we = 0;
 #pragma unroll
-	for (int w = 0; w < 4; ++w)
-	{
-		uint32_t t = lds[0][w], r = lds[1][w], e = lds[2][w];
+	for (int w = 0; w < kThreads / 64; ++w)
 		if (w < wave)
 		{
-			bt += t;
-			br += r;
-			be = e > be ? e : be;
+			wc += red[0][w];
+			wo += red[1][w];
+			we = red[2][w] > we ? red[2][w] : we;
 		}
-		at += t;
-		ar += r;
-		ae = e > ae ? e : ae;
-	}
-	__syncthreads();
-	total = StopAgg{at, ar, ae};
-	// exclusive: inclusive minus own (sums); for the max, the inclusive value of the previous lane
-	uint32_t pe = __shfl_up(ie, 1, 64);
-	if (__lane_id() == 0)
-		pe = 0;
-	StopAgg ex;
-	ex.tri = bt + it - v.tri;
-	ex.rej = br + ir - v.rej;
-	ex.err = be > pe ? be : pe;
-	return ex;
-}
+	const uint32_t xc = wc + in.commit - own.commit, xo = wo + in.other - own.other;
+	uint32_t committed = before[0] + (xc & 0xffffu), border = before[1] + (xc >> 16);
+	uint32_t rejected = before[2] + (xo & 0xffffu), skipped = before[3] + (xo >> 16);
+	uint32_t best = before[4];
+	best = we > best ? we : best;
+	best = up > best ? up : best;
 
-__global__ void __launch_bounds__(kThreads) k_stop_reduce(const uint8_t* status, const uint32_t* r_v0, const uint8_t* kind, const float* r_err,
-                                                          size_t count, uint32_t* tiles, const CallScalars* sc, bool conditional)
-{
-	if (conditional && !sc->extended)
-		return;
-	size_t base = (size_t)blockIdx.x * kScanTile;
-	StopAgg acc{0, 0, 0};
-	for (int j = 0; j < kScanItems; ++j)
-	{
-		size_t k = base + (size_t)j * kThreads + threadIdx.x;
-		if (k < count)
-		{
-			StopAgg a = stop_item(status[k], kind[r_v0[k]], r_err[k]);
-			acc.tri += a.tri;
-			acc.rej += a.rej;
-			acc.err = a.err > acc.err ? a.err : acc.err;
-		}
-	}
-	StopAgg total;
-	block_scan3(acc, total);
-	if (threadIdx.x == 0)
-	{
-		tiles[blockIdx.x * 3 + 0] = total.tri;
-		tiles[blockIdx.x * 3 + 1] = total.rej;
-		tiles[blockIdx.x * 3 + 2] = total.err;
-	}
-}
-
-// single block: exclusive prefix of the tile aggregates; the max starts at the incoming result_error
-__global__ void __launch_bounds__(kThreads) k_stop_tiles(uint32_t* tiles, uint32_t ntiles, const CallScalars* sc, bool conditional)
-{
-	if (conditional && !sc->extended)
-		return;
-	StopAgg carry{0, 0, __float_as_uint(sc->result_error)};
-	for (uint32_t b = 0; b < ntiles; b += kThreads)
-	{
-		uint32_t i = b + threadIdx.x;
-		StopAgg v{0, 0, 0};
-		if (i < ntiles)
-			v = StopAgg{tiles[i * 3 + 0], tiles[i * 3 + 1], tiles[i * 3 + 2]};
-		StopAgg total;
-		StopAgg ex = block_scan3(v, total);
-		if (i < ntiles)
-		{
-			tiles[i * 3 + 0] = carry.tri + ex.tri;
-			tiles[i * 3 + 1] = carry.rej + ex.rej;
-			uint32_t e = ex.err > carry.err ? ex.err : carry.err;
-			tiles[i * 3 + 2] = e;
-		}
-		carry.tri += total.tri;
-		carry.rej += total.rej;
-		carry.err = total.err > carry.err ? total.err : carry.err;
-	}
-}
-
-__global__ void __launch_bounds__(kThreads) k_stop_find(const uint8_t* status, const uint32_t* r_v0, const uint8_t* kind, const float* r_err,
-                                                        size_t count, size_t cand_count, const uint32_t* tiles, uint32_t goal, float error_limit,
-                                                        CallScalars* sc, bool conditional)
-{
-	if (conditional && !sc->extended)
-		return;
-	size_t base = (size_t)blockIdx.x * kScanTile;
-	StopAgg carry{tiles[blockIdx.x * 3 + 0], tiles[blockIdx.x * 3 + 1], tiles[blockIdx.x * 3 + 2]};
 	const uint32_t half = goal / 2, sixth = goal / 6;
-	// ranks grow with the lane and the item, so a wavefront's first stopping rank is its minimum:
-	// one atomic per wavefront (stopping ranks form long runs; same-address atomics serialise)
-	bool found = false;
-	for (int j = 0; j < kScanItems; ++j)
-	{
-		size_t k = base + (size_t)j * kThreads + threadIdx.x;
-		StopAgg v{0, 0, 0};
-		float err = 0.f;
-		if (k < count)
-		{
-			err = r_err[k];
-			v = stop_item(status[k], kind[r_v0[k]], err);
-		}
-		StopAgg total;
-		StopAgg ex = block_scan3(v, total);
-		bool stop = false;
-		if (k < count)
-		{
-			uint32_t tri = carry.tri + ex.tri;
-			uint32_t rej = carry.rej + ex.rej;
-			uint32_t eb = ex.err > carry.err ? ex.err : carry.err;
-			float result_error = __uint_as_float(eb);
-			size_t eg = (size_t)half + rej;
-			float error_goal = eg < cand_count ? 1.5f * r_err[eg] : FLT_MAX;
-			stop = err > error_limit || tri >= goal || (err > error_goal && err > result_error && tri > sixth);
-		}
-		const uint64_t stops = __ballot(stop);
-		if (stops && !found)
-		{
-			found = true;
-			if (__lane_id() == (uint32_t)__builtin_ctzll(stops))
-				atomicMin(&sc->stop, (uint32_t)k);
-		}
-		carry.tri += total.tri;
-		carry.rej += total.rej;
-		carry.err = total.err > carry.err ? total.err : carry.err;
-	}
-}
-
-// totals below the stop rank (one atomic per workgroup and counter)
-__global__ void __launch_bounds__(kThreads) k_stop_totals(const uint8_t* status, const uint32_t* r_v0, const uint8_t* kind, const float* r_err,
-                                                          CallScalars* sc, bool conditional)
-{
-	if (conditional && !sc->extended)
-		return;
-	__shared__ uint32_t red[5][4];
-	uint32_t stop = sc->stop;
-	uint32_t v[5] = {0, 0, 0, 0, 0}; // committed, skipped, rejected, tri, max error bits
-	for (uint32_t k = blockIdx.x * kThreads + threadIdx.x; k < stop; k += gridDim.x * kThreads)
-	{
-		uint8_t st = status[k];
-		StopAgg a = stop_item(st, kind[r_v0[k]], r_err[k]);
-		v[0] += st == kCommitted;
-		v[1] += st == kSkipped;
-		v[2] += st == kRejected;
-		v[3] += a.tri;
-		v[4] = a.err > v[4] ? a.err : v[4];
-	}
+	uint32_t reason = 0, at = kNone;
 #pragma unroll
-	for (int o = 32; o > 0; o >>= 1)
+	for (int q = 0; q < kItems; ++q)
 	{
-#pragma unroll
-		for (int q = 0; q < 4; ++q)
-			v[q] += __shfl_xor(v[q], o, 64);
-		uint32_t t = __shfl_xor(v[4], o, 64);
-		v[4] = t > v[4] ? t : v[4];
-	}
-	const int wave = threadIdx.x >> 6;
-	if (__lane_id() == 0)
-		for (int q = 0; q < 5; ++q)
-			red[q][wave] = v[q];
-	__syncthreads();
-	if (threadIdx.x == 0)
-	{
-		uint32_t t[5] = {0, 0, 0, 0, 0};
-		for (int w = 0; w < kThreads / 64; ++w)
-		{
-			for (int q = 0; q < 4; ++q)
-				t[q] += red[q][w];
-			t[4] = red[4][w] > t[4] ? red[4][w] : t[4];
-		}
-		if (t[0])
-			atomicAdd(&sc->committed, t[0]);
-		if (t[1])
-			atomicAdd(&sc->skipped, t[1]);
-		if (t[2])
-			atomicAdd(&sc->rejected, t[2]);
-		if (t[3])
-			atomicAdd(&sc->tri_collapses, t[3]);
-		if (t[4])
-			atomicMax(&sc->work[1], t[4]);
-	}
-}
-
-__global__ void k_stop_finish(const float* r_err, uint32_t count, uint32_t goal, float error_limit, CallScalars* sc)
-{
-	uint32_t stop = sc->stop;
-	float prev = sc->result_error;
-	float best = __uint_as_float(sc->work[1]);
-	sc->result_error = prev < best ? best : prev;
-	uint32_t reason = 0;
-	if (stop < count)
-	{
-		float err = r_err[stop];
-		if (err > error_limit)
+		const uint32_t k = base + q;
+		if (k >= count || reason)
+			continue;
+		const uint32_t tri = 2 * committed - border;
+		if (err[q] > error_limit)
 			reason = 1;
-		else if (sc->tri_collapses >= goal)
+		else if (tri >= goal)
 			reason = 2;
-		else
-			reason = 3;
+		else if (tri > sixth && err[q] > __uint_as_float(best))
+		{
+			const size_t eg = (size_t)half + rejected;
+			const float error_goal = eg < cand_count ? 1.5f * r_err[eg] : FLT_MAX;
+			reason = err[q] > error_goal ? 3u : 0u;
+		}
+		if (reason)
+		{
+			at = k;
+			continue;
+		}
+		committed += is_commit(st[q]);
+		border += st[q] == kCommittedBorder;
+		rejected += st[q] == kRejected;
+		skipped += st[q] == kSkipped;
+		const uint32_t e = is_commit(st[q]) && err[q] == err[q] ? __float_as_uint(err[q]) : 0u;
+		best = e > best ? e : best;
 	}
-	sc->stop_reason = reason;
-}
-
-// undo commits at or past the stop rank: a commit wrote only its source class's wedges
-__global__ void k_revert(const uint8_t* status, const uint32_t* r_r0, const uint32_t* wedge, size_t count, const CallScalars* sc, uint32_t* cremap)
-{
-	size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= count || k < sc->stop || status[k] != kCommitted)
-		return;
-	uint32_t r = r_r0[k];
-	uint32_t v = r;
-	do
+	// ranks grow with the thread: the first stopping thread holds the tile's first stop; without one
+	// the last thread's totals are the tile's end
+	const uint64_t stops = __ballot(reason != 0);
+	if (stops && lane == __builtin_ctzll(stops))
+		atomicMin(&s_first, threadIdx.x);
+	__syncthreads();
+	const uint32_t owner = s_first != kNone ? s_first : kThreads - 1;
+	if (threadIdx.x == owner)
 	{
-		cremap[v] = v;
-		v = wedge[v];
-	} while (v != r);
-}
-
-__global__ void k_stop_reset(CallScalars* sc, uint32_t window, bool conditional)
-{
-	if (conditional && !sc->extended)
+		uint32_t* rec = records + (size_t)blockIdx.x * kRecWords;
+		const uint32_t w[kRecWords] = {at, committed, border, rejected, skipped, best, reason};
+#pragma unroll
+		for (int q = 0; q < kRecWords; ++q)
+			__hip_atomic_store(&rec[q], w[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		__threadfence();
+		s_last = atomicAdd(&sc->stop_done, 1u) + 1 == gridDim.x;
+	}
+	__syncthreads();
+	if (!s_last || threadIdx.x >= 64)
 		return;
-	sc->stop = window;
-	sc->committed = 0;
-	sc->skipped = 0;
-	sc->rejected = 0;
-	sc->tri_collapses = 0;
-	sc->work[1] = 0;
-}
-
-// repeatable: reads the decisions of ranks [0, window) and writes only the stop rank (window
-// if no rank in it breaks the loop) and the totals below it.  `conditional`: only when the window
-// was extended on the device (sc->extended), else every kernel leaves at once
-void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, uint32_t goal, float error_limit, bool conditional)
-{
-	k_stop_reset<<<1, 1, 0, s>>>(m.sc, (uint32_t)window, conditional);
-	if (!window)
+	if (threadIdx.x == 0)
+		sc->split = 0;
+	// the first record with a break, else the last tile's: one wavefront
+	__threadfence();
+	uint32_t hit = gridDim.x - 1;
+	for (uint32_t b0 = 0; b0 < gridDim.x; b0 += 64)
+	{
+		const uint32_t b = b0 + lane;
+		const bool found = b < gridDim.x && __hip_atomic_load(&records[(size_t)b * kRecWords + kRecRank], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != kNone;
+		const uint64_t m = __ballot(found);
+		if (m)
+		{
+			hit = b0 + (uint32_t)__builtin_ctzll(m);
+			break;
+		}
+	}
+	if (lane)
 		return;
-	unsigned int tiles = div_up(window, kScanTile);
-	k_stop_reduce<<<tiles, kThreads, 0, s>>>(m.status, m.r_v0, m.kind, m.r_err, window, m.stop_tile, m.sc, conditional);
-	k_stop_tiles<<<1, kThreads, 0, s>>>(m.stop_tile, tiles, m.sc, conditional);
-	k_stop_find<<<tiles, kThreads, 0, s>>>(m.status, m.r_v0, m.kind, m.r_err, window, cand_count, m.stop_tile, goal, error_limit, m.sc, conditional);
-	unsigned int blocks = div_up(window, kThreads * 4);
-	blocks = blocks < 1 ? 1 : (blocks > 512 ? 512 : blocks);
-	k_stop_totals<<<blocks, kThreads, 0, s>>>(m.status, m.r_v0, m.kind, m.r_err, m.sc, conditional);
+	uint32_t w[kRecWords];
+	for (int q = 0; q < kRecWords; ++q)
+		w[q] = __hip_atomic_load(&records[(size_t)hit * kRecWords + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	const bool more = w[kRecRank] == kNone && count < cand_count; // no break in the window: the host decides the rest
+	sc->stop_done = 0;
+	sc->extend = more;
+	sc->stop = w[kRecRank] == kNone ? count : w[kRecRank];
+	sc->stop_reason = w[kRecReason];
+	sc->committed = w[kRecCommitted];
+	sc->rejected = w[kRecRejected];
+	sc->skipped = w[kRecSkipped];
+	if (!more)
+	{
+		sc->result_error = __uint_as_float(w[kRecError]);
+	}
 }
 
-// once every rank of the window is decided: advance result_error and undo the commits at or
-// past the stop rank
-void launch_stop_commit(hipStream_t s, Mesh& m, size_t window, uint32_t goal, float error_limit)
+// repeatable: reads the decisions of ranks [0, window) and writes only the stop rank (window if no
+// rank in it breaks the loop), the totals below it and, unless the list goes on past a window
+// without a break (sc->extend), the pass's result error
+void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, uint32_t goal, float error_limit)
 {
-	k_stop_finish<<<1, 1, 0, s>>>(m.r_err, (uint32_t)window, goal, error_limit, m.sc);
-	if (window)
-		k_revert<<<grid_for(window), kThreads, 0, s>>>(m.status, m.r_r0, m.wedge, window, m.sc, m.cremap);
+	const uint32_t n = (uint32_t)window, c = (uint32_t)cand_count;
+	// four ranks a thread until the tiles would be many (each workgroup reads those before it)
+	const bool wide = window > (size_t)1024 * 1024;
+	const unsigned int tiles = div_up(window, (size_t)kThreads * (wide ? 16 : 4));
+	uint32_t* records = m.stop_tile + (size_t)kStopWords * tiles;
+	if (wide)
+	{
+		k_stop_reduce<16><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, m.r_r0, m.r_r1, m.lock_rank, n, m.stop_tile);
+		k_stop_find<16><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, n, c, m.stop_tile, records, goal, error_limit, m.sc);
+	}
+	else
+	{
+		k_stop_reduce<4><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, m.r_r0, m.r_r1, m.lock_rank, n, m.stop_tile);
+		k_stop_find<4><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, n, c, m.stop_tile, records, goal, error_limit, m.sc);
+	}
+}
+
+size_t stop_scan_words(size_t cand_count)
+{
+	// at most 1024 tiles of four ranks a thread, or tiles of sixteen
+	return (kStopWords + kRecWords) * ((size_t)div_up(cand_count, kThreads * 16) + 1026);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1412,137 +1585,274 @@ __device__ __forceinline__ uint32_t update_one(size_t k, const uint32_t* r_r0, c
 	return 0;
 }
 
-__global__ void k_update_quadrics(const uint8_t* status, const uint32_t* r_r0, const uint32_t* r_r1, const CallScalars* sc_in, const uint32_t* cremap,
-                                  const uint32_t* wedge, const float4* pos, int attr_count, Quad* vq, Grad* vg, Quad* aq, Grad* ag, CallScalars* sc)
+// After the stop is known, one launch over two ranges of workgroups that never touch each other's
+// state: the ranks (updateQuadrics), and the vertices, each of which
+//   - takes back a move at or past the stop (a commit wrote only its source class's wedges).  Other
+//     vertices read collapse_remap through settled_remap, which gives the same before and after;
+//   - remaps its edge loops (remapEdgeLoops, src/simplifier.cpp:1845-1864): collapse_remap is
+//     idempotent within a pass (targets are locked, never sources), so reading loop[l] before or
+//     after its own update gives the same result and the in-place loop becomes a double-buffered map;
+//   - as a primary, leaves its class's new id and adds the room its adjacency may need to its tile;
+//     as a secondary, checks that its class moves as one (every wedge of a seam or complex class
+//     goes into the target class unless its loops were inconsistent).
+struct ApplyArgs
 {
-	size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	const bool commit = k < sc_in->stop && status[k] == kCommitted;
-	// the largest positional error of the pass's commits (attribute path): one atomic per
-	// wavefront, so every lane stays to the reduction
-	uint32_t err_bits = 0;
-	if (commit)
-		err_bits = update_one(k, r_r0, r_r1, cremap, wedge, pos, attr_count, vq, vg, aq, ag);
-	if (attr_count)
-	{
-#pragma unroll
-		for (int o = 32; o > 0; o >>= 1)
-		{
-			uint32_t t = __shfl_xor(err_bits, o, 64);
-			err_bits = t > err_bits ? t : err_bits;
-		}
-		if (__lane_id() == 0 && err_bits)
-			atomicMax(&sc->vertex_error_bits, err_bits);
-	}
+	const uint8_t* status;
+	const uint32_t* r_r0;
+	const uint32_t* r_r1;
+	uint32_t* cremap;
+	const uint32_t* lock_rank;
+	const uint32_t* remap;
+	const uint32_t* wedge;
+	const float4* pos;
+	Quad* vq;
+	Grad* vg;
+	Quad* aq;
+	Grad* ag;
+	const uint32_t* loop_in;
+	const uint32_t* back_in;
+	uint32_t* loop_out;
+	uint32_t* back_out;
+	const uint2* range_in;
+	const uint2* adj_in;
+	uint2* range_out;
+	uint2* adj_out;
+	uint32_t* new_class;
+	uint2* sums;
+	CallScalars* sc;
+	int attr_count;
+	uint32_t ranks;
+	uint32_t rank_blocks;
+	uint32_t vertices;
+	uint32_t items;
+};
+
+__device__ __forceinline__ uint32_t settled_remap(const ApplyArgs& a, uint32_t v, uint32_t stop)
+{
+	const uint32_t c = a.cremap[v];
+	return c != v && a.lock_rank[a.remap[v]] >= stop ? v : c;
 }
 
-// remapEdgeLoops, src/simplifier.cpp:1845-1864.  collapse_remap is idempotent within a pass
-// (targets are locked, never sources), so reading loop[l] before or after its own update
-// gives the same result and the in-place loop becomes a double-buffered map.
-__global__ void k_remap_loops(const uint32_t* cremap, size_t n, const uint32_t* loop_in, uint32_t* loop_out, const uint32_t* back_in, uint32_t* back_out)
+__device__ __forceinline__ uint32_t remap_loop(const ApplyArgs& a, const uint32_t* in, uint32_t i, uint32_t stop)
 {
-	size_t ii = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (ii >= n)
-		return;
-	uint32_t i = (uint32_t)ii;
-	const uint32_t* in[2] = {loop_in, back_in};
-	uint32_t* out[2] = {loop_out, back_out};
-#pragma unroll
-	for (int q = 0; q < 2; ++q)
+	const uint32_t l = in[i];
+	if (l == kNone)
+		return kNone;
+	const uint32_t r = settled_remap(a, l, stop);
+	if (i != r)
+		return r;
+	const uint32_t ll = in[l];
+	return ll != kNone ? settled_remap(a, ll, stop) : kNone;
+}
+
+// the old adjacency lists a class's new one is made of: its own, and that of the class collapsed
+// into it this pass; none once it is collapsed itself (one commit at most touches a class)
+struct ClassLists
+{
+	uint2 own, other;
+	__device__ __forceinline__ uint32_t room() const
 	{
-		uint32_t l = in[q][i];
-		uint32_t res = kNone;
-		if (l != kNone)
+		return (own.y - own.x) + (other.y - other.x);
+	}
+};
+
+__device__ __forceinline__ ClassLists class_lists(const ApplyArgs& a, uint32_t v, uint32_t stop)
+{
+	ClassLists l;
+	l.own = a.range_in[v];
+	l.other = make_uint2(0, 0);
+	const uint32_t k = a.lock_rank[v];
+	if (k < stop)
+	{
+		const uint32_t source = a.r_r0[k];
+		if (source == v)
+			l.own = make_uint2(0, 0);
+		else
+			l.other = a.range_in[source];
+	}
+	return l;
+}
+
+__global__ void __launch_bounds__(kThreads) k_apply(ApplyArgs a)
+{
+	__shared__ uint2 red[kThreads / 64];
+	if (a.sc->extend)
+		return;
+	const uint32_t stop = a.sc->stop;
+	if (blockIdx.x < a.rank_blocks)
+	{
+		const uint32_t k = blockIdx.x * kThreads + threadIdx.x;
+		// the largest positional error of the pass's commits (attribute path): one atomic per
+		// wavefront, so every lane stays to the reduction
+		uint32_t err_bits = 0;
+		if (k < stop && is_commit(a.status[k]))
+			err_bits = update_one(k, a.r_r0, a.r_r1, a.cremap, a.wedge, a.pos, a.attr_count, a.vq, a.vg, a.aq, a.ag);
+		if (a.attr_count)
 		{
-			uint32_t r = cremap[l];
-			if (i == r)
+			err_bits = wave_max(err_bits);
+			if (__lane_id() == 0 && err_bits)
+				atomicMax(&a.sc->vertex_error_bits, err_bits);
+		}
+		return;
+	}
+	const uint32_t tile = blockIdx.x - a.rank_blocks;
+	uint2 room = make_uint2(0, 0);
+	for (uint32_t j = 0; j < a.items; ++j)
+	{
+		const uint32_t v = (tile * a.items + j) * kThreads + threadIdx.x;
+		if (v >= a.vertices)
+			break;
+		const uint32_t c = settled_remap(a, v, stop);
+		if (c != a.cremap[v])
+			a.cremap[v] = c;
+		a.loop_out[v] = remap_loop(a, a.loop_in, v, stop);
+		a.back_out[v] = remap_loop(a, a.back_in, v, stop);
+		const uint32_t r = a.remap[v];
+		if (r == v)
+		{
+			a.new_class[v] = a.remap[c];
+			room.x += class_lists(a, v, stop).room();
+		}
+		else if (a.remap[c] != a.remap[settled_remap(a, r, stop)])
+			a.sc->split = 1; // this wedge went elsewhere than its primary: the lists by class do not hold
+	}
+	room = block_sum2(room, red);
+	if (threadIdx.x == 0)
+		a.sums[tile] = room;
+}
+
+// The next pass's welded adjacency from this one's: a class's list is its old one and that of the
+// class collapsed into it, every entry through the classes' new ids, without the triangles that
+// have fallen together (the rule of the index remap).  The lists lie at the sum of the rooms before
+// them, so nothing is counted first and nothing is placed by atomics.  Lists of more than
+// kLongList entries are walked by the whole wavefront.  Icosphere L8, after its first pass (919 k
+// triangles left): 48 us, where counting by atomics, scan and fill took 176.
+constexpr uint32_t kLongList = 64;
+
+__device__ __forceinline__ bool entry_stays(uint32_t v, uint32_t x, uint32_t y)
+{
+	return x != y && x != v && y != v;
+}
+
+__global__ void __launch_bounds__(kThreads) k_adj_walk(ApplyArgs a)
+{
+	__shared__ uint2 red2[kThreads / 64];
+	__shared__ uint32_t red[kThreads / 64];
+	if (a.sc->extend)
+		return;
+	const uint32_t stop = a.sc->stop;
+	uint32_t at = sums_before(a.sums, blockIdx.x, red2).x;
+	const uint32_t lane = __lane_id();
+	for (uint32_t j = 0; j < a.items; ++j)
+	{
+		const uint32_t v = (blockIdx.x * a.items + j) * kThreads + threadIdx.x;
+		ClassLists l{make_uint2(0, 0), make_uint2(0, 0)};
+		if (v < a.vertices && a.remap[v] == v)
+			l = class_lists(a, v, stop);
+		const uint32_t room = l.room();
+		uint32_t total;
+		const uint32_t begin = at + block_scan(room, red, total);
+		uint32_t end = begin;
+		const bool longer = room > kLongList;
+		if (!longer)
+		{
+			for (int part = 0; part < 2; ++part)
 			{
-				uint32_t ll = in[q][l];
-				res = ll != kNone ? cremap[ll] : kNone;
+				const uint2 r = part ? l.other : l.own;
+				for (uint32_t p0 = r.x; p0 < r.y; p0 += 4)
+				{
+					uint2 e[4];
+#pragma unroll
+					for (int q = 0; q < 4; ++q)
+						e[q] = p0 + q < r.y ? a.adj_in[p0 + q] : make_uint2(v, v);
+					uint32_t x[4], y[4];
+#pragma unroll
+					for (int q = 0; q < 4; ++q)
+					{
+						x[q] = a.new_class[e[q].x];
+						y[q] = a.new_class[e[q].y];
+					}
+#pragma unroll
+					for (int q = 0; q < 4; ++q)
+						if (p0 + q < r.y && entry_stays(v, x[q], y[q]))
+							a.adj_out[end++] = make_uint2(x[q], y[q]);
+				}
 			}
-			else
-				res = r;
 		}
-		out[q][i] = res;
+		for (uint64_t left = __ballot(longer); left; left &= left - 1)
+		{
+			const int from = __builtin_ctzll(left);
+			const uint32_t w = __shfl(v, from, 64);
+			uint32_t to = __shfl(begin, from, 64);
+			for (int part = 0; part < 2; ++part)
+			{
+				const uint2 r = part ? l.other : l.own;
+				const uint32_t rb = __shfl(r.x, from, 64), re = __shfl(r.y, from, 64);
+				for (uint32_t p0 = rb; p0 < re; p0 += 64)
+				{
+					uint32_t x = w, y = w;
+					if (p0 + lane < re)
+					{
+						const uint2 e = a.adj_in[p0 + lane];
+						x = a.new_class[e.x];
+						y = a.new_class[e.y];
+					}
+					const bool stays = entry_stays(w, x, y);
+					const uint64_t m = __ballot(stays);
+					if (stays)
+						a.adj_out[to + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = make_uint2(x, y);
+					to += (uint32_t)__popcll(m);
+				}
+			}
+			if ((int)lane == from)
+				end = to;
+		}
+		if (v < a.vertices)
+			a.range_out[v] = make_uint2(begin, end);
+		at += total;
 	}
 }
 
-__global__ void k_vertex_error_from_result(CallScalars* sc)
+// the other set of index, loop and adjacency buffers is written; the caller makes it current once
+// the read-back says that the pass committed something
+void launch_apply(hipStream_t s, Mesh& m, size_t window, size_t tri_count)
 {
-	sc->vertex_error = sc->result_error;
-}
-
-__global__ void k_vertex_error_from_bits(CallScalars* sc)
-{
-	float v = __uint_as_float(sc->vertex_error_bits);
-	float prev = sc->vertex_error;
-	sc->vertex_error = prev < v ? v : prev;
-}
-
-void launch_apply(hipStream_t s, Mesh& m, size_t cand_count)
-{
-	if (cand_count)
-		k_update_quadrics<<<grid_for(cand_count), kThreads, 0, s>>>(m.status, m.r_r0, m.r_r1, m.sc, m.cremap, m.wedge, m.pos, (int)m.attr_count,
-		                                                           m.vq, m.vg, m.aq, m.ag, m.sc);
-	if (m.attr_count)
-		k_vertex_error_from_bits<<<1, 1, 0, s>>>(m.sc);
-	else
-		k_vertex_error_from_result<<<1, 1, 0, s>>>(m.sc);
-
-	int cur = m.loop_cur;
-	if (m.vertex_count)
-		k_remap_loops<<<grid_for(m.vertex_count), kThreads, 0, s>>>(m.cremap, m.vertex_count, m.loop[cur], m.loop[cur ^ 1], m.loopback[cur],
-		                                                          m.loopback[cur ^ 1]);
-	m.loop_cur = cur ^ 1;
-}
-
-// ------------------------------------------------------------------------------------------
-// remapIndexBuffer, src/simplifier.cpp:1811-1843: apply collapse_remap, drop triangles whose
-// primaries are no longer distinct, keep the survivors' order
-
-__device__ __forceinline__ bool remap_triangle(const uint32_t* ib, size_t t, const uint32_t* cremap, const uint32_t* remap, uint32_t v[3])
-{
-	v[0] = cremap[ib[t * 3 + 0]];
-	v[1] = cremap[ib[t * 3 + 1]];
-	v[2] = cremap[ib[t * 3 + 2]];
-	uint32_t r0 = remap[v[0]], r1 = remap[v[1]], r2 = remap[v[2]];
-	return r0 != r1 && r0 != r2 && r1 != r2;
-}
-
-__global__ void k_tri_keep(const uint32_t* ib, size_t tris, const uint32_t* cremap, const uint32_t* remap, uint32_t* keep)
-{
-	size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= tris)
-		return;
-	uint32_t v[3];
-	keep[t] = remap_triangle(ib, t, cremap, remap, v);
-}
-
-__global__ void k_tri_write(const uint32_t* ib, size_t tris, const uint32_t* cremap, const uint32_t* remap, const uint32_t* offsets, uint32_t* out)
-{
-	size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= tris)
-		return;
-	uint32_t v[3];
-	if (remap_triangle(ib, t, cremap, remap, v))
-	{
-		size_t o = (size_t)offsets[t] * 3;
-		out[o + 0] = v[0];
-		out[o + 1] = v[1];
-		out[o + 2] = v[2];
-	}
-}
-
-void launch_remap_triangles(hipStream_t s, Mesh& m, size_t tri_count)
-{
-	HIP_CHECK(hipMemsetAsync(&m.sc->next_triangles, 0, sizeof(uint32_t), s));
-	if (!tri_count)
-		return;
-	const uint32_t* in = m.ib[m.ib_cur];
-	uint32_t* out = m.ib[m.ib_cur ^ 1];
-	k_tri_keep<<<grid_for(tri_count), kThreads, 0, s>>>(in, tri_count, m.cremap, m.remap, m.tri_cnt);
-	scan_exclusive(s, m.tri_cnt, m.tri_off, tri_count, nullptr, &m.sc->next_triangles, m.temp);
-	k_tri_write<<<grid_for(tri_count), kThreads, 0, s>>>(in, tri_count, m.cremap, m.remap, m.tri_off, out);
-	m.ib_cur ^= 1;
+	ApplyArgs a;
+	a.status = m.status;
+	a.r_r0 = m.r_r0;
+	a.r_r1 = m.r_r1;
+	a.cremap = m.cremap;
+	a.lock_rank = m.lock_rank;
+	a.remap = m.remap;
+	a.wedge = m.wedge;
+	a.pos = m.pos;
+	a.vq = m.vq;
+	a.vg = m.vg;
+	a.aq = m.aq;
+	a.ag = m.ag;
+	a.loop_in = m.loop[m.loop_cur];
+	a.back_in = m.loopback[m.loop_cur];
+	a.loop_out = m.loop[m.loop_cur ^ 1];
+	a.back_out = m.loopback[m.loop_cur ^ 1];
+	a.range_in = m.adj_range[m.adj_cur];
+	a.adj_in = m.adj[m.adj_cur];
+	a.range_out = m.adj_range[m.adj_cur ^ 1];
+	a.adj_out = m.adj[m.adj_cur ^ 1];
+	a.new_class = m.new_class;
+	a.sums = m.tile_sums + tile_sum_words(0);
+	a.sc = m.sc;
+	a.attr_count = (int)m.attr_count;
+	a.ranks = (uint32_t)window;
+	a.rank_blocks = grid_for(window);
+	a.vertices = m.vertex_count;
+	a.items = tile_items(m.vertex_count);
+	const unsigned int tiles = div_up(m.vertex_count, (size_t)kThreads * a.items);
+	k_apply<<<a.rank_blocks + tiles, kThreads, 0, s>>>(a);
+	const TriArgs t = tri_args(m, tri_count, nullptr, m.loop_cur ^ 1);
+	const unsigned int tri_tiles = div_up(tri_count, (size_t)kThreads * t.items);
+	k_tri_count<true><<<tri_tiles, kThreads, 0, s>>>(t);
+	k_tri_write<true><<<tri_tiles, kThreads, 0, s>>>(t);
+	k_adj_walk<<<tiles, kThreads, 0, s>>>(a);
 }
 
 // ------------------------------------------------------------------------------------------

@@ -447,11 +447,11 @@ void launch_classify(hipStream_t s, Mesh& m, const uint32_t* raw_off, const uint
 	uint32_t* loop = m.loop[0];
 	uint32_t* loopback = m.loopback[0];
 	if (ni)
-		k_corner_adjacency<<<grid_for(ni), kThreads, 0, s>>>(m.ib[0], raw_corners, ni, m.adj);
-	k_open_edges<<<grid_for(n), kThreads, 0, s>>>(raw_off, m.adj, n, loop, loopback);
+		k_corner_adjacency<<<grid_for(ni), kThreads, 0, s>>>(m.ib[0], raw_corners, ni, m.adj[1]);
+	k_open_edges<<<grid_for(n), kThreads, 0, s>>>(raw_off, m.adj[1], n, loop, loopback);
 	k_classify_primary<<<grid_for(n), kThreads, 0, s>>>(m.remap, m.wedge, loop, loopback, n, m.kind);
 	if (options & kOptPermissive)
-		k_permissive<<<grid_for(n), kThreads, 0, s>>>(raw_off, m.adj, m.remap, m.wedge, vertex_lock, sparse_remap, n, m.kind);
+		k_permissive<<<grid_for(n), kThreads, 0, s>>>(raw_off, m.adj[1], m.remap, m.wedge, vertex_lock, sparse_remap, n, m.kind);
 	if (vertex_lock)
 		k_lock_mark<<<grid_for(n), kThreads, 0, s>>>(m.remap, vertex_lock, sparse_remap, n, m.kind);
 	k_kind_finalize<<<grid_for(n), kThreads, 0, s>>>(m.remap, n, options, m.kind);
@@ -628,7 +628,8 @@ void launch_rescale_attributes(hipStream_t s, Mesh& m, const float* attributes, 
 }
 
 // ------------------------------------------------------------------------------------------
-// vertex quadrics (src/simplifier.cpp:1057-1157).  One thread per primary r walks r's
+// vertex quadrics (src/simplifier.cpp:1057-1157), and the first pass's welded adjacency (the lists
+// are read here anyway).  One thread per primary r walks r's
 // corners in (triangle, corner) order and adds, as the reference's three sequential fills
 // do: every face quadric, then the regularising point quadric, then the border/seam edge
 // quadrics in (triangle, edge, endpoint) order.  No float atomics; each sum starts at +0.
@@ -650,12 +651,13 @@ __device__ __forceinline__ bool edge_loop_qualifies(const uint8_t* kind, const u
 
 __global__ void k_vertex_quadrics(const uint32_t* ib, const float4* pos, const uint32_t* remap, const uint8_t* kind, const uint32_t* loop,
                                   const uint32_t* loopback, const uint32_t* woff, const uint32_t* wcorners, const uint8_t* vertex_lock,
-                                  const uint32_t* sparse_remap, size_t n, float factor, Quad* vq, Grad* vg)
+                                  const uint32_t* sparse_remap, size_t n, float factor, Quad* vq, Grad* vg, uint2* adj_range, uint2* adj)
 {
 	size_t ri = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (ri >= n)
 		return;
 	uint32_t r = (uint32_t)ri;
+	adj_range[r] = make_uint2(woff[r], woff[r + 1]); // empty for a secondary: the lists are keyed by primaries
 	if (remap[r] != r)
 		return;
 
@@ -666,8 +668,11 @@ __global__ void k_vertex_quadrics(const uint32_t* ib, const float4* pos, const u
 
 	for (uint32_t p = begin; p < end; ++p)
 	{
-		uint32_t t = wcorners[p] / 3;
-		V3 p0 = load_pos(pos, ib[t * 3 + 0]), p1 = load_pos(pos, ib[t * 3 + 1]), p2 = load_pos(pos, ib[t * 3 + 2]);
+		const uint32_t t = wcorners[p] / 3, c = wcorners[p] - t * 3;
+		const uint32_t i0 = ib[t * 3 + 0], i1 = ib[t * 3 + 1], i2 = ib[t * 3 + 2];
+		V3 p0 = load_pos(pos, i0), p1 = load_pos(pos, i1), p2 = load_pos(pos, i2);
+		// the first pass's adjacency: the corner's next and previous classes
+		adj[p] = make_uint2(remap[c == 0 ? i1 : (c == 1 ? i2 : i0)], remap[c == 0 ? i2 : (c == 1 ? i0 : i1)]);
 		Quad F;
 		quad_from_triangle(F, p0, p1, p2, 1.f);
 		quad_add(Q, F);
@@ -731,7 +736,7 @@ void launch_vertex_quadrics(hipStream_t s, Mesh& m, const uint32_t* welded_off, 
 		return;
 	float factor = (options & kOptRegularizeLight) ? 1e-2f : ((options & kOptRegularize) ? 1e-1f : 1e-7f);
 	k_vertex_quadrics<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], m.pos, m.remap, m.kind, m.loop[0], m.loopback[0], welded_off, welded_corners,
-	                                                   vertex_lock, sparse_remap, n, factor, m.vq, m.vg);
+	                                                   vertex_lock, sparse_remap, n, factor, m.vq, m.vg, m.adj_range[0], m.adj[0]);
 }
 
 // attribute quadrics and gradients (src/simplifier.cpp:1159-1179), per wedge (not welded),

@@ -241,7 +241,7 @@ void launch_solve_setup(hipStream_t s, Mesh& m, const SolveBuffers& b, size_t re
 	launch_adjacency(s, m, result_count / 3);
 	k_solve_flags<<<grid_for(n), kThreads, 0, s>>>(b.update, m.remap, m.kind, n, b.listed);
 	launch_solve_decide(s, m, b);
-	k_solve_waiting<<<grid_for(n), kThreads, 0, s>>>(b.state, m.adj_off, m.adj, n, b.waiting, b.queue[0], &m.sc->work[5], m.sc);
+	k_solve_waiting<<<grid_for(n), kThreads, 0, s>>>(b.state, m.adj_off, m.adj[m.adj_cur], n, b.waiting, b.queue[0], &m.sc->work[5], m.sc);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -429,7 +429,7 @@ static SolveRound solve_round_args(Mesh& m, const SolveBuffers& b)
 	a.attr_count = (int)m.attr_count;
 	a.wedge = m.wedge;
 	a.adj_off = m.adj_off;
-	a.adj = m.adj;
+	a.adj = m.adj[m.adj_cur];
 	a.cand = b.cand;
 	a.state = b.state;
 	a.listed = b.listed;
