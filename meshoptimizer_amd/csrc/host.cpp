@@ -497,17 +497,15 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	m.tri_cnt = prune ? a.take<uint32_t>(T) : nullptr;
 	m.tri_off = prune ? a.take<uint32_t>(T) : nullptr;
 
-	m.c_v0 = a.take<uint32_t>(cap);
-	m.c_v1 = a.take<uint32_t>(cap);
+	m.c_v = a.take<uint2>(cap);
 	m.c_err = a.take<float>(cap);
+	m.rank_counts = a.take<uint32_t>(rank_sort_words(cap));
 	m.keys = a.take<uint32_t>(cap);
 	m.vals = a.take<uint32_t>(cap);
 	m.keys_alt = a.take<uint32_t>(cap);
 	m.vals_alt = a.take<uint32_t>(cap);
-	m.r_v0 = a.take<uint32_t>(cap);
-	m.r_v1 = a.take<uint32_t>(cap);
-	m.r_r0 = a.take<uint32_t>(cap);
-	m.r_r1 = a.take<uint32_t>(cap);
+	m.r_v = a.take<uint2>(cap);
+	m.r_class = a.take<uint2>(cap);
 	m.r_err = a.take<float>(cap);
 	m.src_rank = a.take<uint32_t>(cap);
 	m.src_val = a.take<uint32_t>(cap);
@@ -525,11 +523,11 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	p.v_c = a.take<uint32_t>(Vp);
 	p.v_d = a.take<uint32_t>(Vp);
 	p.raw_off = a.take<uint32_t>(Vp + 1);
-	p.raw_keys = m.r_v0;
-	p.raw_corners = m.r_v1;
+	p.raw_keys = reinterpret_cast<uint32_t*>(m.r_v);
+	p.raw_corners = p.raw_keys + cap;
 	p.w_off = a.take<uint32_t>(Vp + 1);
-	p.w_keys = m.r_r0;
-	p.w_corners = m.r_r1;
+	p.w_keys = reinterpret_cast<uint32_t*>(m.r_class);
+	p.w_corners = p.w_keys + cap;
 	p.i_alt0 = m.keys_alt;
 	p.i_alt1 = m.vals_alt;
 	p.kind_counts = a.take<uint32_t>(8);
@@ -544,7 +542,7 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	p.solve.state = solve ? a.take<uint8_t>(Vp + 8) : nullptr;
 
 	size_t biggest = std::max(std::max(I, cap), Vp + 1);
-	size_t temp_words = std::max(sort_temp_words(biggest), scan_temp_words(biggest + 16));
+	size_t temp_words = std::max(sort_temp_words(biggest), scan_temp_words(std::max(biggest + 16, rank_sort_words(cap))));
 	m.temp = a.take<uint32_t>(temp_words + 64);
 	m.sc = a.take<CallScalars>(1);
 }
@@ -825,7 +823,6 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		if (C == 0)
 			break;
 
-		launch_rank_sort(s, m, C);
 		uint32_t goal = (uint32_t)((result_count - c.target_index_count) / 3);
 
 		// rank window: the first pass guesses from the triangle goal, later passes from the
@@ -842,17 +839,18 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		// alternatives from round kDeepFromHead on, which decides ranks far earlier on such meshes
 		const int deep_heads = g_deep_heads.load(std::memory_order_relaxed), deep_from = g_deep_from_head.load(std::memory_order_relaxed);
 		bool deep = long_chains || learned > deep_heads || deep_heads < 0;
-		launch_perform_init(s, m, C, deep);
+		launch_rank_sort(s, m, C, W);
+		if (deep)
+			launch_source_lists(s, m, C);
 		// head rounds with one thread per rank of the window (the list only shrinks; workgroups
 		// past its current length leave at once, while a grid smaller than the list would make
-		// each thread walk several ranks' dependent gathers in turn), then the tail; their grid strides over any list length, so a grid capped at
-		// `max_threads` stays correct
-		auto window_rounds = [&](size_t lo, size_t hi, int head_base, int head_count, size_t max_threads) {
+		// each thread walk several ranks' dependent gathers in turn), then the tail
+		auto window_rounds = [&](size_t lo, size_t hi, int head_base, int head_count) {
 			for (int hd = 0; hd < head_count; ++hd)
-				launch_round(s, m, std::min(hi - lo, max_threads), head_base + hd, hd, deep && hd >= deep_from);
-			launch_round_tail(s, m, head_count, (uint32_t)(hi - lo + 2), deep);
+				launch_round(s, m, hi - lo, head_base + hd, hd + 1, deep && hd + 1 >= deep_from);
+			launch_round_tail(s, m, head_count + 1, (uint32_t)(hi - lo + 2), deep);
 		};
-		launch_window_open(s, m, 0, W);
+		launch_window_open(s, m, 0, W, true);
 		int heads_run = heads;
 		bool switched_deep = false;
 		if (!learned && W > kWholeWindow && heads)
@@ -866,11 +864,11 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 			for (;;)
 			{
 				for (int k = 0; k < batch && done < kMaxHeadRounds; ++k, ++done)
-					launch_round(s, m, W, done, done, deep && done >= deep_from);
+					launch_round(s, m, W, done, done + 1, deep && done + 1 >= deep_from);
 				sync_scalars(ctx, m);
 				uint32_t left = 0;
 				for (int q = 0; q < kListSegments; ++q)
-					left += h.list_count[(h.round + done) % 3][q];
+					left += h.list_count[(h.round + done + 1) % 3][q];
 				if (left < kTailStart || done >= kMaxHeadRounds)
 					break;
 				if (!deep && deep_heads >= 0 && done >= deep_heads && left >= kTailList)
@@ -881,10 +879,10 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 				batch = done;
 			}
 			heads_run = done;
-			launch_round_tail(s, m, done, (uint32_t)(W + 2), deep);
+			launch_round_tail(s, m, done + 1, (uint32_t)(W + 2), deep);
 		}
 		else
-			window_rounds(0, W, 0, heads, (size_t)-1);
+			window_rounds(0, W, 0, heads);
 		launch_stop_scan(s, m, W, C, goal, error_limit);
 		launch_apply(s, m, W, T);
 		sync_scalars(ctx, m);
@@ -895,8 +893,8 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		if (extended)
 		{
 			// the rest of the list
-			launch_window_open(s, m, W, C);
-			window_rounds(W, C, heads_run, ext_heads, (size_t)-1);
+			launch_window_open(s, m, W, C, false);
+			window_rounds(W, C, heads_run, ext_heads);
 			launch_stop_scan(s, m, C, C, goal, error_limit);
 			launch_apply(s, m, C, T);
 			sync_scalars(ctx, m);

@@ -61,18 +61,16 @@ struct Mesh
 	uint32_t* tri_cnt;       // per-triangle flags and offsets (Prune only)
 	uint32_t* tri_off;
 
-	uint32_t* c_v0;          // candidates in pick order
-	uint32_t* c_v1;
+	uint2* c_v;              // candidates in pick order
 	float* c_err;
-	uint32_t* keys;          // sort buffers
+	uint32_t* rank_counts;   // candidates per key value and tile (rank_sort_words)
+	uint32_t* keys;          // sort buffers of the set-up and the prune; rank slots of the source lists
 	uint32_t* vals;
 	uint32_t* keys_alt;
 	uint32_t* vals_alt;
 
-	uint32_t* r_v0;          // candidates in rank order
-	uint32_t* r_v1;
-	uint32_t* r_r0;          // remap[r_v0]: source class
-	uint32_t* r_r1;          // remap[r_v1]: target class
+	uint2* r_v;              // candidates in rank order
+	uint2* r_class;          // their source and target classes (remap of r_v)
 	float* r_err;
 	uint8_t* status;
 	uint4* list[2];          // undecided work lists: (rank, source class, target class, 0)
@@ -111,15 +109,16 @@ void launch_pick(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live 
 void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count);
 void launch_adjacency_ranges(hipStream_t s, Mesh& m, size_t tri_count);
 size_t tile_sum_words(size_t n); // entries of one m.tile_sums array (there are two)
-void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count);
-// commit state of a pass; with source_lists, also the candidate ranks grouped by source class
-// that deep rounds read
-void launch_perform_init(hipStream_t s, Mesh& m, size_t cand_count, bool source_lists);
+// errors and rank order of the candidates, the commit state of the pass, and the work-list counts of
+// the ranks below `window`
+void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count, size_t window);
+size_t rank_sort_words(size_t cand_count); // words of m.rank_counts
 void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count);
 void launch_pick_capacity(hipStream_t s, Mesh& m, size_t index_count);
 void launch_round(hipStream_t s, Mesh& m, size_t list_bound, int head_index, int rel, bool deep);
 void launch_round_tail(hipStream_t s, Mesh& m, int rel, uint32_t max_rounds, bool deep);
-void launch_window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi);
+// the list of ranks [lo, hi) and their first publishing round; the rounds that follow have rel >= 1
+void launch_window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi, bool counted);
 void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, uint32_t goal, float error_limit);
 size_t stop_scan_words(size_t cand_count); // words of m.stop_tile
 // what follows the stop of a pass whose window was [0, window), into the other set of loop, index

@@ -5,6 +5,8 @@
 #include "prims.h"
 #include "quadric.h"
 
+#include <algorithm>
+
 namespace mhip
 {
 
@@ -191,8 +193,7 @@ struct TriArgs
 	const uint32_t* loop;
 	const uint32_t* loopback;
 	uint2* sums; // (kept triangles, candidates) per tile
-	uint32_t* c_v0;
-	uint32_t* c_v1;
+	uint2* c_v;
 	float* c_err;
 	CallScalars* sc;
 	uint32_t tris;
@@ -326,8 +327,7 @@ __global__ void __launch_bounds__(kThreads) k_tri_write(TriArgs a)
 				for (uint32_t q = 0; q < 3; ++q)
 					if (q < count)
 					{
-						a.c_v0[c + q] = v0[q];
-						a.c_v1[c + q] = v1[q];
+						a.c_v[c + q] = make_uint2(v0[q], v1[q]);
 						a.c_err[c + q] = __uint_as_float(bd[q] ? 1u : 0u); // the two-way flag until ranked
 					}
 				// the taken triangle after which the next does not fit ends the list
@@ -359,8 +359,7 @@ static TriArgs tri_args(Mesh& m, size_t tri_count, const uint32_t* live, int loo
 	a.loop = m.loop[loop_set];
 	a.loopback = m.loopback[loop_set];
 	a.sums = m.tile_sums;
-	a.c_v0 = m.c_v0;
-	a.c_v1 = m.c_v1;
+	a.c_v = m.c_v;
 	a.c_err = m.c_err;
 	a.sc = m.sc;
 	a.tris = (uint32_t)tri_count;
@@ -390,7 +389,7 @@ void launch_pick_capacity(hipStream_t s, Mesh& m, size_t index_count)
 }
 
 // ------------------------------------------------------------------------------------------
-// rankEdgeCollapses, src/simplifier.cpp:1374-1450
+// rankEdgeCollapses, src/simplifier.cpp:1374-1450, and sortEdgeCollapses, 1452-1496
 
 __device__ __forceinline__ uint32_t complex_target(uint32_t v, uint32_t target, const uint32_t* remap, const uint32_t* loop, const uint32_t* loopback)
 {
@@ -426,14 +425,9 @@ __device__ __forceinline__ float attr_error(const RankArgs& a, uint32_t v, uint3
 	return quad_error_attr(load_quad(a.aq, v), a.ag + (size_t)v * A, A, load_pos(a.pos, t), a.va + (size_t)t * A);
 }
 
-__global__ void k_rank(RankArgs a, size_t count, uint32_t* c_v0, uint32_t* c_v1, float* c_err, uint32_t* keys, uint32_t* vals)
+// the error of candidate i0 -> i1, and of i1 -> i0 when the edge collapses both ways (else FLT_MAX)
+__device__ __forceinline__ float2 rank_errors(const RankArgs& a, uint32_t i0, uint32_t i1, bool bidi)
 {
-	size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (c >= count)
-		return;
-	uint32_t i0 = c_v0[c], i1 = c_v1[c];
-	bool bidi = __float_as_uint(c_err[c]) != 0;
-
 	float ei = quad_error(load_quad(a.vq, a.remap[i0]), load_pos(a.pos, i1));
 	float ej = bidi ? quad_error(load_quad(a.vq, a.remap[i1]), load_pos(a.pos, i0)) : FLT_MAX;
 
@@ -463,36 +457,207 @@ __global__ void k_rank(RankArgs a, size_t count, uint32_t* c_v0, uint32_t* c_v1,
 					ej += attr_error(a, v, complex_target(v, i0, a.remap, a.loop, a.loopback));
 		}
 	}
+	return make_float2(ei, ej);
+}
 
-	bool rev = bidi & (ej < ei);
-	float err = ej < ei ? ej : ei;
-	c_v0[c] = rev ? i1 : i0;
-	c_v1[c] = rev ? i0 : i1;
+// The sort by the 12-bit key is one stable counting pass over the key's 2560 values: the rank kernel
+// counts each tile of candidates in LDS, the scan of the (value, tile) counts gives every tile its
+// place in every value's run, and the scatter writes the ranked copies there directly.  Its
+// wavefronts own consecutive parts of the tile with a count of their own per value, so nothing
+// waits between 64 candidates and the next.  Icosphere L8's first pass, 2 M candidates: 85 us after
+// the rank, where two 8-bit digits with their scans and a gather of the ranked copies took 150 in
+// nine launches.
+constexpr int kKeyValues = 2560;
+constexpr int kRankThreads = 1024;
+constexpr int kScatterThreads = 512;
+constexpr int kScatterWaves = kScatterThreads / 64;
+
+// tiles large enough that the counts stay well below the candidates, small enough to fill the chip
+static uint32_t rank_tile(size_t cand_count)
+{
+	return cand_count <= 65536 ? 1024u : (cand_count <= 524288 ? 2048u : (cand_count <= 2097152 ? 4096u : 8192u));
+}
+
+// words of the counts for up to cand_count candidates (the largest of the steps of rank_tile below)
+size_t rank_sort_words(size_t cand_count)
+{
+	size_t tiles = div_up(cand_count ? cand_count : 1, rank_tile(cand_count));
+	for (size_t step : {(size_t)65536, (size_t)524288, (size_t)2097152})
+		if (cand_count > step)
+			tiles = std::max(tiles, (size_t)div_up(step, rank_tile(step)));
+	return tiles * kKeyValues;
+}
+
+// one candidate's error and orientation
+__device__ __forceinline__ float rank_one(const RankArgs& a, uint2* c_v, float* c_err, uint32_t c)
+{
+	const uint2 v = c_v[c];
+	const bool bidi = __float_as_uint(c_err[c]) != 0;
+	const float2 e = rank_errors(a, v.x, v.y, bidi);
+	const bool rev = bidi & (e.y < e.x);
+	const float err = e.y < e.x ? e.y : e.x;
+	if (rev)
+		c_v[c] = make_uint2(v.y, v.x);
 	c_err[c] = err;
-	keys[c] = collapse_sort_key(err);
-	vals[c] = (uint32_t)c;
+	return err;
 }
 
-__global__ void k_gather_ranked(const uint32_t* order, size_t count, const uint32_t* c_v0, const uint32_t* c_v1, const float* c_err,
-                                const uint32_t* remap, uint32_t* r_v0, uint32_t* r_v1, uint32_t* r_r0, uint32_t* r_r1, float* r_err, uint8_t* status)
+// the commit state of the pass (collapse_remap, locks, list counters), set up beside the ranking
+struct CommitInit
 {
-	size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (k >= count)
-		return;
-	status[k] = kUndecided;
-	uint32_t c = order[k];
-	uint32_t v0 = c_v0[c], v1 = c_v1[c];
-	r_v0[k] = v0;
-	r_v1[k] = v1;
-	r_r0[k] = remap[v0];
-	r_r1[k] = remap[v1];
-	r_err[k] = c_err[c];
+	uint32_t* cremap;
+	uint32_t* lock_rank;
+	uint32_t vertices;
+	CallScalars* sc;
+};
+
+__device__ __forceinline__ void commit_init(const CommitInit& i)
+{
+	if (blockIdx.x == 0 && threadIdx.x < kListSegments)
+	{
+		CallScalars* sc = i.sc;
+		sc->list_count[0][threadIdx.x] = 0;
+		sc->list_count[1][threadIdx.x] = 0;
+		sc->list_count[2][threadIdx.x] = 0;
+		sc->window_count[threadIdx.x] = 0;
+		if (threadIdx.x == 0)
+		{
+			sc->tail_rounds = 0;
+			sc->round = 0;
+		}
+	}
+	for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < i.vertices; v += gridDim.x * blockDim.x)
+	{
+		i.cremap[v] = v;
+		i.lock_rank[v] = kNone;
+	}
 }
 
-void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count)
+// Short lists: ranking and counting in one launch, a thread per candidate of the tile.  Longer ones
+// rank with a thread per candidate in small workgroups first (the gathers want the whole chip in
+// flight: 3.1 M candidates with attributes took 300 us from 383 workgroups of 1024 threads, 190 so).
+template <bool kRank>
+__global__ void __launch_bounds__(kRankThreads) k_rank_count(RankArgs a, CommitInit init, uint32_t count, uint32_t tile, uint2* c_v, float* c_err,
+                                                             uint32_t* counts)
 {
-	if (!cand_count)
-		return;
+	__shared__ uint32_t hist[kKeyValues];
+	for (uint32_t d = threadIdx.x; d < kKeyValues; d += kRankThreads)
+		hist[d] = 0;
+	if (kRank)
+		commit_init(init);
+	__syncthreads();
+	const uint32_t begin = blockIdx.x * tile, end = count - begin < tile ? count : begin + tile;
+	for (uint32_t c = begin + threadIdx.x; c < end; c += kRankThreads)
+		atomicAdd(&hist[collapse_sort_key(kRank ? rank_one(a, c_v, c_err, c) : c_err[c])], 1u);
+	__syncthreads();
+	for (uint32_t d = threadIdx.x; d < kKeyValues; d += kRankThreads)
+		counts[(size_t)d * gridDim.x + blockIdx.x] = hist[d];
+}
+
+__global__ void __launch_bounds__(kThreads) k_rank(RankArgs a, CommitInit init, uint32_t count, uint2* c_v, float* c_err)
+{
+	commit_init(init);
+	const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
+	if (c < count)
+		rank_one(a, c_v, c_err, c);
+}
+
+// list segment of a source class (see RoundState)
+__device__ __forceinline__ uint32_t list_segment(uint64_t seg_mul, uint32_t c)
+{
+	return (uint32_t)(((uint64_t)c * seg_mul) >> 32);
+}
+
+__global__ void __launch_bounds__(kScatterThreads) k_rank_scatter(const uint2* c_v, const float* c_err, const uint32_t* remap, uint32_t count, uint32_t tile,
+                                                                  const uint32_t* places, uint2* r_v, uint2* r_class, float* r_err, uint8_t* status,
+                                                                  uint32_t window, uint64_t seg_mul, CallScalars* sc)
+{
+	__shared__ uint32_t before[kScatterWaves][kKeyValues / 2]; // two 16-bit counts a word
+	__shared__ uint32_t place[kKeyValues];
+	__shared__ uint32_t seg[kListSegments];
+	const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+	for (uint32_t d = threadIdx.x; d < kScatterWaves * kKeyValues / 2; d += kScatterThreads)
+		(&before[0][0])[d] = 0;
+	for (uint32_t d = threadIdx.x; d < kKeyValues; d += kScatterThreads)
+		place[d] = places[(size_t)d * gridDim.x + blockIdx.x];
+	if (threadIdx.x < kListSegments)
+		seg[threadIdx.x] = 0;
+	__syncthreads();
+	const uint32_t part = tile / kScatterWaves, first = blockIdx.x * tile + wave * part;
+	const uint32_t end = first < count ? (count - first < part ? count : first + part) : first;
+	uint32_t* mine = before[wave];
+	for (uint32_t c = first + lane; c < end; c += 64)
+	{
+		const uint32_t key = collapse_sort_key(c_err[c]);
+		atomicAdd(&mine[key >> 1], key & 1 ? 0x10000u : 1u);
+	}
+	__syncthreads();
+	// each wavefront's counts become the sums of those before it
+	for (uint32_t d = threadIdx.x; d < kKeyValues / 2; d += kScatterThreads)
+	{
+		uint32_t run = 0;
+#pragma unroll
+		for (int w = 0; w < kScatterWaves; ++w)
+		{
+			const uint32_t n = before[w][d];
+			before[w][d] = run;
+			run += n;
+		}
+	}
+	__syncthreads();
+	uint32_t in_segment = 0; // lane q: this wavefront's ranks in the window and segment q
+	for (uint32_t c0 = first; c0 < end; c0 += 64)
+	{
+		const uint32_t c = c0 + lane;
+		const bool valid = c < end;
+		const float err = valid ? c_err[c] : 0.f;
+		const uint2 v = valid ? c_v[c] : make_uint2(0, 0);
+		const uint32_t key = collapse_sort_key(err), shift = key & 1 ? 16u : 0u;
+		const uint2 cls = valid ? make_uint2(remap[v.x], remap[v.y]) : make_uint2(0, 0);
+		uint64_t peers = __ballot(valid);
+#pragma unroll
+		for (int b = 0; b < 12; ++b)
+		{
+			const uint64_t set = __ballot((key >> b) & 1u);
+			peers &= ((key >> b) & 1u) ? set : ~set;
+		}
+		const uint32_t ahead = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+		const uint32_t rank = place[key] + ((mine[key >> 1] >> shift) & 0xffffu) + ahead;
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		if (valid && ahead == 0)
+			atomicAdd(&mine[key >> 1], (uint32_t)__popcll(peers) << shift);
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		__builtin_amdgcn_wave_barrier();
+		if (valid)
+		{
+			r_v[rank] = v;
+			r_class[rank] = cls;
+			r_err[rank] = err;
+			status[c] = kUndecided;
+		}
+		const uint32_t q = valid && rank < window ? list_segment(seg_mul, cls.x) : kNone;
+#pragma unroll
+		for (uint32_t k = 0; k < kListSegments; ++k)
+		{
+			const uint64_t m = __ballot(q == k);
+			in_segment += lane == k ? (uint32_t)__popcll(m) : 0u;
+		}
+	}
+	if (lane < kListSegments && in_segment)
+		atomicAdd(&seg[lane], in_segment);
+	__syncthreads();
+	if (threadIdx.x < kListSegments && seg[threadIdx.x])
+		atomicAdd(&sc->window_count[threadIdx.x], seg[threadIdx.x]);
+}
+
+static uint64_t segment_mul(const Mesh& m)
+{
+	return m.vertex_count ? ((uint64_t)kListSegments << 32) / m.vertex_count : 0;
+}
+
+void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count, size_t window)
+{
 	RankArgs a;
 	a.pos = m.pos;
 	a.va = m.va;
@@ -505,11 +670,19 @@ void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count)
 	a.kind = m.kind;
 	a.loop = m.loop[m.loop_cur];
 	a.loopback = m.loopback[m.loop_cur];
-	k_rank<<<grid_for(cand_count), kThreads, 0, s>>>(a, cand_count, m.c_v0, m.c_v1, m.c_err, m.keys, m.vals);
-	// sortEdgeCollapses (src/simplifier.cpp:1452-1496): stable by the 12-bit key, ties in pick order
-	radix_sort_pairs(s, m.keys, m.vals, m.keys_alt, m.vals_alt, cand_count, nullptr, 12, m.temp);
-	k_gather_ranked<<<grid_for(cand_count), kThreads, 0, s>>>(m.vals, cand_count, m.c_v0, m.c_v1, m.c_err, m.remap, m.r_v0, m.r_v1, m.r_r0,
-	                                                          m.r_r1, m.r_err, m.status);
+	const uint32_t tile = rank_tile(cand_count), n = (uint32_t)cand_count;
+	const unsigned int tiles = div_up(cand_count, tile);
+	const CommitInit init{m.cremap, m.lock_rank, m.vertex_count, m.sc};
+	if (tile == kRankThreads)
+		k_rank_count<true><<<tiles, kRankThreads, 0, s>>>(a, init, n, tile, m.c_v, m.c_err, m.rank_counts);
+	else
+	{
+		k_rank<<<grid_for(cand_count), kThreads, 0, s>>>(a, init, n, m.c_v, m.c_err);
+		k_rank_count<false><<<tiles, kRankThreads, 0, s>>>(a, init, n, tile, m.c_v, m.c_err, m.rank_counts);
+	}
+	scan_exclusive(s, m.rank_counts, m.rank_counts, (size_t)kKeyValues * tiles, nullptr, nullptr, m.temp);
+	k_rank_scatter<<<tiles, kScatterThreads, 0, s>>>(m.c_v, m.c_err, m.remap, n, tile, m.rank_counts, m.r_v, m.r_class, m.r_err, m.status,
+	                                                (uint32_t)window, segment_mul(m), m.sc);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -573,8 +746,7 @@ __device__ __forceinline__ uint8_t commit_collapse(uint32_t* cremap, uint32_t i0
 
 struct RoundState
 {
-	const uint32_t* r_v0;
-	const uint32_t* r_v1;
+	const uint2* r_v;
 	const uint2* adj_range; // a class's entries of adj: (begin, end)
 	const uint2* adj;
 	const float4* pos;
@@ -595,21 +767,17 @@ struct RoundState
 	                          // roles is the smaller of the two
 	uint4* list[2];           // work-list entries: (rank, source class, target class, 0)
 	CallScalars* sc;
-	uint64_t seg_mul;         // list segment of class c: (c * seg_mul) >> 32, below kListSegments
+	uint64_t seg_mul;         // list segment of class c: (c * seg_mul) >> 32, below kListSegments.
+	                          // Classes are numbered close to their neighbours in most meshes (grids,
+	                          // subdivided and locality-optimised meshes), so a segment's ranks touch
+	                          // mostly one range of the class arrays
 };
-
-// classes are numbered close to their neighbours in most meshes (grids, subdivided and
-// locality-optimised meshes), so a segment's ranks touch mostly one range of the class arrays
-__device__ __forceinline__ uint32_t list_segment(const RoundState& a, uint32_t c)
-{
-	return (uint32_t)(((uint64_t)c * a.seg_mul) >> 32);
-}
 
 // the value rank r's commit writes into collapse_remap[p], p the primary of its source class
 // (src/simplifier.cpp:1573-1605)
 __device__ __forceinline__ uint32_t commit_value_at(const RoundState& a, uint32_t r, uint32_t p)
 {
-	uint32_t i0 = a.r_v0[r], i1 = a.r_v1[r];
+	const uint32_t i0 = a.r_v[r].x, i1 = a.r_v[r].y;
 	uint8_t kd = a.kind[i0];
 	if (kd == kComplex)
 		return complex_target(p, i1, a.remap, a.loop, a.loopback);
@@ -856,7 +1024,8 @@ __device__ __forceinline__ bool round_x(const RoundState& a, uint4 w, uint32_t e
 	}
 	if (now == kFlipPass && low0 && low1)
 	{
-		a.status[k] = commit_collapse(a.cremap, a.r_v0[k], a.r_v1[k], a.kind, a.wedge, a.remap, a.loop, a.loopback);
+		const uint2 v = a.r_v[k];
+		a.status[k] = commit_collapse(a.cremap, v.x, v.y, a.kind, a.wedge, a.remap, a.loop, a.loopback);
 		a.lock_rank[r0] = k;
 		a.lock_rank[r1] = k;
 		return false;
@@ -1021,36 +1190,22 @@ __global__ void __launch_bounds__(kTailThreads) k_round_tail(RoundState a, uint3
 	}
 }
 
-__global__ void k_perform_init_scalars(CallScalars* sc)
-{
-	for (int q = 0; q < kListSegments; ++q)
-	{
-		sc->list_count[0][q] = 0;
-		sc->list_count[1][q] = 0;
-		sc->list_count[2][q] = 0;
-		sc->list_off[q] = 0;
-		sc->window_count[q] = 0;
-	}
-	sc->tail_rounds = 0;
-	sc->round = 0;
-}
-
 // candidate ranks grouped by source class (order inside a group is irrelevant): one atomic pass
 // counts the ranks per source class and hands each its slot in the class's group; after the scan
 // the fill places the ranks without atomics
-__global__ void k_src_count(const uint32_t* r_r0, size_t count, uint32_t* counts, uint32_t* slot)
+__global__ void k_src_count(const uint2* r_class, size_t count, uint32_t* counts, uint32_t* slot)
 {
 	size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (k < count)
-		slot[k] = atomicAdd(&counts[r_r0[k]], 1u);
+		slot[k] = atomicAdd(&counts[r_class[k].x], 1u);
 }
 
-__global__ void k_src_fill(RoundState a, const uint32_t* r_r0, size_t count, const uint32_t* slot, uint32_t* src_rank, uint32_t* src_val)
+__global__ void k_src_fill(RoundState a, const uint2* r_class, size_t count, const uint32_t* slot, uint32_t* src_rank, uint32_t* src_val)
 {
 	size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= count)
 		return;
-	uint32_t r0 = r_r0[k];
+	uint32_t r0 = r_class[k].x;
 	uint32_t at = a.src_off[r0] + slot[k];
 	src_rank[at] = (uint32_t)k;
 	src_val[at] = commit_value_at(a, (uint32_t)k, r0);
@@ -1059,8 +1214,7 @@ __global__ void k_src_fill(RoundState a, const uint32_t* r_r0, size_t count, con
 static RoundState round_state(Mesh& m)
 {
 	RoundState a;
-	a.r_v0 = m.r_v0;
-	a.r_v1 = m.r_v1;
+	a.r_v = m.r_v;
 	a.adj_range = m.adj_range[m.adj_cur];
 	a.adj = m.adj[m.adj_cur];
 	a.pos = m.pos;
@@ -1081,18 +1235,8 @@ static RoundState round_state(Mesh& m)
 		a.list[b] = m.list[b];
 	}
 	a.sc = m.sc;
-	a.seg_mul = m.vertex_count ? ((uint64_t)kListSegments << 32) / m.vertex_count : 0;
+	a.seg_mul = segment_mul(m);
 	return a;
-}
-
-void launch_perform_init(hipStream_t s, Mesh& m, size_t cand_count, bool source_lists)
-{
-	size_t n = m.vertex_count;
-	iota_u32(s, m.cremap, n);
-	fill_u32(s, m.lock_rank, kNone, n);
-	k_perform_init_scalars<<<1, 1, 0, s>>>(m.sc);
-	if (source_lists)
-		launch_source_lists(s, m, cand_count);
 }
 
 // the per-source candidate lists deep rounds read (they depend on the ranks alone, so they may
@@ -1103,75 +1247,132 @@ void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count)
 	fill_u32(s, m.src_off, 0, n + 1);
 	// the rank slots go to m.keys, free once the ranked copies are gathered
 	if (cand_count)
-		k_src_count<<<grid_for(cand_count), kThreads, 0, s>>>(m.r_r0, cand_count, m.src_off, m.keys);
+		k_src_count<<<grid_for(cand_count), kThreads, 0, s>>>(m.r_class, cand_count, m.src_off, m.keys);
 	scan_exclusive(s, m.src_off, m.src_off, n, nullptr, m.src_off + n, m.temp);
 	if (cand_count)
-		k_src_fill<<<grid_for(cand_count), kThreads, 0, s>>>(round_state(m), m.r_r0, cand_count, m.keys, m.src_rank, m.src_val);
+		k_src_fill<<<grid_for(cand_count), kThreads, 0, s>>>(round_state(m), m.r_class, cand_count, m.keys, m.src_rank, m.src_val);
 }
 
-// ranks [lo, hi) become the list of the next round (sc->round), in segments by source class.  Two
-// kernels: the count of each segment (into sc->window_count, zero since the previous window's
-// tail), then the placement, each segment at the sum of the counts before it.
-__global__ void __launch_bounds__(kThreads) k_window_count(RoundState a, uint32_t lo, uint32_t hi, const uint32_t* r_r0)
+// Ranks [lo, hi) become a work list, in segments by source class, and publish: the first round of a
+// window, in which no rank can do anything else.  sc->window_count holds the ranks per segment (the
+// scatter's counts; k_window_count's for the rest of a list); a workgroup takes its places with
+// one atomic per segment.  77 us for the 885 k ranks of icosphere L8's first window,
+// where a count and a placement of 256 ranks per workgroup, with LDS atomics on eight words, and
+// the publishing round took 268.
+constexpr int kOpenItems = 4;
+
+__device__ __forceinline__ uint32_t segment_of(const RoundState& a, uint32_t k, uint32_t hi, const uint2* r_class, uint2& cls)
 {
-	__shared__ uint32_t s_cnt[kListSegments];
-	CallScalars* sc = a.sc;
-	const uint32_t round = sc->round;
+	cls = k < hi ? r_class[k] : make_uint2(0, 0);
+	return k < hi ? list_segment(a.seg_mul, cls.x) : kNone;
+}
+
+template <int kOpenThreads>
+__global__ void __launch_bounds__(kOpenThreads) k_window_count(RoundState a, uint32_t lo, uint32_t hi, const uint2* r_class)
+{
+	__shared__ uint32_t seg[kListSegments];
 	if (threadIdx.x < kListSegments)
+		seg[threadIdx.x] = 0;
+	__syncthreads();
+	const uint32_t lane = __lane_id();
+	uint32_t n = 0;
+	for (int j = 0; j < kOpenItems; ++j)
 	{
-		s_cnt[threadIdx.x] = 0;
-		if (blockIdx.x == 0)
+		uint2 cls;
+		const uint32_t q = segment_of(a, lo + (blockIdx.x * kOpenItems + j) * kOpenThreads + threadIdx.x, hi, r_class, cls);
+#pragma unroll
+		for (uint32_t k = 0; k < kListSegments; ++k)
 		{
-			sc->list_count[round % 3][threadIdx.x] = 0; // filled by the placement
-			sc->list_count[(round + 1) % 3][threadIdx.x] = 0;
+			const uint64_t m = __ballot(q == k);
+			n += lane == k ? (uint32_t)__popcll(m) : 0u;
 		}
 	}
+	if (lane < kListSegments && n)
+		atomicAdd(&seg[lane], n);
 	__syncthreads();
-	const uint32_t k = lo + blockIdx.x * blockDim.x + threadIdx.x;
-	if (k < hi)
-		atomicAdd(&s_cnt[list_segment(a, r_r0[k])], 1u);
-	__syncthreads();
-	if (threadIdx.x < kListSegments && s_cnt[threadIdx.x])
-		atomicAdd(&sc->window_count[threadIdx.x], s_cnt[threadIdx.x]);
+	if (threadIdx.x < kListSegments && seg[threadIdx.x])
+		atomicAdd(&a.sc->window_count[threadIdx.x], seg[threadIdx.x]);
 }
 
-__global__ void __launch_bounds__(kThreads) k_window_open(RoundState a, uint32_t lo, uint32_t hi, const uint32_t* r_r0, const uint32_t* r_r1)
+template <int kOpenThreads>
+__global__ void __launch_bounds__(kOpenThreads) k_window_open(RoundState a, uint32_t lo, uint32_t hi, const uint2* r_class)
 {
-	__shared__ uint32_t s_off[kListSegments], s_cnt[kListSegments], s_base[kListSegments];
+	__shared__ uint32_t count[kOpenThreads / 64][kListSegments], start[kListSegments];
 	CallScalars* sc = a.sc;
-	const uint32_t round = sc->round;
+	const uint32_t round = sc->round, epoch = sc->epoch + 1;
+	const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
+	const uint64_t below = (1ull << lane) - 1ull;
+	uint2 cls[kOpenItems];
+	uint32_t seg[kOpenItems], at[kOpenItems];
+	uint32_t n = 0; // lane q: this wavefront's ranks of segment q so far
+#pragma unroll
+	for (int j = 0; j < kOpenItems; ++j)
+	{
+		seg[j] = segment_of(a, lo + (blockIdx.x * kOpenItems + j) * kOpenThreads + threadIdx.x, hi, r_class, cls[j]);
+		at[j] = __shfl(n, (int)(seg[j] & (kListSegments - 1)), 64);
+#pragma unroll
+		for (uint32_t k = 0; k < kListSegments; ++k)
+		{
+			const uint64_t m = __ballot(seg[j] == k);
+			at[j] += seg[j] == k ? (uint32_t)__popcll(m & below) : 0u;
+			n += lane == k ? (uint32_t)__popcll(m) : 0u;
+		}
+	}
+	if (lane < kListSegments)
+		count[wave][lane] = n;
+	__syncthreads();
 	if (threadIdx.x < kListSegments)
 	{
-		uint32_t off = 0;
+		uint32_t off = 0, total = 0;
 		for (uint32_t q = 0; q < threadIdx.x; ++q)
 			off += sc->window_count[q];
-		s_off[threadIdx.x] = off;
-		s_cnt[threadIdx.x] = 0;
+		for (int w = 0; w < kOpenThreads / 64; ++w)
+		{
+			const uint32_t c = count[w][threadIdx.x];
+			count[w][threadIdx.x] = total;
+			total += c;
+		}
+		start[threadIdx.x] = off + (total ? atomicAdd(&sc->list_count[(round + 1) % 3][threadIdx.x], total) : 0u);
 		if (blockIdx.x == 0)
 			sc->list_off[threadIdx.x] = off;
 	}
 	__syncthreads();
-	const uint32_t k = lo + blockIdx.x * blockDim.x + threadIdx.x;
-	const bool in = k < hi;
-	const uint32_t r0 = in ? r_r0[k] : 0;
-	const uint32_t seg = list_segment(a, r0);
-	uint32_t local = 0;
-	if (in)
-		local = atomicAdd(&s_cnt[seg], 1u);
-	__syncthreads();
-	if (threadIdx.x < kListSegments && s_cnt[threadIdx.x])
-		s_base[threadIdx.x] = atomicAdd(&sc->list_count[round % 3][threadIdx.x], s_cnt[threadIdx.x]);
-	__syncthreads();
-	if (in)
-		a.list[round & 1][s_off[seg] + s_base[seg] + local] = make_uint4(k, r0, r_r1[k], 0);
+	uint4* list = a.list[(round + 1) & 1];
+	unsigned long long* wr = (unsigned long long*)a.pend[epoch & 1];
+#pragma unroll
+	for (int j = 0; j < kOpenItems; ++j)
+	{
+		const uint32_t k = lo + (blockIdx.x * kOpenItems + j) * kOpenThreads + threadIdx.x;
+		if (k >= hi)
+			continue;
+		list[start[seg[j]] + count[wave][seg[j]] + at[j]] = make_uint4(k, cls[j].x, cls[j].y, 0);
+		const uint64_t key = round_key(epoch, k);
+		atomicMin(&wr[2 * (size_t)cls[j].x], (unsigned long long)key);
+		atomicMin(&wr[2 * (size_t)cls[j].y + 1], (unsigned long long)key);
+	}
 }
 
-void launch_window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi)
+template <int kOpenThreads>
+static void window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi, bool counted)
 {
-	const unsigned int grid = grid_for(hi > lo ? hi - lo : 1);
+	const unsigned int grid = div_up(hi > lo ? hi - lo : 1, (size_t)kOpenThreads * kOpenItems);
 	const RoundState a = round_state(m);
-	k_window_count<<<grid, kThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_r0);
-	k_window_open<<<grid, kThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_r0, m.r_r1);
+	if (!counted)
+		k_window_count<kOpenThreads><<<grid, kOpenThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_class);
+	k_window_open<kOpenThreads><<<grid, kOpenThreads, 0, s>>>(a, (uint32_t)lo, (uint32_t)hi, m.r_class);
+}
+
+// `counted`: the segments' counts are there already (launch_rank_sort's window).  Few ranks go to
+// small workgroups, so that the list is spread over the chip (60 k ranks in sixteen workgroups of
+// 1024 threads took 20 us); many go to large ones, for fewer atomics on the eight counters
+void launch_window_open(hipStream_t s, Mesh& m, size_t lo, size_t hi, bool counted)
+{
+	if (hi - lo <= 65536)
+		window_open<64>(s, m, lo, hi, counted);
+	else if (hi - lo <= 262144)
+		window_open<256>(s, m, lo, hi, counted);
+	else
+		window_open<1024>(s, m, lo, hi, counted);
 }
 
 // list_estimate sizes the grid (one rank per thread); the kernels stay correct for any length
@@ -1229,11 +1430,11 @@ __device__ __forceinline__ void stop_add(StopAgg& a, uint8_t st, float err)
 }
 
 // a failed flip test is a rejection unless a lower commit locked an endpoint first
-__device__ __forceinline__ uint8_t settle(uint8_t st, uint32_t k, const uint32_t* r_r0, const uint32_t* r_r1, const uint32_t* lock_rank)
+__device__ __forceinline__ uint8_t settle(uint8_t st, uint32_t k, const uint2* r_class, const uint32_t* lock_rank)
 {
 	if (st != kFlipFail)
 		return st;
-	const uint32_t l0 = lock_rank[r_r0[k]], l1 = lock_rank[r_r1[k]];
+	const uint32_t l0 = lock_rank[r_class[k].x], l1 = lock_rank[r_class[k].y];
 	return ((l0 != kNone && l0 < k) || (l1 != kNone && l1 < k)) ? kSkipped : kRejected;
 }
 
@@ -1261,7 +1462,7 @@ __device__ __forceinline__ void load_status(const uint8_t* status, uint32_t base
 }
 
 template <int kItems>
-__global__ void __launch_bounds__(kThreads) k_stop_reduce(uint8_t* status, const float* r_err, const uint32_t* r_r0, const uint32_t* r_r1,
+__global__ void __launch_bounds__(kThreads) k_stop_reduce(uint8_t* status, const float* r_err, const uint2* r_class,
                                                           const uint32_t* lock_rank, uint32_t count, uint32_t* tiles)
 {
 	__shared__ uint32_t red[kStopWords][kThreads / 64];
@@ -1273,7 +1474,7 @@ __global__ void __launch_bounds__(kThreads) k_stop_reduce(uint8_t* status, const
 	for (int q = 0; q < kItems; ++q)
 		if (base + q < count)
 		{
-			const uint8_t now = settle(st[q], base + q, r_r0, r_r1, lock_rank);
+			const uint8_t now = settle(st[q], base + q, r_class, lock_rank);
 			if (now != st[q])
 				status[base + q] = now;
 			stop_add(acc, now, r_err[base + q]);
@@ -1504,12 +1705,12 @@ void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, 
 	uint32_t* records = m.stop_tile + (size_t)kStopWords * tiles;
 	if (wide)
 	{
-		k_stop_reduce<16><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, m.r_r0, m.r_r1, m.lock_rank, n, m.stop_tile);
+		k_stop_reduce<16><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, m.r_class, m.lock_rank, n, m.stop_tile);
 		k_stop_find<16><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, n, c, m.stop_tile, records, goal, error_limit, m.sc);
 	}
 	else
 	{
-		k_stop_reduce<4><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, m.r_r0, m.r_r1, m.lock_rank, n, m.stop_tile);
+		k_stop_reduce<4><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, m.r_class, m.lock_rank, n, m.stop_tile);
 		k_stop_find<4><<<tiles, kThreads, 0, s>>>(m.status, m.r_err, n, c, m.stop_tile, records, goal, error_limit, m.sc);
 	}
 }
@@ -1541,10 +1742,10 @@ __device__ __forceinline__ uint32_t next_wedge_above(const uint32_t* wedge, uint
 
 // one committed collapse of k_update_quadrics; returns the bits of its non-NaN positional error
 // (non-negative floats order like their bits), 0 without attributes
-__device__ __forceinline__ uint32_t update_one(size_t k, const uint32_t* r_r0, const uint32_t* r_r1, const uint32_t* cremap, const uint32_t* wedge,
+__device__ __forceinline__ uint32_t update_one(size_t k, const uint2* r_class, const uint32_t* cremap, const uint32_t* wedge,
                                                const float4* pos, int attr_count, Quad* vq, Grad* vg, Quad* aq, Grad* ag)
 {
-	uint32_t r0 = r_r0[k], r1 = r_r1[k];
+	const uint32_t r0 = r_class[k].x, r1 = r_class[k].y;
 
 	Quad Q0 = load_quad(vq, r0);
 	Quad Q1 = load_quad(vq, r1);
@@ -1570,11 +1771,25 @@ __device__ __forceinline__ uint32_t update_one(size_t k, const uint32_t* r_r0, c
 			Quad Qt = load_quad(aq, t);
 			quad_add(Qt, load_quad(aq, v));
 			store_quad(aq, t, Qt);
-			for (int a = 0; a < A; ++a)
+			// four gradients at a time, all loads before the stores (which the compiler must take
+			// to alias them)
+			for (int a0 = 0; a0 < A; a0 += 4)
 			{
-				Grad g = ag[(size_t)t * A + a];
-				grad_add(g, ag[(size_t)v * A + a]);
-				ag[(size_t)t * A + a] = g;
+				Grad to[4], from[4];
+#pragma unroll
+				for (int q = 0; q < 4; ++q)
+				{
+					const int a = a0 + q < A ? a0 + q : A - 1;
+					to[q] = ag[(size_t)t * A + a];
+					from[q] = ag[(size_t)v * A + a];
+				}
+#pragma unroll
+				for (int q = 0; q < 4; ++q)
+					if (a0 + q < A)
+					{
+						grad_add(to[q], from[q]);
+						ag[(size_t)t * A + a0 + q] = to[q];
+					}
 			}
 		}
 
@@ -1598,8 +1813,7 @@ __device__ __forceinline__ uint32_t update_one(size_t k, const uint32_t* r_r0, c
 struct ApplyArgs
 {
 	const uint8_t* status;
-	const uint32_t* r_r0;
-	const uint32_t* r_r1;
+	const uint2* r_class;
 	uint32_t* cremap;
 	const uint32_t* lock_rank;
 	const uint32_t* remap;
@@ -1664,7 +1878,7 @@ __device__ __forceinline__ ClassLists class_lists(const ApplyArgs& a, uint32_t v
 	const uint32_t k = a.lock_rank[v];
 	if (k < stop)
 	{
-		const uint32_t source = a.r_r0[k];
+		const uint32_t source = a.r_class[k].x;
 		if (source == v)
 			l.own = make_uint2(0, 0);
 		else
@@ -1686,7 +1900,7 @@ __global__ void __launch_bounds__(kThreads) k_apply(ApplyArgs a)
 		// wavefront, so every lane stays to the reduction
 		uint32_t err_bits = 0;
 		if (k < stop && is_commit(a.status[k]))
-			err_bits = update_one(k, a.r_r0, a.r_r1, a.cremap, a.wedge, a.pos, a.attr_count, a.vq, a.vg, a.aq, a.ag);
+			err_bits = update_one(k, a.r_class, a.cremap, a.wedge, a.pos, a.attr_count, a.vq, a.vg, a.aq, a.ag);
 		if (a.attr_count)
 		{
 			err_bits = wave_max(err_bits);
@@ -1819,8 +2033,7 @@ void launch_apply(hipStream_t s, Mesh& m, size_t window, size_t tri_count)
 {
 	ApplyArgs a;
 	a.status = m.status;
-	a.r_r0 = m.r_r0;
-	a.r_r1 = m.r_r1;
+	a.r_class = m.r_class;
 	a.cremap = m.cremap;
 	a.lock_rank = m.lock_rank;
 	a.remap = m.remap;
