@@ -109,6 +109,9 @@ struct CallScalars
 	uint32_t list_off[kListSegments];      // where each segment starts in the list buffers
 	uint32_t window_count[kListSegments];  // ranks per segment of the window being opened (zero otherwise)
 	uint32_t dual_count;  // boundEdgeCollapses reduction
+	uint32_t kind_counts[6]; // primaries per kind, and all of them
+	uint32_t secondary_count; // vertices that are not their class's primary
+	uint32_t box_done;    // workgroups of the position gather that are done
 	uint32_t unique_count; // sparse remap: number of referenced vertices
 	uint32_t tail_rounds;   // rounds run by the single-workgroup tail of the commit
 	uint32_t component_count; // Prune: connected components of the welded mesh
@@ -148,6 +151,15 @@ __device__ __forceinline__ uint32_t ordered_key(float f)
 	if (u == 0x80000000u)
 		u = 0;
 	return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// waits until the wavefront's own global atomics and stores have been performed.  What a workgroup
+// hands to the one that finishes last goes through device-scope atomics, so this orders it before
+// the workgroup's count; a device-scope fence would write the whole L2 back instead (65 us for the
+// 512 workgroups of the position gather)
+__device__ __forceinline__ void wait_for_memory()
+{
+	asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 }
 
 // 64-bit minimum / maximum over the 64 lanes of a wavefront

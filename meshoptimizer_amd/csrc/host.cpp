@@ -435,7 +435,6 @@ struct Plan
 	uint32_t* w_corners;
 	uint32_t* i_alt0;
 	uint32_t* i_alt1;
-	uint32_t* kind_counts;
 	uint32_t* comp; // Prune: component per vertex
 	float* cerr;    // Prune: error per component
 	SolveBuffers solve; // meshopt_simplifyWithUpdate only
@@ -530,7 +529,6 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	p.w_corners = p.w_keys + cap;
 	p.i_alt0 = m.keys_alt;
 	p.i_alt1 = m.vals_alt;
-	p.kind_counts = a.take<uint32_t>(8);
 	p.comp = prune ? a.take<uint32_t>(Vp) : nullptr;
 	p.cerr = prune ? a.take<float>(Vp) : nullptr;
 	p.solve.update = solve ? a.take<uint8_t>(Vp + 8) : nullptr;
@@ -548,42 +546,6 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 }
 
 // ------------------------------------------------------------------------------------------
-
-__global__ void __launch_bounds__(256) k_count_kinds(const uint32_t* remap, const uint8_t* kind, size_t n, uint32_t* counts)
-{
-	__shared__ uint32_t h[6];
-	if (threadIdx.x < 6)
-		h[threadIdx.x] = 0;
-	__syncthreads();
-	uint32_t local[6] = {0, 0, 0, 0, 0, 0};
-	for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-		if (remap[i] == (uint32_t)i)
-		{
-			uint8_t k = kind[i];
-			local[k < 5 ? k : 4]++;
-			local[5]++;
-		}
-	for (int q = 0; q < 6; ++q)
-	{
-		uint32_t v = local[q];
-		for (int o = 32; o > 0; o >>= 1)
-			v += __shfl_xor(v, o, 64);
-		if (__lane_id() == 0 && v)
-			atomicAdd(&h[q], v);
-	}
-	__syncthreads();
-	if (threadIdx.x < 6 && h[threadIdx.x])
-		atomicAdd(&counts[threadIdx.x], h[threadIdx.x]);
-}
-
-__global__ void k_scalars_init(CallScalars* sc)
-{
-	sc->result_error = 0.f;
-	sc->vertex_error_bits = 0u;
-	sc->candidates = 0;
-	sc->dual_count = 0;
-	sc->work[2] = 0;
-}
 
 static float host_float_bits(uint32_t u)
 {
@@ -719,22 +681,22 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	m.epoch = 0;
 
 	t_read_backs = 0;
-	HIP_CHECK(hipMemsetAsync(m.sc, 0, sizeof(CallScalars), s));
-	k_scalars_init<<<1, 1, 0, s>>>(m.sc);
-	if (I)
-	{
-		HIP_CHECK(hipMemcpyAsync(m.ib[0], c.indices, I * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
-		// every later gather trusts the indices: reject out-of-range ones before any kernel uses them
-		launch_check_indices(s, m.ib[0], I, V_in, &m.sc->work[2]);
-		sync_scalars(ctx, m);
+	// one read-back after the checks and the position remap: the index check, the sparse remap's
+	// vertex count (which its own read-back brings earlier) and the number of secondary vertices
+	launch_call_init(s, m.sc, plan.raw_off, V_alloc + 1);
+	launch_load_indices(s, c.indices, m.ib[0], I, V_in, sparse ? nullptr : plan.raw_off, plan.i_alt0, &m.sc->work[2]);
+	auto check_indices = [&]() {
 		if (ctx.sc_host->work[2])
 			throw std::invalid_argument("index buffer references a vertex >= vertex_count");
-	}
+	};
 
 	size_t V = V_in;
 	const uint32_t* sparse_remap = nullptr;
 	if (sparse)
 	{
+		// every later gather trusts the indices: reject out-of-range ones before any kernel uses them
+		sync_scalars(ctx, m);
+		check_indices();
 		launch_sparse_remap(s, m.ib[0], m.ib[0], I, V_in, plan.sp_first, plan.sp_flags, plan.sp_dense, plan.sparse_remap, &m.sc->unique_count, m.temp);
 		sync_scalars(ctx, m);
 		V = I ? ctx.sc_host->unique_count : 0;
@@ -742,14 +704,18 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	}
 	m.vertex_count = (uint32_t)V;
 
-	launch_gather_positions(s, c.positions, c.position_stride / sizeof(float), sparse_remap, m.praw, V);
-	launch_position_remap(s, m, plan.table, pow2_at_least(2 * V + 2));
-	launch_wedges(s, m, plan.v_flags, plan.v_a, plan.v_b, plan.v_c, plan.v_d);
+	const size_t table_size = pow2_at_least(2 * V + 2);
+	launch_gather_positions(s, m, c.positions, c.position_stride / sizeof(float), sparse_remap, plan.table, table_size);
+	launch_position_remap(s, m, plan.table, table_size);
+	sync_scalars(ctx, m);
+	check_indices();
+	const size_t secondaries = ctx.sc_host->secondary_count;
+	launch_wedges(s, m, secondaries, plan.v_flags, plan.v_a, plan.v_b, plan.v_c, plan.v_d);
 
-	launch_corner_csr(s, m.ib[0], I, nullptr, V, plan.raw_off, plan.raw_keys, plan.raw_corners, plan.i_alt0, plan.i_alt1, m.temp);
-	launch_classify(s, m, plan.raw_off, plan.raw_corners, c.lock, sparse_remap, c.options);
+	const bool permissive = (c.options & kOptPermissive) != 0;
+	launch_corner_lists(s, m, !sparse, permissive, plan.raw_off, plan.i_alt0, plan.raw_keys, plan.raw_corners);
+	launch_classify(s, m, plan.raw_off, secondaries != 0, c.lock, sparse_remap, c.options);
 
-	launch_rescale(s, m);
 	if (A)
 		launch_rescale_attributes(s, m, c.attributes, c.attribute_stride / sizeof(float), sparse_remap, amap, aw);
 	if (prune)
@@ -761,28 +727,19 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		launch_measure_components(s, m, plan.comp, plan.cerr, scratch);
 	}
 
-	launch_corner_csr(s, m.ib[0], I, m.remap, V, plan.w_off, plan.w_keys, plan.w_corners, plan.i_alt0, plan.i_alt1, m.temp);
-	HIP_CHECK(hipMemsetAsync(m.vq, 0, (V + 1) * sizeof(Quad), s));
-	launch_vertex_quadrics(s, m, plan.w_off, plan.w_corners, c.lock, sparse_remap, c.options);
+	const uint32_t *w_off = plan.raw_off, *w_corners = plan.raw_corners;
+	if (secondaries)
+	{
+		launch_welded_corner_lists(s, m, plan.w_off, plan.i_alt0, plan.w_keys, plan.w_corners);
+		w_off = plan.w_off;
+		w_corners = plan.w_corners;
+	}
+	launch_vertex_quadrics(s, m, w_off, w_corners, c.lock, sparse_remap, c.options);
 	if (A)
 		launch_attribute_quadrics(s, m, plan.raw_off, plan.raw_corners);
 
 	// attribute quadrics read the raw corner list; everything after may reuse its space
-	launch_dual_count(s, m, plan.raw_off);
-	HIP_CHECK(hipMemsetAsync(plan.kind_counts, 0, 8 * sizeof(uint32_t), s));
-	if (V)
-		k_count_kinds<<<std::min(div_up(V, 256 * 8), 512u), 256, 0, s>>>(m.remap, m.kind, V, plan.kind_counts);
-	uint32_t kind_counts[8];
-	HIP_CHECK(hipMemcpyAsync(kind_counts, plan.kind_counts, sizeof(kind_counts), hipMemcpyDeviceToHost, s));
-
-	// round minima start as "no entry" (tag of epoch 0, rank all-ones)
-	for (int b = 0; b < 2; ++b)
-	{
-		HIP_CHECK(hipMemsetAsync(m.pend[b], 0xff, 2 * (V + 1) * sizeof(uint64_t), s));
-	}
-
 	// the first pass's candidates go before the set-up read-back, which returns their count
-	launch_pick_capacity(s, m, I);
 	if (I)
 		launch_pick(s, m, I / 3);
 
@@ -792,9 +749,9 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	ctx.window_fraction = 0;
 	t_call = meshopt_hip_call_stats{};
 	t_call.vertex_count = (unsigned int)V;
-	t_call.unique_positions = kind_counts[5];
+	t_call.unique_positions = h.kind_counts[5];
 	for (int k = 0; k < 5; ++k)
-		t_call.kinds[k] = kind_counts[k];
+		t_call.kinds[k] = h.kind_counts[k];
 	t_passes.clear();
 
 	m.capacity = h.pick_capacity;
@@ -1283,8 +1240,8 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 	}
 
 	// rescalePositions (src/simplifier.cpp:549-603)
-	if (V)
-		launch_gather_positions(s, positions, stride / sizeof(float), nullptr, m.praw, V);
+	launch_call_init(s, m.sc, nullptr, 0);
+	launch_gather_positions(s, m, positions, stride / sizeof(float), nullptr, nullptr, 0);
 	launch_rescale(s, m);
 	// the extent meshopt_simplifyScale returns for the same vertices (rescalePositions, without the
 	// rescale), asked for by the clusterlod fallback
@@ -2671,8 +2628,8 @@ extern "C" float meshopt_simplifyScale(const float* vertex_positions, size_t ver
 		m.praw = reinterpret_cast<float4*>(d + off_p);
 		m.sc = reinterpret_cast<CallScalars*>(d + off_sc);
 		m.vertex_count = (uint32_t)vertex_count;
-		launch_gather_positions(s, reinterpret_cast<const float*>(d), vertex_positions_stride / 4, nullptr, m.praw, vertex_count);
-		launch_extent_only(s, m);
+		launch_call_init(s, m.sc, nullptr, 0);
+		launch_gather_positions(s, m, reinterpret_cast<const float*>(d), vertex_positions_stride / 4, nullptr, nullptr, 0);
 		HIP_CHECK(hipMemcpyAsync(ctx.sc_host, m.sc, sizeof(CallScalars), hipMemcpyDeviceToHost, s));
 		HIP_CHECK(hipStreamSynchronize(s));
 		return ctx.sc_host->extent;

@@ -84,21 +84,34 @@ struct Mesh
 void launch_check_indices(hipStream_t s, const uint32_t* ib, size_t index_count, size_t vertex_count, uint32_t* flag);
 void launch_sparse_remap(hipStream_t s, const uint32_t* indices_in, uint32_t* indices_out, size_t index_count, size_t vertex_count,
                          uint32_t* first, uint32_t* flags, uint32_t* dense, uint32_t* sparse_remap, uint32_t* unique_count, uint32_t* temp);
-void launch_gather_positions(hipStream_t s, const float* positions, size_t stride_floats, const uint32_t* sparse_remap, float4* out, size_t vertex_count);
+// sc as at the start of a call, and n zero words at `zeroed`
+void launch_call_init(hipStream_t s, CallScalars* sc, uint32_t* zeroed, size_t n);
+// a copy of the indices; an index >= vertex_count sets the flag.  With `counts` (zero before), the
+// corners per vertex, and in `slot` each corner's place among its vertex's
+void launch_load_indices(hipStream_t s, const uint32_t* in, uint32_t* out, size_t index_count, size_t vertex_count, uint32_t* counts, uint32_t* slot,
+                         uint32_t* flag);
+// m.praw, the box and the extent (m.sc as launch_call_init leaves it), and an empty hash table
+void launch_gather_positions(hipStream_t s, Mesh& m, const float* positions, size_t stride_floats, const uint32_t* sparse_remap, uint32_t* table,
+                             size_t table_size);
+// m.remap, m.pos, sc->secondary_count; wedge rings of one vertex each and empty round minima
 void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size);
-void launch_wedges(hipStream_t s, Mesh& m, uint32_t* flags, uint32_t* scratch_a, uint32_t* scratch_b, uint32_t* scratch_c, uint32_t* scratch_d);
-void launch_corner_csr(hipStream_t s, const uint32_t* ib, size_t index_count, const uint32_t* remap, size_t vertex_count,
-                       uint32_t* offsets, uint32_t* keys, uint32_t* corners, uint32_t* keys_alt, uint32_t* vals_alt, uint32_t* temp);
-void launch_classify(hipStream_t s, Mesh& m, const uint32_t* raw_off, const uint32_t* raw_corners, const uint8_t* vertex_lock,
-                     const uint32_t* sparse_remap, uint32_t options);
+// the wedge rings of the classes with secondaries (their count as read back)
+void launch_wedges(hipStream_t s, Mesh& m, size_t secondaries, uint32_t* flags, uint32_t* scratch_a, uint32_t* scratch_b, uint32_t* scratch_c, uint32_t* scratch_d);
+// each vertex's corners in corner order (offsets: V + 1 words) and its open edges (m.loop[0],
+// m.loopback[0]); `counted`: offsets and slot as launch_load_indices left them, else offsets zero.
+// with_adjacency: (next, prev) per listed corner in m.adj[1], for launch_classify under Permissive
+void launch_corner_lists(hipStream_t s, Mesh& m, bool counted, bool with_adjacency, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners);
+// the same lists by class (no open edges); without secondaries they are the vertices' own
+void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners);
+// m.kind, sc->kind_counts and sc->dual_count
+void launch_classify(hipStream_t s, Mesh& m, const uint32_t* raw_off, bool secondaries, const uint8_t* vertex_lock, const uint32_t* sparse_remap,
+                     uint32_t options);
 void launch_rescale(hipStream_t s, Mesh& m);
-void launch_extent_only(hipStream_t s, Mesh& m);
 void launch_rescale_attributes(hipStream_t s, Mesh& m, const float* attributes, size_t stride_floats, const uint32_t* sparse_remap,
                                const uint32_t* attr_index, const float* attr_weight);
 void launch_vertex_quadrics(hipStream_t s, Mesh& m, const uint32_t* welded_off, const uint32_t* welded_corners, const uint8_t* vertex_lock,
                             const uint32_t* sparse_remap, uint32_t options);
 void launch_attribute_quadrics(hipStream_t s, Mesh& m, const uint32_t* raw_off, const uint32_t* raw_corners);
-void launch_dual_count(hipStream_t s, Mesh& m, const uint32_t* raw_off);
 
 // ---------------------------------------------------------------- passes (pass.hip)
 // the candidates of the current triangles; tri_count sizes the grids, `live`, when given, is a
@@ -114,7 +127,6 @@ size_t tile_sum_words(size_t n); // entries of one m.tile_sums array (there are 
 void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count, size_t window);
 size_t rank_sort_words(size_t cand_count); // words of m.rank_counts
 void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count);
-void launch_pick_capacity(hipStream_t s, Mesh& m, size_t index_count);
 void launch_round(hipStream_t s, Mesh& m, size_t list_bound, int head_index, int rel, bool deep);
 void launch_round_tail(hipStream_t s, Mesh& m, int rel, uint32_t max_rounds, bool deep);
 // the list of ranks [lo, hi) and their first publishing round; the rounds that follow have rel >= 1

@@ -375,19 +375,6 @@ void launch_pick(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live)
 	k_tri_write<false><<<tiles, kThreads, 0, s>>>(a);
 }
 
-// boundEdgeCollapses (src/simplifier.cpp:1292-1308) from the dual count on the device:
-// index_count - dual / 2 + 3, so the first pick needs no read-back
-__global__ void k_pick_capacity(CallScalars* sc, uint64_t index_count)
-{
-	const uint64_t c = index_count - sc->dual_count / 2 + 3;
-	sc->pick_capacity = c < 0xffffffffull ? (uint32_t)c : 0xffffffffu;
-}
-
-void launch_pick_capacity(hipStream_t s, Mesh& m, size_t index_count)
-{
-	k_pick_capacity<<<1, 1, 0, s>>>(m.sc, (uint64_t)index_count);
-}
-
 // ------------------------------------------------------------------------------------------
 // rankEdgeCollapses, src/simplifier.cpp:1374-1450, and sortEdgeCollapses, 1452-1496
 
@@ -464,7 +451,7 @@ __device__ __forceinline__ float2 rank_errors(const RankArgs& a, uint32_t i0, ui
 // counts each tile of candidates in LDS, the scan of the (value, tile) counts gives every tile its
 // place in every value's run, and the scatter writes the ranked copies there directly.  Its
 // wavefronts own consecutive parts of the tile with a count of their own per value, so nothing
-// waits between 64 candidates and the next.  Icosphere L8's first pass, 2 M candidates: 85 us after
+// waits between 64 candidates and the next.  Icosphere L8's first pass, 2 M candidates: 93 us after
 // the rank, where two 8-bit digits with their scans and a gather of the ranked copies took 150 in
 // nine launches.
 constexpr int kKeyValues = 2560;
@@ -1651,8 +1638,8 @@ __global__ void __launch_bounds__(kThreads) k_stop_find(const uint8_t* status, c
 		const uint32_t w[kRecWords] = {at, committed, border, rejected, skipped, best, reason};
 #pragma unroll
 		for (int q = 0; q < kRecWords; ++q)
-			__hip_atomic_store(&rec[q], w[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		__threadfence();
+			(void)__hip_atomic_exchange(&rec[q], w[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		wait_for_memory();
 		s_last = atomicAdd(&sc->stop_done, 1u) + 1 == gridDim.x;
 	}
 	__syncthreads();
@@ -1661,7 +1648,6 @@ __global__ void __launch_bounds__(kThreads) k_stop_find(const uint8_t* status, c
 	if (threadIdx.x == 0)
 		sc->split = 0;
 	// the first record with a break, else the last tile's: one wavefront
-	__threadfence();
 	uint32_t hit = gridDim.x - 1;
 	for (uint32_t b0 = 0; b0 < gridDim.x; b0 += 64)
 	{

@@ -4,6 +4,8 @@
 #include "prims.h"
 #include "quadric.h"
 
+#include <algorithm>
+
 namespace mhip
 {
 
@@ -38,6 +40,51 @@ void launch_check_indices(hipStream_t s, const uint32_t* ib, size_t index_count,
 {
 	if (index_count)
 		k_check_indices<<<grid_for(index_count), kThreads, 0, s>>>(ib, index_count, vertex_count, flag);
+}
+
+// the device scalars of a call (the box reductions empty, everything else 0) and the n words at
+// `zeroed`
+__global__ void __launch_bounds__(kThreads) k_call_init(CallScalars* sc, uint32_t* zeroed, size_t n)
+{
+	for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads)
+		zeroed[i] = 0;
+	if (blockIdx.x)
+		return;
+	uint32_t* w = reinterpret_cast<uint32_t*>(sc);
+	for (size_t i = threadIdx.x; i < sizeof(CallScalars) / 4; i += kThreads)
+		w[i] = 0;
+	__syncthreads();
+	if (threadIdx.x < 3)
+		sc->box_min[threadIdx.x] = ~0ull;
+}
+
+void launch_call_init(hipStream_t s, CallScalars* sc, uint32_t* zeroed, size_t n)
+{
+	const unsigned int grid = grid_for(n);
+	k_call_init<<<grid < 1024 ? grid : 1024, kThreads, 0, s>>>(sc, zeroed, n);
+}
+
+// the call's copy of the indices with the range check; with `counts`, each corner also takes its
+// slot in its vertex's list (order_corners below)
+__global__ void k_load_indices(const uint32_t* in, uint32_t* out, size_t n, size_t limit, uint32_t* counts, uint32_t* slot, uint32_t* flag)
+{
+	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	const uint32_t v = j < n ? in[j] : 0;
+	const bool bad = j < n && v >= limit;
+	if (__ballot(bad) && __lane_id() == 0)
+		atomicOr(flag, 1u);
+	if (j >= n)
+		return;
+	out[j] = v;
+	if (counts && !bad)
+		slot[j] = atomicAdd(&counts[v], 1u);
+}
+
+void launch_load_indices(hipStream_t s, const uint32_t* in, uint32_t* out, size_t index_count, size_t vertex_count, uint32_t* counts, uint32_t* slot,
+                         uint32_t* flag)
+{
+	if (index_count)
+		k_load_indices<<<grid_for(index_count), kThreads, 0, s>>>(in, out, index_count, vertex_count, counts, slot, flag);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -85,22 +132,144 @@ void launch_sparse_remap(hipStream_t s, const uint32_t* indices_in, uint32_t* in
 }
 
 // ------------------------------------------------------------------------------------------
-// positions
+// positions, their box (the rescale's, src/simplifier.cpp:549-603) and the empty hash table in one
+// sweep.  The reference keeps the first element (in vertex order) that compares below the running
+// minimum, so among +0/-0 ties the earliest wins: reduce (ordered key, index) pairs, then read the
+// winning element's own bits.  The workgroup that finishes last turns the box into the extent.
 
-__global__ void k_gather_positions(const float* positions, size_t stride, const uint32_t* sparse_remap, float4* out, size_t n)
+__device__ __forceinline__ float comp(float4 p, int k)
 {
-	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	size_t ri = sparse_remap ? sparse_remap[i] : i;
-	const float* p = positions + ri * stride;
-	out[i] = make_float4(p[0], p[1], p[2], 0.f);
+	return k == 0 ? p.x : (k == 1 ? p.y : p.z);
 }
 
-void launch_gather_positions(hipStream_t s, const float* positions, size_t stride_floats, const uint32_t* sparse_remap, float4* out, size_t vertex_count)
+constexpr int kGatherThreads = 512;
+constexpr unsigned int kGatherBlocks = 512;
+
+__global__ void __launch_bounds__(kGatherThreads) k_gather_positions(const float* positions, size_t stride, const uint32_t* sparse_remap, float4* praw,
+                                                                     size_t n, uint32_t* table, size_t table_size, CallScalars* sc)
 {
-	if (vertex_count)
-		k_gather_positions<<<grid_for(vertex_count), kThreads, 0, s>>>(positions, stride_floats, sparse_remap, out, vertex_count);
+	constexpr int kWaves = kGatherThreads / 64;
+	__shared__ uint64_t red[6][kWaves];
+	__shared__ bool s_last;
+	const size_t step = (size_t)gridDim.x * kGatherThreads, first = (size_t)blockIdx.x * kGatherThreads + threadIdx.x;
+	for (size_t i = first; i < table_size; i += step)
+		table[i] = kNone;
+	uint64_t mn[3], mx[3];
+#pragma unroll
+	for (int k = 0; k < 3; ++k)
+	{
+		mn[k] = ~0ull;
+		mx[k] = 0ull;
+	}
+	for (size_t i = first; i < n; i += step)
+	{
+		const size_t ri = sparse_remap ? sparse_remap[i] : i;
+		const float* p = positions + ri * stride;
+		const float c[3] = {p[0], p[1], p[2]};
+		praw[i] = make_float4(c[0], c[1], c[2], 0.f);
+#pragma unroll
+		for (int k = 0; k < 3; ++k)
+		{
+			if (c[k] != c[k])
+				continue;
+			const uint64_t key = (uint64_t)ordered_key(c[k]) << 32;
+			const uint64_t a = key | (uint64_t)(uint32_t)i;
+			const uint64_t b = key | (uint64_t)(0xffffffffu - (uint32_t)i);
+			mn[k] = a < mn[k] ? a : mn[k];
+			mx[k] = b > mx[k] ? b : mx[k];
+		}
+	}
+	const int wave = threadIdx.x >> 6;
+#pragma unroll
+	for (int k = 0; k < 3; ++k)
+	{
+		const uint64_t a = wave_min64(mn[k]), b = wave_max64(mx[k]);
+		if (__lane_id() == 0)
+		{
+			red[k][wave] = a;
+			red[3 + k][wave] = b;
+		}
+	}
+	__syncthreads();
+	if (threadIdx.x < 3)
+	{
+		const int k = threadIdx.x;
+		uint64_t a = ~0ull, b = 0ull;
+		for (int w = 0; w < kWaves; ++w)
+		{
+			a = red[k][w] < a ? red[k][w] : a;
+			b = red[3 + k][w] > b ? red[3 + k][w] : b;
+		}
+		// a workgroup inside the box found so far adds nothing (same-address atomics serialise)
+		if (a < __hip_atomic_load(&sc->box_min[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+			atomicMin((unsigned long long*)&sc->box_min[k], (unsigned long long)a);
+		if (b > __hip_atomic_load(&sc->box_max[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+			atomicMax((unsigned long long*)&sc->box_max[k], (unsigned long long)b);
+	}
+	// this workgroup's part of the box, before it counts itself done
+	wait_for_memory();
+	__syncthreads();
+	if (threadIdx.x == 0)
+		s_last = atomicAdd(&sc->box_done, 1u) + 1 == gridDim.x;
+	__syncthreads();
+	if (!s_last || threadIdx.x)
+		return;
+	float lo[3], hi[3];
+	for (int k = 0; k < 3; ++k)
+	{
+		const uint64_t a = __hip_atomic_load(&sc->box_min[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		const uint64_t b = __hip_atomic_load(&sc->box_max[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		lo[k] = FLT_MAX;
+		hi[k] = -FLT_MAX;
+		// the caller's own bits of the winning element
+		auto value = [&](uint32_t i) { return positions[(size_t)(sparse_remap ? sparse_remap[i] : i) * stride + k]; };
+		if (a != ~0ull)
+		{
+			const float v = value((uint32_t)a);
+			lo[k] = FLT_MAX > v ? v : FLT_MAX;
+		}
+		if (b != 0ull)
+		{
+			const float v = value(0xffffffffu - (uint32_t)b);
+			hi[k] = -FLT_MAX < v ? v : -FLT_MAX;
+		}
+	}
+	float extent = 0.f;
+	extent = (hi[0] - lo[0]) < extent ? extent : (hi[0] - lo[0]);
+	extent = (hi[1] - lo[1]) < extent ? extent : (hi[1] - lo[1]);
+	extent = (hi[2] - lo[2]) < extent ? extent : (hi[2] - lo[2]);
+	for (int k = 0; k < 3; ++k)
+		sc->lo[k] = lo[k];
+	sc->extent = extent;
+	sc->scale = extent == 0 ? 0.f : 1.f / extent;
+}
+
+void launch_gather_positions(hipStream_t s, Mesh& m, const float* positions, size_t stride_floats, const uint32_t* sparse_remap, uint32_t* table,
+                             size_t table_size)
+{
+	const size_t n = m.vertex_count;
+	const unsigned int grid = div_up(n ? n : 1, kGatherThreads);
+	k_gather_positions<<<grid < kGatherBlocks ? grid : kGatherBlocks, kGatherThreads, 0, s>>>(positions, stride_floats, sparse_remap, m.praw, n, table,
+	                                                                                        table_size, m.sc);
+}
+
+__device__ __forceinline__ float4 rescaled(float4 p, const CallScalars* sc)
+{
+	const float scale = sc->scale;
+	return make_float4((p.x - sc->lo[0]) * scale, (p.y - sc->lo[1]) * scale, (p.z - sc->lo[2]) * scale, 0.f);
+}
+
+__global__ void k_rescale(const float4* praw, size_t n, const CallScalars* sc, float4* pos)
+{
+	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n)
+		pos[i] = rescaled(praw[i], sc);
+}
+
+void launch_rescale(hipStream_t s, Mesh& m)
+{
+	if (m.vertex_count)
+		k_rescale<<<grid_for(m.vertex_count), kThreads, 0, s>>>(m.praw, m.vertex_count, m.sc, m.pos);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -156,30 +325,49 @@ __global__ void k_hash_insert(const float4* pos, size_t n, uint32_t* table, uint
 	}
 }
 
-__global__ void k_hash_lookup(const float4* pos, size_t n, const uint32_t* table, uint32_t mask, uint32_t* remap)
+// each vertex's primary, its rescaled position, a wedge ring of its own and no pending ranks; sc
+// counts the secondaries
+__global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, size_t n, const uint32_t* table, uint32_t mask, uint32_t* remap,
+                                                          uint32_t* wedge, float4* pos, ulonglong2* pend0, ulonglong2* pend1, CallScalars* sc)
 {
-	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	float4 p = pos[i];
+	__shared__ uint32_t secondaries;
+	if (threadIdx.x == 0)
+		secondaries = 0;
+	__syncthreads();
+	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	uint32_t result = (uint32_t)i;
-	if (!has_nan(p))
+	if (i < n)
 	{
-		uint32_t slot = pos_hash(p) & mask;
-		for (uint32_t probe = 0; probe <= mask; ++probe)
+		const float4 p = praw[i];
+		if (!has_nan(p))
 		{
-			uint32_t e = table[slot];
-			if (e == kNone)
-				break; // unreachable: i itself was inserted
-			if (same_pos(pos[e], p))
+			uint32_t slot = pos_hash(p) & mask;
+			for (uint32_t probe = 0; probe <= mask; ++probe)
 			{
-				result = e;
-				break;
+				uint32_t e = table[slot];
+				if (e == kNone)
+					break; // unreachable: i itself was inserted
+				if (e == (uint32_t)i || same_pos(praw[e], p))
+				{
+					result = e;
+					break;
+				}
+				slot = (slot + 1) & mask;
 			}
-			slot = (slot + 1) & mask;
 		}
+		remap[i] = result;
+		wedge[i] = (uint32_t)i;
+		pos[i] = rescaled(p, sc);
+		// round minima start as "no entry" (tag of epoch 0, rank all-ones)
+		pend0[i] = make_ulonglong2(~0ull, ~0ull);
+		pend1[i] = make_ulonglong2(~0ull, ~0ull);
 	}
-	remap[i] = result;
+	const uint64_t second = __ballot(result != (uint32_t)i);
+	if (second && __lane_id() == 0)
+		atomicAdd(&secondaries, (uint32_t)__popcll(second));
+	__syncthreads();
+	if (threadIdx.x == 0 && secondaries)
+		atomicAdd(&sc->secondary_count, secondaries);
 }
 
 void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size)
@@ -187,9 +375,9 @@ void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table
 	size_t n = m.vertex_count;
 	if (!n)
 		return;
-	fill_u32(s, table, kNone, table_size);
 	k_hash_insert<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1));
-	k_hash_lookup<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1), m.remap);
+	k_hash_lookup<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1), m.remap, m.wedge, m.pos,
+	                                               reinterpret_cast<ulonglong2*>(m.pend[0]), reinterpret_cast<ulonglong2*>(m.pend[1]), m.sc);
 }
 
 // wedge rings: for a class r < a_1 < ... < a_m, wedge[r] = a_m, wedge[a_k] = a_{k-1}, wedge[a_1] = r
@@ -214,10 +402,9 @@ __global__ void k_secondary_compact(const uint32_t* remap, size_t n, const uint3
 	}
 }
 
-__global__ void k_wedge_link(const uint32_t* keys, const uint32_t* vals, size_t n_max, const uint32_t* n_dev, uint32_t* wedge)
+__global__ void k_wedge_link(const uint32_t* keys, const uint32_t* vals, size_t n, uint32_t* wedge)
 {
 	size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	size_t n = *n_dev < n_max ? *n_dev : n_max;
 	if (p >= n)
 		return;
 	uint32_t r = keys[p];
@@ -227,25 +414,29 @@ __global__ void k_wedge_link(const uint32_t* keys, const uint32_t* vals, size_t 
 		wedge[r] = i;
 }
 
-void launch_wedges(hipStream_t s, Mesh& m, uint32_t* flags, uint32_t* scratch_a, uint32_t* scratch_b, uint32_t* scratch_c, uint32_t* scratch_d)
+void launch_wedges(hipStream_t s, Mesh& m, size_t secondaries, uint32_t* flags, uint32_t* scratch_a, uint32_t* scratch_b, uint32_t* scratch_c,
+                   uint32_t* scratch_d)
 {
 	size_t n = m.vertex_count;
-	if (!n)
-		return;
-	iota_u32(s, m.wedge, n);
-	uint32_t* count = &m.sc->work[0];
+	if (!secondaries)
+		return; // every ring is a vertex of its own
 	k_secondary_flags<<<grid_for(n), kThreads, 0, s>>>(m.remap, n, flags);
-	scan_exclusive(s, flags, scratch_a, n, nullptr, count, m.temp);
+	scan_exclusive(s, flags, scratch_a, n, nullptr, nullptr, m.temp);
 	k_secondary_compact<<<grid_for(n), kThreads, 0, s>>>(m.remap, n, flags, scratch_a, scratch_b, scratch_c);
-	radix_sort_pairs(s, scratch_b, scratch_c, scratch_d, scratch_a, n, count, key_bits(n), m.temp);
-	k_wedge_link<<<grid_for(n), kThreads, 0, s>>>(scratch_b, scratch_c, n, count, m.wedge);
+	radix_sort_pairs(s, scratch_b, scratch_c, scratch_d, scratch_a, secondaries, nullptr, key_bits(n), m.temp);
+	k_wedge_link<<<grid_for(secondaries), kThreads, 0, s>>>(scratch_b, scratch_c, secondaries, m.wedge);
 }
 
 // ------------------------------------------------------------------------------------------
-// corner CSR sorted by (vertex, corner): the order in which the reference visits a vertex's
-// triangles (triangle order, then corner order)
+// Corner lists: each vertex's (or class's) corners in corner order, the order in which the reference
+// visits its triangles.  One atomic per corner hands it a slot in its list, in any order; the scan
+// of the counts and a placement make the lists, and each is then put in order where it lies: up to
+// eight corners by a sorting network in registers, more by the wavefront, every corner's place the
+// number of smaller ones.  (Sorting all corners by vertex with three radix digits took 370 us for
+// the 3.9 M of icosphere L8 and the open edges 140; lists and open edges now take 300 with the index
+// copy and check, 250 of it the count's and the placement's scattered words.)
 
-__global__ void k_corner_keys(const uint32_t* ib, size_t n, const uint32_t* remap, uint32_t* keys, uint32_t* vals, uint32_t* counts)
+__global__ void k_corner_count(const uint32_t* ib, size_t n, const uint32_t* remap, uint32_t* counts, uint32_t* slot)
 {
 	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (j >= n)
@@ -253,44 +444,202 @@ __global__ void k_corner_keys(const uint32_t* ib, size_t n, const uint32_t* rema
 	uint32_t v = ib[j];
 	if (remap)
 		v = remap[v];
-	keys[j] = v;
-	vals[j] = (uint32_t)j;
-	atomicAdd(&counts[v], 1u);
+	slot[j] = atomicAdd(&counts[v], 1u);
 }
 
-void launch_corner_csr(hipStream_t s, const uint32_t* ib, size_t index_count, const uint32_t* remap, size_t vertex_count,
-                       uint32_t* offsets, uint32_t* keys, uint32_t* corners, uint32_t* keys_alt, uint32_t* vals_alt, uint32_t* temp)
+__global__ void k_corner_place(const uint32_t* ib, size_t n, const uint32_t* remap, const uint32_t* off, const uint32_t* slot, uint32_t* placed)
 {
-	fill_u32(s, offsets, 0, vertex_count + 1);
-	if (index_count == 0)
+	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (j >= n)
 		return;
-	k_corner_keys<<<grid_for(index_count), kThreads, 0, s>>>(ib, index_count, remap, keys, corners, offsets);
-	scan_exclusive(s, offsets, offsets, vertex_count, nullptr, offsets + vertex_count, temp);
-	radix_sort_pairs(s, keys, corners, keys_alt, vals_alt, index_count, nullptr, key_bits(vertex_count), temp);
+	uint32_t v = ib[j];
+	if (remap)
+		v = remap[v];
+	placed[off[v] + slot[j]] = (uint32_t)j;
 }
 
-// ------------------------------------------------------------------------------------------
-// unwelded half-edge data (next, prev) per sorted corner
-
-__global__ void k_corner_adjacency(const uint32_t* ib, const uint32_t* corners, size_t n, uint2* adj)
+struct CornerArgs
 {
-	size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (p >= n)
+	const uint32_t* ib;
+	const uint32_t* off;
+	const uint32_t* placed;
+	uint32_t* corners;
+	uint32_t* openout;
+	uint32_t* openinc;
+	uint2* adj; // (next, prev) per listed corner, or null
+	size_t n;
+};
+
+// the vertices after and before corner j in its triangle
+__device__ __forceinline__ uint2 corner_neighbours(const uint32_t* ib, uint32_t j)
+{
+	const uint32_t t = j / 3, c = j - t * 3;
+	return make_uint2(ib[t * 3 + (c == 2 ? 0 : c + 1)], ib[t * 3 + (c == 0 ? 2 : c - 1)]);
+}
+
+__device__ __forceinline__ void compare_exchange(uint32_t& a, uint32_t& b)
+{
+	const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
+	a = lo;
+	b = hi;
+}
+
+__device__ __forceinline__ uint32_t open_end(uint32_t v, bool self, uint32_t count, uint32_t last)
+{
+	return (self || count > 1) ? v : (count == 1 ? last : kNone);
+}
+
+// kOpen: also the open half-edges per vertex (src/simplifier.cpp:379-400): an outgoing edge v->t is
+// open when t has no edge t->v, an incoming edge u->v when v has no edge v->u.  The opposite of
+// either half-edge lies in a triangle around v as well, where the other vertex comes before v
+// (t->v) or after it (v->u), so v's own list answers both.  Result: none, the single other endpoint,
+// or v itself when there are several open edges or a self edge.
+template <bool kOpen>
+__global__ void __launch_bounds__(kThreads) k_corner_order(CornerArgs a)
+{
+	constexpr int kNet = 8;
+	const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
+	const uint32_t v = (uint32_t)i, lane = __lane_id();
+	const uint32_t b = i < a.n ? a.off[i] : 0, e = i < a.n ? a.off[i + 1] : 0, len = e - b;
+	if (i < a.n && len <= kNet)
+	{
+		uint32_t c[kNet];
+#pragma unroll
+		for (int q = 0; q < kNet; ++q)
+			c[q] = (uint32_t)q < len ? a.placed[b + q] : kNone;
+		constexpr uint8_t net[19][2] = {{0, 1}, {2, 3}, {4, 5}, {6, 7}, {0, 2}, {1, 3}, {4, 6}, {5, 7}, {1, 2}, {5, 6},
+		                                {0, 4}, {3, 7}, {1, 5}, {2, 6}, {1, 4}, {3, 6}, {2, 4}, {3, 5}, {3, 4}};
+#pragma unroll
+		for (int k = 0; k < 19; ++k)
+			compare_exchange(c[net[k][0]], c[net[k][1]]);
+#pragma unroll
+		for (int q = 0; q < kNet; ++q)
+			if ((uint32_t)q < len)
+				a.corners[b + q] = c[q];
+		if (kOpen)
+		{
+			uint2 nb[kNet];
+#pragma unroll
+			for (int q = 0; q < kNet; ++q)
+				nb[q] = (uint32_t)q < len ? corner_neighbours(a.ib, c[q]) : make_uint2(kNone, kNone);
+			uint32_t outs = 0, out_last = kNone, ins = 0, in_last = kNone;
+			bool self = false;
+#pragma unroll
+			for (int q = 0; q < kNet; ++q)
+			{
+				if ((uint32_t)q >= len)
+					continue;
+				if (a.adj)
+					a.adj[b + q] = nb[q];
+				bool opposite_out = false, opposite_in = false;
+#pragma unroll
+				for (int r = 0; r < kNet; ++r)
+				{
+					opposite_out |= nb[r].y == nb[q].x;
+					opposite_in |= nb[r].x == nb[q].y;
+				}
+				if (nb[q].x == v)
+					self = true;
+				else if (!opposite_out)
+				{
+					outs++;
+					out_last = nb[q].x;
+				}
+				if (nb[q].y == v)
+					self = true;
+				else if (!opposite_in)
+				{
+					ins++;
+					in_last = nb[q].y;
+				}
+			}
+			a.openout[v] = open_end(v, self, outs, out_last);
+			a.openinc[v] = open_end(v, self, ins, in_last);
+		}
+	}
+	for (uint64_t left = __ballot(len > kNet); left; left &= left - 1)
+	{
+		const int from = __builtin_ctzll(left);
+		const uint32_t w = __builtin_amdgcn_readlane(v, from), wb = __builtin_amdgcn_readlane(b, from), we = __builtin_amdgcn_readlane(e, from);
+		uint32_t outs = 0, out_last = kNone, ins = 0, in_last = kNone;
+		bool self = false;
+		for (uint32_t x0 = wb; x0 < we; x0 += 64)
+		{
+			const bool in = x0 + lane < we;
+			const uint32_t cx = in ? a.placed[x0 + lane] : kNone;
+			const uint2 nx = kOpen && in ? corner_neighbours(a.ib, cx) : make_uint2(kNone, kNone);
+			uint32_t place = 0;
+			bool opposite_out = false, opposite_in = false;
+			for (uint32_t y0 = wb; y0 < we; y0 += 64)
+			{
+				const bool iny = y0 + lane < we;
+				const uint32_t cy = iny ? a.placed[y0 + lane] : kNone;
+				const uint2 ny = kOpen && iny ? corner_neighbours(a.ib, cy) : make_uint2(kNone, kNone);
+				const uint32_t m = we - y0 < 64 ? we - y0 : 64;
+				for (uint32_t k = 0; k < m; ++k)
+				{
+					place += (uint32_t)__builtin_amdgcn_readlane(cy, k) < cx ? 1u : 0u;
+					if (kOpen)
+					{
+						opposite_out |= (uint32_t)__builtin_amdgcn_readlane(ny.y, k) == nx.x;
+						opposite_in |= (uint32_t)__builtin_amdgcn_readlane(ny.x, k) == nx.y;
+					}
+				}
+			}
+			if (in)
+			{
+				a.corners[wb + place] = cx;
+				if (kOpen && a.adj)
+					a.adj[wb + place] = nx;
+			}
+			if (kOpen)
+			{
+				const uint64_t out_mask = __ballot(in && nx.x != w && !opposite_out), in_mask = __ballot(in && nx.y != w && !opposite_in);
+				self |= __ballot(in && (nx.x == w || nx.y == w)) != 0;
+				if (out_mask)
+					out_last = __builtin_amdgcn_readlane(nx.x, __builtin_ctzll(out_mask));
+				if (in_mask)
+					in_last = __builtin_amdgcn_readlane(nx.y, __builtin_ctzll(in_mask));
+				outs += (uint32_t)__popcll(out_mask);
+				ins += (uint32_t)__popcll(in_mask);
+			}
+		}
+		if (kOpen && (int)lane == from)
+		{
+			a.openout[w] = open_end(w, self, outs, out_last);
+			a.openinc[w] = open_end(w, self, ins, in_last);
+		}
+	}
+}
+
+// offsets (n + 1 words) hold the counts when `counted` (the slots are then given), else zeros
+static void corner_lists(hipStream_t s, Mesh& m, const uint32_t* remap, bool counted, uint32_t* offsets, uint32_t* slot, uint32_t* placed)
+{
+	const size_t n = m.index_count;
+	if (!counted && n)
+		k_corner_count<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], n, remap, offsets, slot);
+	scan_exclusive(s, offsets, offsets, m.vertex_count, nullptr, offsets + m.vertex_count, m.temp);
+	if (n)
+		k_corner_place<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], n, remap, offsets, slot, placed);
+}
+
+void launch_corner_lists(hipStream_t s, Mesh& m, bool counted, bool with_adjacency, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners)
+{
+	if (!m.vertex_count)
 		return;
-	uint32_t j = corners[p];
-	uint32_t t = j / 3, c = j - t * 3;
-	uint32_t cn = c == 2 ? 0 : c + 1;
-	uint32_t cp = c == 0 ? 2 : c - 1;
-	adj[p] = make_uint2(ib[t * 3 + cn], ib[t * 3 + cp]);
+	corner_lists(s, m, nullptr, counted, offsets, slot, placed);
+	const CornerArgs a{m.ib[0], offsets, placed, corners, m.loop[0], m.loopback[0], with_adjacency ? m.adj[1] : nullptr, m.vertex_count};
+	k_corner_order<true><<<grid_for(m.vertex_count), kThreads, 0, s>>>(a);
 }
 
-// hasEdge, src/simplifier.cpp:333-343
-__device__ __forceinline__ bool has_edge(const uint32_t* off, const uint2* adj, uint32_t a, uint32_t b)
+void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners)
 {
-	for (uint32_t p = off[a], e = off[a + 1]; p < e; ++p)
-		if (adj[p].x == b)
-			return true;
-	return false;
+	if (!m.vertex_count)
+		return;
+	fill_u32(s, offsets, 0, (size_t)m.vertex_count + 1);
+	corner_lists(s, m, m.remap, false, offsets, slot, placed);
+	const CornerArgs a{m.ib[0], offsets, placed, corners, nullptr, nullptr, nullptr, m.vertex_count};
+	k_corner_order<false><<<grid_for(m.vertex_count), kThreads, 0, s>>>(a);
 }
 
 // hasEdge over the wedges of a, src/simplifier.cpp:345-362
@@ -308,50 +657,9 @@ __device__ __forceinline__ bool has_edge_wedged(const uint32_t* off, const uint2
 	return false;
 }
 
-// open half-edges per vertex (src/simplifier.cpp:379-400), gathered from the vertex's own
-// corners: an outgoing edge v->t is open when t has no edge t->v, an incoming edge u->v is
-// open when v has no edge v->u.  Result: none, the single other endpoint, or v itself when
-// there are several open edges or a self edge.
-__global__ void k_open_edges(const uint32_t* off, const uint2* adj, size_t n, uint32_t* openout, uint32_t* openinc)
-{
-	size_t iv = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (iv >= n)
-		return;
-	uint32_t v = (uint32_t)iv;
-	uint32_t out_count = 0, out_last = kNone, in_count = 0, in_last = kNone;
-	bool self = false;
-	for (uint32_t p = off[v], e = off[v + 1]; p < e; ++p)
-	{
-		uint2 np = adj[p];
-		if (np.x == v)
-			self = true;
-		else if (!has_edge(off, adj, np.x, v))
-		{
-			out_count++;
-			out_last = np.x;
-		}
-		if (np.y == v)
-			self = true;
-		else if (!has_edge(off, adj, v, np.y))
-		{
-			in_count++;
-			in_last = np.y;
-		}
-	}
-	openout[v] = (self || out_count > 1) ? v : (out_count == 1 ? out_last : kNone);
-	openinc[v] = (self || in_count > 1) ? v : (in_count == 1 ? in_last : kNone);
-}
-
 // classifyVertices primary rules, src/simplifier.cpp:406-470
-__global__ void k_classify_primary(const uint32_t* remap, const uint32_t* wedge, const uint32_t* loop, const uint32_t* loopback, size_t n, uint8_t* kind)
+__device__ __forceinline__ uint8_t classify_primary(const uint32_t* remap, const uint32_t* wedge, const uint32_t* loop, const uint32_t* loopback, uint32_t i)
 {
-	size_t ii = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (ii >= n)
-		return;
-	uint32_t i = (uint32_t)ii;
-	if (remap[i] != i)
-		return;
-
 	uint8_t k;
 	if (wedge[i] == i)
 	{
@@ -378,7 +686,14 @@ __global__ void k_classify_primary(const uint32_t* remap, const uint32_t* wedge,
 	}
 	else
 		k = kLocked;
-	kind[i] = k;
+	return k;
+}
+
+__global__ void k_classify_primary(const uint32_t* remap, const uint32_t* wedge, const uint32_t* loop, const uint32_t* loopback, size_t n, uint8_t* kind)
+{
+	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < n && remap[i] == (uint32_t)i)
+		kind[i] = classify_primary(remap, wedge, loop, loopback, (uint32_t)i);
 }
 
 // permissive mode, src/simplifier.cpp:481-515 (primaries; wedges copy later)
@@ -425,179 +740,69 @@ __global__ void k_lock_mark(const uint32_t* remap, const uint8_t* vertex_lock, c
 
 // every wedge takes its primary's final kind; LockBorder turns Border into Locked
 // (src/simplifier.cpp:470-477, 527-536; the Border->Locked map is idempotent, so primaries
-// updating in place race harmlessly with wedges reading them)
-__global__ void k_kind_finalize(const uint32_t* remap, size_t n, uint32_t options, uint8_t* kind)
+// updating in place race harmlessly with wedges reading them).  Counted on the way: the primaries
+// of each kind, and the corners of the manifold and seam vertices (boundEdgeCollapses, 1292-1308).
+// kDirect: nothing changes a kind between the primary rules and here, and no vertex has a second
+// wedge, so each vertex takes the rules' kind itself.
+template <bool kDirect>
+__global__ void __launch_bounds__(kThreads) k_kind_finalize(const uint32_t* remap, const uint32_t* wedge, const uint32_t* loop, const uint32_t* loopback,
+                                                            const uint32_t* off, size_t n, uint32_t options, uint8_t* kind, CallScalars* sc)
 {
-	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	uint8_t k = kind[remap[i]];
-	if ((options & kOptLockBorder) && k == kBorder)
-		k = kLocked;
-	kind[i] = k;
+	__shared__ uint32_t h[7];
+	if (threadIdx.x < 7)
+		h[threadIdx.x] = 0;
+	__syncthreads();
+	uint32_t local[7] = {0, 0, 0, 0, 0, 0, 0};
+	for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads)
+	{
+		const uint32_t r = kDirect ? (uint32_t)i : remap[i];
+		uint8_t k = kDirect ? classify_primary(remap, wedge, loop, loopback, (uint32_t)i) : kind[r];
+		if ((options & kOptLockBorder) && k == kBorder)
+			k = kLocked;
+		kind[i] = k;
+		if (r == (uint32_t)i)
+		{
+#pragma unroll
+			for (int q = 0; q < 5; ++q)
+				local[q] += k == q;
+			local[5]++;
+		}
+		local[6] += (k == kManifold || k == kSeam) ? off[i + 1] - off[i] : 0u;
+	}
+#pragma unroll
+	for (int q = 0; q < 7; ++q)
+	{
+		uint32_t v = local[q];
+		for (int o = 32; o > 0; o >>= 1)
+			v += __shfl_xor(v, o, 64);
+		if (__lane_id() == 0 && v)
+			atomicAdd(&h[q], v);
+	}
+	__syncthreads();
+	if (threadIdx.x < 7 && h[threadIdx.x])
+		atomicAdd(threadIdx.x < 6 ? &sc->kind_counts[threadIdx.x] : &sc->dual_count, h[threadIdx.x]);
 }
 
-void launch_classify(hipStream_t s, Mesh& m, const uint32_t* raw_off, const uint32_t* raw_corners, const uint8_t* vertex_lock,
-                     const uint32_t* sparse_remap, uint32_t options)
+void launch_classify(hipStream_t s, Mesh& m, const uint32_t* raw_off, bool secondaries, const uint8_t* vertex_lock, const uint32_t* sparse_remap,
+                     uint32_t options)
 {
 	size_t n = m.vertex_count;
-	size_t ni = m.index_count;
 	if (!n)
 		return;
 	uint32_t* loop = m.loop[0];
 	uint32_t* loopback = m.loopback[0];
-	if (ni)
-		k_corner_adjacency<<<grid_for(ni), kThreads, 0, s>>>(m.ib[0], raw_corners, ni, m.adj[1]);
-	k_open_edges<<<grid_for(n), kThreads, 0, s>>>(raw_off, m.adj[1], n, loop, loopback);
+	const unsigned int grid = std::min(grid_for(n), 1024u);
+	if (!secondaries && !vertex_lock && !(options & kOptPermissive))
+	{
+		k_kind_finalize<true><<<grid, kThreads, 0, s>>>(m.remap, m.wedge, loop, loopback, raw_off, n, options, m.kind, m.sc);
+		return;
+	}
 	k_classify_primary<<<grid_for(n), kThreads, 0, s>>>(m.remap, m.wedge, loop, loopback, n, m.kind);
 	if (options & kOptPermissive)
 		k_permissive<<<grid_for(n), kThreads, 0, s>>>(raw_off, m.adj[1], m.remap, m.wedge, vertex_lock, sparse_remap, n, m.kind);
 	if (vertex_lock)
 		k_lock_mark<<<grid_for(n), kThreads, 0, s>>>(m.remap, vertex_lock, sparse_remap, n, m.kind);
-	k_kind_finalize<<<grid_for(n), kThreads, 0, s>>>(m.remap, n, options, m.kind);
-}
-
-// ------------------------------------------------------------------------------------------
-// rescale (src/simplifier.cpp:549-603).  The reference keeps the first element (in vertex
-// order) that compares below the running minimum, so among +0/-0 ties the earliest wins:
-// reduce (ordered key, index) pairs, then read the winning element's own bits.
-
-__global__ void __launch_bounds__(256) k_bbox(const float4* praw, size_t n, CallScalars* sc)
-{
-	__shared__ uint64_t red[6][4];
-	uint64_t mn[3], mx[3];
-#pragma unroll
-	for (int k = 0; k < 3; ++k)
-	{
-		mn[k] = ~0ull;
-		mx[k] = 0ull;
-	}
-	for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-	{
-		float4 p = praw[i];
-		float c[3] = {p.x, p.y, p.z};
-#pragma unroll
-		for (int k = 0; k < 3; ++k)
-		{
-			if (c[k] != c[k])
-				continue;
-			uint64_t key = (uint64_t)ordered_key(c[k]) << 32;
-			uint64_t a = key | (uint64_t)(uint32_t)i;
-			uint64_t b = key | (uint64_t)(0xffffffffu - (uint32_t)i);
-			mn[k] = a < mn[k] ? a : mn[k];
-			mx[k] = b > mx[k] ? b : mx[k];
-		}
-	}
-	const int wave = threadIdx.x >> 6;
-#pragma unroll
-	for (int k = 0; k < 3; ++k)
-	{
-		uint64_t a = wave_min64(mn[k]);
-		uint64_t b = wave_max64(mx[k]);
-		if (__lane_id() == 0)
-		{
-			red[k][wave] = a;
-			red[3 + k][wave] = b;
-		}
-	}
-	__syncthreads();
-	if (threadIdx.x < 3)
-	{
-		int k = threadIdx.x;
-		uint64_t a = ~0ull, b = 0ull;
-		for (int w = 0; w < 4; ++w)
-		{
-			a = red[k][w] < a ? red[k][w] : a;
-			b = red[3 + k][w] > b ? red[3 + k][w] : b;
-		}
-		if (a != ~0ull)
-			atomicMin((unsigned long long*)&sc->box_min[k], (unsigned long long)a);
-		if (b != 0ull)
-			atomicMax((unsigned long long*)&sc->box_max[k], (unsigned long long)b);
-	}
-}
-
-__global__ void k_bbox_init(CallScalars* sc)
-{
-	for (int k = 0; k < 3; ++k)
-	{
-		sc->box_min[k] = ~0ull;
-		sc->box_max[k] = 0ull;
-	}
-}
-
-__device__ __forceinline__ float comp(float4 p, int k)
-{
-	return k == 0 ? p.x : (k == 1 ? p.y : p.z);
-}
-
-__global__ void k_extent(const float4* praw, CallScalars* sc)
-{
-	float lo[3], hi[3];
-	for (int k = 0; k < 3; ++k)
-	{
-		lo[k] = FLT_MAX;
-		hi[k] = -FLT_MAX;
-		if (sc->box_min[k] != ~0ull)
-		{
-			float v = comp(praw[(uint32_t)sc->box_min[k]], k);
-			lo[k] = FLT_MAX > v ? v : FLT_MAX;
-		}
-		if (sc->box_max[k] != 0ull)
-		{
-			float v = comp(praw[0xffffffffu - (uint32_t)sc->box_max[k]], k);
-			hi[k] = -FLT_MAX < v ? v : -FLT_MAX;
-		}
-	}
-
-	float extent = 0.f;
-	extent = (hi[0] - lo[0]) < extent ? extent : (hi[0] - lo[0]);
-	extent = (hi[1] - lo[1]) < extent ? extent : (hi[1] - lo[1]);
-	extent = (hi[2] - lo[2]) < extent ? extent : (hi[2] - lo[2]);
-
-	for (int k = 0; k < 3; ++k)
-		sc->lo[k] = lo[k];
-	sc->extent = extent;
-	sc->scale = extent == 0 ? 0.f : 1.f / extent;
-}
-
-__global__ void k_rescale(const float4* praw, size_t n, const CallScalars* sc, float4* pos)
-{
-	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	float4 p = praw[i];
-	float scale = sc->scale;
-	pos[i] = make_float4((p.x - sc->lo[0]) * scale, (p.y - sc->lo[1]) * scale, (p.z - sc->lo[2]) * scale, 0.f);
-}
-
-void launch_rescale(hipStream_t s, Mesh& m)
-{
-	size_t n = m.vertex_count;
-	k_bbox_init<<<1, 1, 0, s>>>(m.sc);
-	if (n)
-	{
-		unsigned int blocks = div_up(n, 256 * 8);
-		blocks = blocks > 512 ? 512 : blocks;
-		k_bbox<<<blocks, 256, 0, s>>>(m.praw, n, m.sc);
-	}
-	k_extent<<<1, 1, 0, s>>>(m.praw, m.sc);
-	if (n)
-		k_rescale<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, m.sc, m.pos);
-}
-
-// bounding box and extent only (meshopt_simplifyScale, src/simplifier.cpp:2938-2948)
-void launch_extent_only(hipStream_t s, Mesh& m)
-{
-	size_t n = m.vertex_count;
-	k_bbox_init<<<1, 1, 0, s>>>(m.sc);
-	if (n)
-	{
-		unsigned int blocks = div_up(n, 256 * 8);
-		blocks = blocks > 512 ? 512 : blocks;
-		k_bbox<<<blocks, 256, 0, s>>>(m.praw, n, m.sc);
-	}
-	k_extent<<<1, 1, 0, s>>>(m.praw, m.sc);
+	k_kind_finalize<false><<<grid, kThreads, 0, s>>>(m.remap, m.wedge, loop, loopback, raw_off, n, options, m.kind, m.sc);
 }
 
 // rescaleAttributes, src/simplifier.cpp:605-621 (only attributes with weight > 0)
@@ -651,37 +856,71 @@ __device__ __forceinline__ bool edge_loop_qualifies(const uint8_t* kind, const u
 
 __global__ void k_vertex_quadrics(const uint32_t* ib, const float4* pos, const uint32_t* remap, const uint8_t* kind, const uint32_t* loop,
                                   const uint32_t* loopback, const uint32_t* woff, const uint32_t* wcorners, const uint8_t* vertex_lock,
-                                  const uint32_t* sparse_remap, size_t n, float factor, Quad* vq, Grad* vg, uint2* adj_range, uint2* adj)
+                                  const uint32_t* sparse_remap, size_t n, float factor, Quad* vq, Grad* vg, uint2* adj_range, uint2* adj, uint64_t index_count,
+                                  CallScalars* sc)
 {
 	size_t ri = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (ri >= n)
 		return;
 	uint32_t r = (uint32_t)ri;
-	adj_range[r] = make_uint2(woff[r], woff[r + 1]); // empty for a secondary: the lists are keyed by primaries
-	if (remap[r] != r)
-		return;
-
+	// boundEdgeCollapses (src/simplifier.cpp:1292-1308) from the dual count: the first pick reads it here
+	if (r == 0)
+	{
+		const uint64_t c = index_count - sc->dual_count / 2 + 3;
+		sc->pick_capacity = c < 0xffffffffull ? (uint32_t)c : 0xffffffffu;
+	}
+	const uint32_t begin = woff[r], end = woff[r + 1];
+	adj_range[r] = make_uint2(begin, end); // empty for a secondary: the lists are keyed by primaries
 	Quad Q;
 	quad_zero(Q);
-	Grad GV = {0.f, 0.f, 0.f, 0.f};
-	uint32_t begin = woff[r], end = woff[r + 1];
-
-	for (uint32_t p = begin; p < end; ++p)
+	if (remap[r] != r)
 	{
-		const uint32_t t = wcorners[p] / 3, c = wcorners[p] - t * 3;
-		const uint32_t i0 = ib[t * 3 + 0], i1 = ib[t * 3 + 1], i2 = ib[t * 3 + 2];
-		V3 p0 = load_pos(pos, i0), p1 = load_pos(pos, i1), p2 = load_pos(pos, i2);
-		// the first pass's adjacency: the corner's next and previous classes
-		adj[p] = make_uint2(remap[c == 0 ? i1 : (c == 1 ? i2 : i0)], remap[c == 0 ? i2 : (c == 1 ? i0 : i1)]);
-		Quad F;
-		quad_from_triangle(F, p0, p1, p2, 1.f);
-		quad_add(Q, F);
-		if (vg)
+		store_quad(vq, r, Q);
+		return;
+	}
+	Grad GV = {0.f, 0.f, 0.f, 0.f};
+
+	// kChunk corners' gathers in flight at a time; the sums stay in corner order
+	constexpr int kChunk = 4;
+	for (uint32_t p0 = begin; p0 < end; p0 += kChunk)
+	{
+		uint32_t t[kChunk], c[kChunk];
+#pragma unroll
+		for (int q = 0; q < kChunk; ++q)
 		{
-			// volume gradients of the position solve, summed in the same corner order
-			Grad G;
-			grad_volume(G, p0, p1, p2);
-			grad_add(GV, G);
+			const uint32_t j = wcorners[p0 + q < end ? p0 + q : begin];
+			t[q] = j / 3;
+			c[q] = j - t[q] * 3;
+		}
+		uint32_t i[kChunk][3];
+#pragma unroll
+		for (int q = 0; q < kChunk; ++q)
+#pragma unroll
+			for (int k = 0; k < 3; ++k)
+				i[q][k] = ib[t[q] * 3 + k];
+		V3 p[kChunk][3];
+#pragma unroll
+		for (int q = 0; q < kChunk; ++q)
+#pragma unroll
+			for (int k = 0; k < 3; ++k)
+				p[q][k] = load_pos(pos, i[q][k]);
+#pragma unroll
+		for (int q = 0; q < kChunk; ++q)
+		{
+			if (p0 + q >= end)
+				continue;
+			// the first pass's adjacency: the corner's next and previous classes
+			adj[p0 + q] = make_uint2(remap[c[q] == 0 ? i[q][1] : (c[q] == 1 ? i[q][2] : i[q][0])], remap[c[q] == 0 ? i[q][2] : (c[q] == 1 ? i[q][0] : i[q][1])]);
+			Quad F;
+			quad_from_triangle(F, p[q][0], p[q][1], p[q][2], 1.f);
+			quad_add(Q, F);
+			if (vg)
+			{
+				// volume gradients of the position solve, summed in the same corner order
+				Grad G;
+				grad_volume(G, p[q][0], p[q][1], p[q][2]);
+				grad_add(GV, G);
+			}
 		}
 	}
 	if (vg)
@@ -697,8 +936,10 @@ __global__ void k_vertex_quadrics(const uint32_t* ib, const float4* pos, const u
 		quad_add(Q, P);
 	}
 
+	// a manifold vertex has no open edge, and only open edges qualify below (loop and loopback are
+	// the open edges of the set-up)
 	uint32_t last_t = kNone;
-	for (uint32_t p = begin; p < end; ++p)
+	for (uint32_t p = kind[r] == kManifold ? end : begin; p < end; ++p)
 	{
 		uint32_t t = wcorners[p] / 3;
 		if (t == last_t)
@@ -736,7 +977,8 @@ void launch_vertex_quadrics(hipStream_t s, Mesh& m, const uint32_t* welded_off, 
 		return;
 	float factor = (options & kOptRegularizeLight) ? 1e-2f : ((options & kOptRegularize) ? 1e-1f : 1e-7f);
 	k_vertex_quadrics<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], m.pos, m.remap, m.kind, m.loop[0], m.loopback[0], welded_off, welded_corners,
-	                                                   vertex_lock, sparse_remap, n, factor, m.vq, m.vg, m.adj_range[0], m.adj[0]);
+	                                                   vertex_lock, sparse_remap, n, factor, m.vq, m.vg, m.adj_range[0], m.adj[0],
+	                                                   (uint64_t)m.index_count, m.sc);
 }
 
 // attribute quadrics and gradients (src/simplifier.cpp:1159-1179), per wedge (not welded),
@@ -819,40 +1061,6 @@ void launch_attribute_quadrics(hipStream_t s, Mesh& m, const uint32_t* raw_off, 
 #undef CASE
 	default:
 		k_attribute_quadrics<0><<<g, kThreads, 0, s>>>(m.ib[0], m.pos, m.va, raw_off, raw_corners, n, A, m.aq, m.ag);
-	}
-}
-
-// boundEdgeCollapses dual count, src/simplifier.cpp:1292-1308
-__global__ void __launch_bounds__(256) k_dual_count(const uint8_t* kind, const uint32_t* off, size_t n, uint32_t* out)
-{
-	__shared__ uint32_t red[4];
-	uint32_t v = 0;
-	for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-	{
-		uint8_t k = kind[i];
-		v += (k == kManifold || k == kSeam) ? off[i + 1] - off[i] : 0u;
-	}
-	for (int o = 32; o > 0; o >>= 1)
-		v += __shfl_xor(v, o, 64);
-	if (__lane_id() == 0)
-		red[threadIdx.x >> 6] = v;
-	__syncthreads();
-	if (threadIdx.x == 0)
-	{
-		uint32_t t = red[0] + red[1] + red[2] + red[3];
-		if (t)
-			atomicAdd(out, t);
-	}
-}
-
-void launch_dual_count(hipStream_t s, Mesh& m, const uint32_t* raw_off)
-{
-	HIP_CHECK(hipMemsetAsync(&m.sc->dual_count, 0, sizeof(uint32_t), s));
-	if (m.vertex_count)
-	{
-		unsigned int blocks = div_up(m.vertex_count, 256 * 8);
-		blocks = blocks > 512 ? 512 : blocks;
-		k_dual_count<<<blocks, 256, 0, s>>>(m.kind, raw_off, m.vertex_count, &m.sc->dual_count);
 	}
 }
 
