@@ -1792,6 +1792,10 @@ static int simplify_batch_on_device(Context& ctx, const BatchMemory& mem, unsign
 		if (timed)
 			HIP_CHECK(hipEventRecord(ctx.batch_ev[0], s));
 		static_assert(kBatchClasses <= 4, "one count word per class before the id lists");
+		// the classifier writes the class counts to host memory too: marked here, to see them arrive
+		constexpr uint32_t kNotYet = 0xffffffffu;
+		volatile uint32_t* const h_large = h_status + P + kBatchClasses - 1;
+		*h_large = kNotYet;
 		if (!launch_batch_classify_order(s, a, classes, ids, counts, host_counts))
 		{
 			fill_u32(s, counts, 0u, kBatchClasses);
@@ -1839,7 +1843,7 @@ static int simplify_batch_on_device(Context& ctx, const BatchMemory& mem, unsign
 		// shorter tail (the 4096-patch batch split over classes 1 and 2 at 6 and 5 per CU measured
 		// 0.557 ms with the largest class launched last, 0.512 ms with it first).
 		// A workgroup of class 3 takes a whole CU's LDS, so even one that leaves at once waits for
-		// a free CU: class 3 launches after the status read-back, only when it has meshes, with at
+		// a free CU: class 3 launches on its own (below), only when it has meshes, with at
 		// most one workgroup per CU looping over them (reading the counts back before launching
 		// classes 2 and 3 instead measured 4.5% slower on the 4096-patch batch).
 		static constexpr int kLaunchOrder[kBatchClasses - 1] = {2, 1, 0};
@@ -1855,6 +1859,25 @@ static int simplify_batch_on_device(Context& ctx, const BatchMemory& mem, unsign
 			{
 				HIP_CHECK(hipEventRecord(ctx.join_ev[c - 1], cs));
 				HIP_CHECK(hipStreamWaitEvent(s, ctx.join_ev[c - 1], 0));
+			}
+		}
+		// class 3 does not wait for the others: its count comes to host memory as soon as the classifier
+		// has ended (about when the launches above are through), and its workgroups take the CUs that
+		// the others leave free.  Launched after the status read-back instead, 777 meshes of 20-1900
+		// triangles took 0.97 ms against 0.90
+		if (!big_early && mem.host_dev && classes.icap[big])
+		{
+			const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+			while (*h_large == kNotYet && std::chrono::steady_clock::now() < give_up)
+				;
+			const uint32_t large = *h_large;
+			if (large != kNotYet && large)
+			{
+				big_early = true;
+				HIP_CHECK(hipStreamWaitEvent(ctx.aux[big - 1], ctx.fork_ev, 0));
+				launch_class(ctx.aux[big - 1], big, ids + (size_t)big * P, counts + big, large, big);
+				HIP_CHECK(hipEventRecord(ctx.join_ev[big - 1], ctx.aux[big - 1]));
+				HIP_CHECK(hipStreamWaitEvent(s, ctx.join_ev[big - 1], 0));
 			}
 		}
 		if (timed)

@@ -121,16 +121,31 @@ __device__ __forceinline__ float quad_error(const Quad& Q, const V3& v)
 }
 
 // quadricError (attributes), src/simplifier.cpp:784-799
+template <int kGroup = 4>
 __device__ __forceinline__ float quad_error_attr(const Quad& Q, const Grad* G, int n, const V3& v, const float* va)
 {
 	float r = quad_eval(Q, v);
 
-	for (int k = 0; k < n; ++k)
+	// the loads of kGroup attributes before the first is used; the sum stays in attribute order
+	// (one attribute at a time, with 5 of them: 1024 x 1024 seamed grid 8.78 ms, so 8.68)
+	for (int k0 = 0; k0 < n; k0 += kGroup)
 	{
-		float a = va[k];
-		Grad g4 = G[k];
-		float g = v.x * g4.gx + v.y * g4.gy + v.z * g4.gz + g4.gw;
-		r += a * (a * Q.w - 2 * g);
+		float a[kGroup];
+		Grad g4[kGroup];
+#pragma unroll
+		for (int q = 0; q < kGroup; ++q)
+		{
+			const int k = k0 + q < n ? k0 + q : n - 1;
+			a[q] = va[k];
+			g4[q] = G[k];
+		}
+#pragma unroll
+		for (int q = 0; q < kGroup; ++q)
+		{
+			float g = v.x * g4[q].gx + v.y * g4[q].gy + v.z * g4[q].gz + g4[q].gw;
+			const float t = a[q] * (a[q] * Q.w - 2 * g);
+			r = k0 + q < n ? r + t : r;
+		}
 	}
 
 	return fabsf(r);
