@@ -226,13 +226,6 @@ __device__ __forceinline__ int thread_id()
 	return t;
 }
 
-// orders the wavefront's own LDS accesses before it against those after it
-__device__ __forceinline__ void wave_fence()
-{
-	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-}
-
 // exclusive scan of one value per thread across the workgroup; `part` holds kBatchThreads/64 words
 __device__ __forceinline__ uint32_t wg_scan(uint32_t v, uint32_t* part, uint32_t& total)
 {

@@ -162,6 +162,13 @@ __device__ __forceinline__ void wait_for_memory()
 	asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 }
 
+// orders the wavefront's own LDS accesses before it against those after it
+__device__ __forceinline__ void wave_fence()
+{
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+}
+
 // 64-bit minimum / maximum over the 64 lanes of a wavefront
 __device__ __forceinline__ uint64_t wave_min64(uint64_t v)
 {

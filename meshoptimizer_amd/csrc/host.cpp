@@ -1181,7 +1181,7 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 	const size_t o_ek = take(4 * (3 * T + 1)), o_ev = take(4 * (3 * T + 1)), o_eka = take(4 * (3 * T + 1)), o_eva = take(4 * (3 * T + 1));
 	const size_t o_coff = take(4 * (V + 2)), o_stemp = take(4 * sort_words), o_ctemp = take(4 * scan_words), o_cq = take(sizeof(Quad) * (V + 1));
 	const size_t o_best = take(8 * (V + 1)), o_cremap = take(4 * (V + 1)), o_tri = take(16 * (T + 1)), o_ttable = take(4 * (size_t)ttable_size);
-	const size_t o_keep = take(4 * (T + 2)), o_face = take(sizeof(Quad) * (T + 1));
+	const size_t o_keep = take(4 * (T + 2)), o_parts = take(8 * sloppy_count_parts()), o_single = take(8 * (T / 64 + 1));
 	ctx.ensure_arena(off);
 	char* base = ctx.arena;
 
@@ -1190,7 +1190,8 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 	m.praw = reinterpret_cast<float4*>(base + o_praw);
 	m.pos = reinterpret_cast<float4*>(base + o_pos);
 	m.sc = reinterpret_cast<CallScalars*>(base + o_sc);
-	uint32_t* words = reinterpret_cast<uint32_t*>(base + o_words); // count, cell count, kept, error bits, index check
+	uint32_t* words = reinterpret_cast<uint32_t*>(base + o_words); // workgroups done, error bits, index check
+	uint32_t* h = ctx.sloppy_pinned(); // written by kernels: two counts, cell count, kept, error bits; copied: index check
 
 	SloppyBuffers b{};
 	b.indices = indices;
@@ -1198,7 +1199,9 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 	b.lock = lock;
 	b.vertex_count = (uint32_t)V;
 	b.index_count = (uint32_t)I;
-	b.count = words + 0;
+	b.count_parts = reinterpret_cast<uint64_t*>(base + o_parts);
+	b.count_done = words + 0;
+	b.host_counts = h;
 	b.ids = reinterpret_cast<uint32_t*>(base + o_ids);
 	b.vtable = reinterpret_cast<uint32_t*>(base + o_vtable);
 	b.vtable_size = vtable_size;
@@ -1210,39 +1213,35 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 	b.entry_vals = reinterpret_cast<uint32_t*>(base + o_ev);
 	b.entry_keys_alt = reinterpret_cast<uint32_t*>(base + o_eka);
 	b.entry_vals_alt = reinterpret_cast<uint32_t*>(base + o_eva);
+	b.single_bits = reinterpret_cast<uint64_t*>(base + o_single);
 	b.cell_off = reinterpret_cast<uint32_t*>(base + o_coff);
 	b.sort_temp = reinterpret_cast<uint32_t*>(base + o_stemp);
 	b.scan_temp = reinterpret_cast<uint32_t*>(base + o_ctemp);
 	b.cq = reinterpret_cast<Quad*>(base + o_cq);
 	b.best = reinterpret_cast<uint64_t*>(base + o_best);
 	b.cell_remap = reinterpret_cast<uint32_t*>(base + o_cremap);
-	b.error_bits = words + 3;
+	b.error_bits = words + 1;
 	b.tri = reinterpret_cast<uint4*>(base + o_tri);
 	b.ttable = reinterpret_cast<uint32_t*>(base + o_ttable);
 	b.ttable_size = ttable_size;
 	b.keep = reinterpret_cast<uint32_t*>(base + o_keep);
-	b.face = reinterpret_cast<Quad*>(base + o_face);
 
-	uint32_t* h = ctx.sloppy_pinned();
-	auto read_words = [&](int first, int count) {
-		HIP_CHECK(hipMemcpyAsync(h + first, words + first, count * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-		HIP_CHECK(hipStreamSynchronize(s));
-	};
-
+	launch_call_init(s, m.sc, words, 8);
+	if (I)
+	{
+		launch_check_indices(s, indices, I, V, words + 2);
+		HIP_CHECK(hipMemcpyAsync(h + 5, words + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+	}
+	// rescalePositions (src/simplifier.cpp:549-603)
+	launch_gather_positions(s, m, positions, stride / sizeof(float), nullptr, nullptr, 0);
+	launch_rescale(s, m);
 	// every later gather trusts the indices: reject out-of-range ones before any kernel uses them
 	if (I)
 	{
-		HIP_CHECK(hipMemsetAsync(words + 4, 0, sizeof(uint32_t), s));
-		launch_check_indices(s, indices, I, V, words + 4);
-		read_words(4, 1);
-		if (h[4])
+		HIP_CHECK(hipStreamSynchronize(s));
+		if (h[5])
 			throw std::invalid_argument("meshopt_simplifySloppy: index buffer references a vertex >= vertex_count");
 	}
-
-	// rescalePositions (src/simplifier.cpp:549-603)
-	launch_call_init(s, m.sc, nullptr, 0);
-	launch_gather_positions(s, m, positions, stride / sizeof(float), nullptr, nullptr, 0);
-	launch_rescale(s, m);
 	// the extent meshopt_simplifyScale returns for the same vertices (rescalePositions, without the
 	// rescale), asked for by the clusterlod fallback
 	if (out_extent)
@@ -1251,10 +1250,9 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 		HIP_CHECK(hipStreamSynchronize(s));
 	}
 
-	auto count_at = [&](int grid_size) -> size_t {
-		launch_sloppy_count(s, b, grid_size);
-		read_words(0, 1);
-		return h[0];
+	auto count_at = [&](int grid_size, int second_grid_size) {
+		launch_sloppy_count(s, b, grid_size, second_grid_size);
+		HIP_CHECK(hipStreamSynchronize(s));
 	};
 
 	// the guided grid-size search (src/simplifier.cpp:2667-2723)
@@ -1264,17 +1262,25 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 	int max_grid = 1025;
 	size_t min_triangles = 0;
 	size_t max_triangles = T;
-	if (min_grid > 1 || lock)
-		min_triangles = count_at(min_grid);
-
 	int next_grid_size = int(sqrtf(float(target_cell_count)) + 0.5f);
+	auto clamped = [&](int grid_size) { return (grid_size <= min_grid) ? min_grid + 1 : (grid_size >= max_grid ? max_grid - 1 : grid_size); };
+	int counted = 0; // grid size of the search's first step, when it was counted with min_grid
+	if (min_grid > 1 || lock)
+	{
+		counted = max_grid - min_grid > 1 ? clamped(next_grid_size) : 0;
+		count_at(min_grid, counted);
+		min_triangles = h[0];
+	}
+
 	for (int pass = 0; pass < 10 + interpolation_passes; ++pass)
 	{
 		if (min_triangles >= target_index_count / 3 || max_grid - min_grid <= 1)
 			break;
-		int grid_size = next_grid_size;
-		grid_size = (grid_size <= min_grid) ? min_grid + 1 : (grid_size >= max_grid ? max_grid - 1 : grid_size);
-		const size_t triangles = count_at(grid_size);
+		const int grid_size = clamped(next_grid_size);
+		const bool known = pass == 0 && counted;
+		if (!known)
+			count_at(grid_size, 0);
+		const size_t triangles = known ? h[1] : h[0];
 		const float tip = sloppy_interpolate(float(size_t(target_index_count / 3)), float(min_grid), float(min_triangles), float(grid_size),
 		                                     float(triangles), float(max_grid), float(max_triangles));
 		if (triangles <= target_index_count / 3)
@@ -1297,15 +1303,14 @@ static size_t sloppy_on_device(Context& ctx, unsigned int* destination, const un
 		return 0;
 	}
 
-	launch_sloppy_cells(s, b, min_grid, words + 1);
-	read_words(1, 1);
-	const uint32_t cell_count = h[1];
-	launch_sloppy_quadrics(s, b, cell_count);
-	launch_sloppy_filter(s, b, cell_count, destination, words + 2);
-	read_words(2, 2);
-	const uint32_t kept = h[2];
+	launch_sloppy_cells(s, b, min_grid, h + 2);
+	HIP_CHECK(hipStreamSynchronize(s));
+	launch_sloppy_quadrics(s, b, h[2]);
+	launch_sloppy_filter(s, b, destination, h + 3, h + 4);
+	HIP_CHECK(hipStreamSynchronize(s));
+	const uint32_t kept = h[3];
 	float err_sq;
-	memcpy(&err_sq, &h[3], sizeof(float));
+	memcpy(&err_sq, &h[4], sizeof(float));
 	if (out_result_error)
 		*out_result_error = sqrtf(err_sq);
 	return (size_t)kept * 3;

@@ -26,8 +26,10 @@ void scan_exclusive(hipStream_t s, const uint32_t* in, uint32_t* out, size_t n, 
 size_t sort_temp_words(size_t n);
 
 // stable sort of (keys, vals) by the low `bits` bits of the key; the sorted pairs end in
-// (keys, vals) on return (the alt buffers are ping-pong space of the same size)
-void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, size_t n, const uint32_t* n_dev, int bits, uint32_t* temp);
+// (keys, vals) on return (the alt buffers are ping-pong space of the same size); with
+// places_as_vals the values on entry are 0, 1, 2, ... and vals need not hold them
+void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, size_t n, const uint32_t* n_dev, int bits, uint32_t* temp,
+                      bool places_as_vals = false);
 
 void fill_u32(hipStream_t s, uint32_t* p, uint32_t value, size_t n);
 void iota_u32(hipStream_t s, uint32_t* p, size_t n);

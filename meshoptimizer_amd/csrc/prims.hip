@@ -180,86 +180,98 @@ void scan_exclusive(hipStream_t s, const uint32_t* in, uint32_t* out, size_t n, 
 __global__ void __launch_bounds__(kSortThreads) k_radix_hist(const uint32_t* keys, size_t n_max, const uint32_t* n_dev, int shift, uint32_t* counts)
 {
 	__shared__ uint32_t hist[256];
-	size_t n = live_count(n_dev, n_max);
-	hist[threadIdx.x] = 0;
-	__syncthreads();
-	size_t base = (size_t)blockIdx.x * kSortTile;
-#pragma unroll 4
+	const size_t n = live_count(n_dev, n_max);
+	const size_t base = (size_t)blockIdx.x * kSortTile + threadIdx.x;
+	uint32_t key[kSortItems];
+#pragma unroll
 	for (int j = 0; j < kSortItems; ++j)
 	{
-		size_t e = base + (size_t)j * kSortThreads + threadIdx.x;
-		if (e < n)
-			atomicAdd(&hist[(keys[e] >> shift) & 255u], 1u);
+		const size_t e = base + (size_t)j * kSortThreads;
+		key[j] = e < n ? keys[e] : 0u;
 	}
+	hist[threadIdx.x] = 0;
+	__syncthreads();
+#pragma unroll
+	for (int j = 0; j < kSortItems; ++j)
+		if (base + (size_t)j * kSortThreads < n)
+			atomicAdd(&hist[(key[j] >> shift) & 255u], 1u);
 	__syncthreads();
 	counts[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = hist[threadIdx.x];
 }
 
+// A tile per workgroup, a quarter of it per wavefront, which has a row of the digits' places to
+// itself: the rows are counted and turned into places once, then each wavefront goes through its
+// 16 chunks of 64 without a barrier, its pairs loaded beforehand (two barriers for every 256 pairs,
+// each loaded when its turn came, took 47 us for 3.9 million pairs against 34).
+// Without `vals`, an element's value is its place in `keys`.
 __global__ void __launch_bounds__(kSortThreads) k_radix_scatter(const uint32_t* keys, const uint32_t* vals, uint32_t* keys_out, uint32_t* vals_out, size_t n_max, const uint32_t* n_dev, int shift, const uint32_t* offsets)
 {
-	__shared__ uint32_t run[256];
-	__shared__ uint32_t woff[2][4][256];
+	constexpr int kWaves = kSortThreads / 64;
+	__shared__ uint32_t places[kWaves][256];
 
-	size_t n = live_count(n_dev, n_max);
-	size_t base = (size_t)blockIdx.x * kSortTile;
-	if (base >= n)
+	const size_t n = live_count(n_dev, n_max);
+	if ((size_t)blockIdx.x * kSortTile >= n)
 		return;
 
 	const int t = threadIdx.x;
-	const int wave = t >> 6;
 	const int lane = __lane_id();
+	uint32_t* row = places[t >> 6];
+	const size_t base = (size_t)blockIdx.x * kSortTile + (size_t)(t >> 6) * (kSortTile / kWaves) + lane;
 
-	run[t] = offsets[(size_t)t * gridDim.x + blockIdx.x];
+	uint32_t key[kSortItems], val[kSortItems];
 #pragma unroll
-	for (int w = 0; w < 4; ++w)
+	for (int j = 0; j < kSortItems; ++j)
 	{
-		woff[0][w][t] = 0;
-		woff[1][w][t] = 0;
+		const size_t e = base + j * 64;
+		key[j] = e < n ? keys[e] : 0u;
+		val[j] = (uint32_t)e;
+		if (vals && e < n)
+			val[j] = vals[e];
+	}
+#pragma unroll
+	for (int q = 0; q < 256 / 64; ++q)
+		row[q * 64 + lane] = 0;
+	wave_fence();
+#pragma unroll
+	for (int j = 0; j < kSortItems; ++j)
+		if (base + j * 64 < n)
+			atomicAdd(&row[(key[j] >> shift) & 255u], 1u);
+	__syncthreads();
+	{
+		uint32_t at = offsets[(size_t)t * gridDim.x + blockIdx.x];
+#pragma unroll
+		for (int w = 0; w < kWaves; ++w)
+		{
+			const uint32_t c = places[w][t];
+			places[w][t] = at;
+			at += c;
+		}
 	}
 	__syncthreads();
 
+#pragma unroll
 	for (int j = 0; j < kSortItems; ++j)
 	{
-		uint32_t* off = &woff[j & 1][0][0];
-		uint32_t* off_next = &woff[(j + 1) & 1][0][0];
-
-		size_t e = base + (size_t)j * kSortThreads + t;
-		bool valid = e < n;
-		uint32_t key = valid ? keys[e] : 0u;
-		uint32_t d = (key >> shift) & 255u;
+		const bool valid = base + j * 64 < n;
+		const uint32_t d = (key[j] >> shift) & 255u;
 
 		uint64_t peers = __ballot(valid);
 #pragma unroll
 		for (int b = 0; b < 8; ++b)
 		{
-			uint64_t bb = __ballot((d >> b) & 1u);
+			const uint64_t bb = __ballot((d >> b) & 1u);
 			peers &= ((d >> b) & 1u) ? bb : ~bb;
 		}
-		uint64_t lower = peers & ((1ull << lane) - 1ull);
-		uint32_t rank = (uint32_t)__popcll(lower);
-		if (valid && (63 - __clzll((long long)peers)) == lane)
-			off[wave * 256 + d] = (uint32_t)__popcll(peers);
-		__syncthreads();
-
-		{
-			uint32_t c0 = off[0 * 256 + t], c1 = off[1 * 256 + t], c2 = off[2 * 256 + t], c3 = off[3 * 256 + t];
-			uint32_t r = run[t];
-			off[0 * 256 + t] = r;
-			off[1 * 256 + t] = r + c0;
-			off[2 * 256 + t] = r + c0 + c1;
-			off[3 * 256 + t] = r + c0 + c1 + c2;
-			run[t] = r + c0 + c1 + c2 + c3;
-#pragma unroll
-			for (int w = 0; w < 4; ++w)
-				off_next[w * 256 + t] = 0;
-		}
-		__syncthreads();
-
+		const uint32_t ahead = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+		const uint32_t place = row[d] + ahead;
+		wave_fence();
+		if (valid && ahead == 0)
+			row[d] += (uint32_t)__popcll(peers);
+		wave_fence();
 		if (valid)
 		{
-			uint32_t pos = off[wave * 256 + d] + rank;
-			keys_out[pos] = key;
-			vals_out[pos] = vals[e];
+			keys_out[place] = key[j];
+			vals_out[place] = val[j];
 		}
 	}
 }
@@ -270,7 +282,7 @@ size_t sort_temp_words(size_t n)
 	return 256 * blocks + scan_temp_words(256 * blocks) + 16;
 }
 
-void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, size_t n, const uint32_t* n_dev, int bits, uint32_t* temp)
+void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, size_t n, const uint32_t* n_dev, int bits, uint32_t* temp, bool places_as_vals)
 {
 	if (n == 0 || bits <= 0)
 		return;
@@ -285,7 +297,7 @@ void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* k
 		int shift = p * 8;
 		k_radix_hist<<<blocks, kSortThreads, 0, s>>>(ka, n, n_dev, shift, counts);
 		scan_exclusive(s, counts, counts, 256 * (size_t)blocks, nullptr, nullptr, scan_tmp);
-		k_radix_scatter<<<blocks, kSortThreads, 0, s>>>(ka, va, kb, vb, n, n_dev, shift, counts);
+		k_radix_scatter<<<blocks, kSortThreads, 0, s>>>(ka, p == 0 && places_as_vals ? nullptr : va, kb, vb, n, n_dev, shift, counts);
 		uint32_t* t;
 		t = ka, ka = kb, kb = t;
 		t = va, va = vb, vb = t;

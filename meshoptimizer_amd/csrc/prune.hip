@@ -337,9 +337,8 @@ void launch_measure_components(hipStream_t s, Mesh& m, const uint32_t* comp, flo
 	uint32_t* vals_alt = scratch[3];
 	uint32_t* off = scratch[4];
 	k_copy_u32<<<prune_grid(V), kPruneThreads, 0, s>>>(comp, keys, V);
-	iota_u32(s, vals, V);
 	// stable: each component's vertices stay in index order (the reference's summation order)
-	radix_sort_pairs(s, keys, vals, keys_alt, vals_alt, V, nullptr, bits_for(V), m.temp);
+	radix_sort_pairs(s, keys, vals, keys_alt, vals_alt, V, nullptr, bits_for(V), m.temp, true);
 	k_component_offsets<<<prune_grid(V), kPruneThreads, 0, s>>>(keys, V, off);
 	// the sorted keys are not needed any more: their space holds the list of long components
 	k_set_u32<<<1, 1, 0, s>>>(&m.sc->work[0], 0u);

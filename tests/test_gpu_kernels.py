@@ -113,3 +113,23 @@ def test_candidate_tiles(side):
         ro, eo = O.simplify(m.indices, m.vertices, target, err, 0)
         assert np.array_equal(rg, ro)
         assert same_bits(eg, eo), (eg, eo)
+
+
+@pytest.mark.parametrize("side,grid", [(2, 2), (17, 3), (27, 3), (27, 26), (64, 4), (64, 20), (300, 6), (300, 150), (516, 40)])
+def test_sloppy_cells(side, grid):
+    """Cells of few and of many triangles (both forms of the cell sums) and entry counts around the
+    sort's tile, with runs of vertices in one cell longer and shorter than a wavefront; locked
+    vertices are cells of their own."""
+    rng = np.random.default_rng(side * 1000 + grid)
+    g = np.linspace(0, 1, side, dtype=np.float32)
+    x, y = np.meshgrid(g, g)
+    v = np.stack([x.ravel(), y.ravel(), 0.1 * rng.random(side * side).astype(np.float32)], axis=1).astype(np.float32)
+    q = (np.arange(side - 1)[:, None] * side + np.arange(side - 1)).ravel()
+    ib = np.stack([q, q + 1, q + side, q + 1, q + side + 1, q + side], axis=1).reshape(-1).astype(np.uint32)
+    for lock in (None, (rng.random(side * side) < 0.02).astype(np.uint8)):
+        for target in (0, ib.size // 3 // 4 * 3):
+            announce(f"sloppy cells side={side} grid={grid} lock={lock is not None} target={target}")
+            rg, eg = M.simplify_sloppy(ib, v, target, 1.0 / grid, lock=lock)
+            ro, eo = O.simplify_sloppy(ib, v, target, 1.0 / grid, lock=lock)
+            assert np.array_equal(rg, ro)
+            assert same_bits(eg, eo), (eg, eo)
