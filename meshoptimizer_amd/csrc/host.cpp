@@ -798,7 +798,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		bool deep = long_chains || learned > deep_heads || deep_heads < 0;
 		launch_rank_sort(s, m, C, W);
 		if (deep)
-			launch_source_lists(s, m, C);
+			launch_source_lists(s, m, W);
 		// head rounds with one thread per rank of the window (the list only shrinks; workgroups
 		// past its current length leave at once, while a grid smaller than the list would make
 		// each thread walk several ranks' dependent gathers in turn), then the tail
@@ -830,7 +830,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 					break;
 				if (!deep && deep_heads >= 0 && done >= deep_heads && left >= kTailList)
 				{
-					launch_source_lists(s, m, C);
+					launch_source_lists(s, m, W);
 					deep = switched_deep = true;
 				}
 				batch = done;
@@ -850,6 +850,8 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		if (extended)
 		{
 			// the rest of the list
+			if (deep)
+				launch_source_lists(s, m, C);
 			launch_window_open(s, m, W, C, false);
 			window_rounds(W, C, heads_run, ext_heads);
 			launch_stop_scan(s, m, C, C, goal, error_limit);

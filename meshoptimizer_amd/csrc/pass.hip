@@ -792,37 +792,43 @@ __device__ __forceinline__ uint32_t commit_value_at(const RoundState& a, uint32_
 // the per-source candidate lists; a candidate counts unless it is known never to commit (skipped,
 // flip-failed, rejected), so the set is never smaller than the true one, whatever stores of the
 // same round the test sees.  An outcome that holds in every combination is final; a triangle
-// without a moving corner decides alone.  Limited to kMaxAlternatives per corner and
-// kMaxPendingSlots moving corners; beyond that the rank waits.
+// without a moving corner decides alone.  Limited to kMaxAlternatives per corner; beyond that the
+// rank waits.
 //
-// The test is a chain of dependent gathers, so the adjacency is read in chunks of kFlipChunk
-// entries, and a source list kSrcChunk ranks at a time, with the gathers of each level issued
-// before any is used.
+// The test is a chain of dependent gathers.  The deep test has kDeepLanes lanes for a rank, one for
+// each adjacency entry, so that the entries' chains run side by side: its rounds have few ranks
+// (tens of thousands falling to hundreds) and are bound by the length of the chain.  One thread
+// going through the entries one after the other took 42 us a round on the 998 x 998 grid
+// whatever the list's length; the lanes take 42 at 50 thousand ranks, 25 at 15 thousand and 12 below
+// 4 thousand, and the call went from 17.3 to 10.9 ms.  The cheap test, whose first rounds have
+// hundreds of thousands of ranks, keeps a thread for a rank and reads the adjacency
+// kCheapFlipChunk entries at a time, the gathers of each level issued before any is used.
 
-constexpr int kFlipChunk = 4;      // the deep test's adjacency chunk
-constexpr int kCheapFlipChunk = 4; // the cheap test's
+constexpr int kDeepLanes = 8;
+constexpr int kCheapFlipChunk = 4;
 constexpr int kCheapWaves = 5;     // waves per SIMD the cheap round kernel is built for
-constexpr int kSrcChunk = 8;
+constexpr int kSrcChunk = 8;       // ranks of a source list read at a time
 constexpr int kMaxAlternatives = 2; // per corner: its current value and one possible move
-constexpr int kMaxPendingSlots = 4; // moving corners before the rank waits
 
-// one adjacency entry with moving corners (pend2: bit h set when corner h moves): 0 mixed, 1 passes
-// in all combinations, 2 fails in all, 3 too many alternatives
-__device__ int flip_entry_pending(const RoundState& a, uint32_t k, const uint32_t nb[2], const uint32_t seen[2], uint32_t pend2, const V3& v0,
-                                  const V3& v1, uint32_t i1)
+// collapse_remap of a class as rank k sees it: a move committed by a higher rank (possible once flip
+// tests are decided early) reads as "not moved"
+__device__ __forceinline__ uint32_t seen_by(uint32_t k, uint32_t cls, uint32_t moved, uint32_t lock_rank)
+{
+	return moved != cls && lock_rank > k ? cls : moved;
+}
+
+// one adjacency entry with moving corners (pend2: bit h set when corner h moves; tb, te: the corners'
+// source lists): 0 mixed or too many alternatives, 1 passes in all combinations, 2 fails in all
+__device__ int flip_entry_pending(const RoundState& a, uint32_t k, const uint32_t nb[2], const uint32_t seen[2], uint32_t pend2, uint32_t tb[2],
+                                  uint32_t te[2], const V3& v0, const V3& v1, uint32_t i1)
 {
 	uint32_t alt[2][kMaxAlternatives];
 	int na[2] = {1, 1};
 	alt[0][0] = seen[0];
 	alt[1][0] = seen[1];
-	uint32_t tb[2], te[2];
 #pragma unroll
 	for (int q = 0; q < 2; ++q)
-	{
-		const bool scan = (pend2 >> q) & 1u;
-		tb[q] = scan ? a.src_off[nb[q]] : 0;
-		te[q] = scan ? a.src_off[nb[q] + 1] : 0;
-	}
+		te[q] = (pend2 >> q) & 1u ? te[q] : tb[q];
 	bool more = true;
 	for (uint32_t step = 0; more; step += kSrcChunk)
 	{
@@ -853,7 +859,7 @@ __device__ int flip_entry_pending(const RoundState& a, uint32_t k, const uint32_
 				if (st[q][u] == kSkipped || st[q][u] == kRejected || st[q][u] == kFlipFail || val[q][u] == alt[q][0])
 					continue;
 				if (na[q] == kMaxAlternatives)
-					return 3;
+					return 0;
 				alt[q][na[q]++] = val[q][u];
 			}
 			more |= tb[q] + step + kSrcChunk < te[q];
@@ -877,14 +883,14 @@ __device__ int flip_entry_pending(const RoundState& a, uint32_t k, const uint32_
 }
 
 // begin/end: rank k's source's adjacency range; v0, v1: the positions of its source and target.
-// kDeep: examine the combinations of the moving corners' alternatives; otherwise a rank with a
-// moving corner waits (the cheap test of the first rounds of a window, when most corners move)
-template <bool kDeep, int kChunk = kDeep ? kFlipChunk : kCheapFlipChunk>
-__device__ int flip_outcome(const RoundState& a, uint32_t i1, uint32_t k, uint32_t epoch, uint32_t begin, uint32_t end, const V3& v0, const V3& v1)
+// The cheap test: a rank with a moving corner waits (in the first rounds of a window most corners
+// move), unless a triangle without one fails
+__device__ __forceinline__ int flip_outcome_cheap(const RoundState& a, uint32_t i1, uint32_t k, uint32_t epoch, uint32_t begin, uint32_t end, const V3& v0,
+                                                  const V3& v1)
 {
+	constexpr int kChunk = kCheapFlipChunk;
 	const uint64_t* prev_pend = a.pend[(epoch - 1) & 1];
 	const uint32_t prev_tag = ~(epoch - 1);
-	int pending = 0;
 	bool all_pass = true;
 	for (uint32_t p0 = begin; p0 < end; p0 += kChunk)
 	{
@@ -906,20 +912,15 @@ __device__ int flip_outcome(const RoundState& a, uint32_t i1, uint32_t k, uint32
 			lr[q] = a.lock_rank[nb[q]];
 			ps[q] = prev_pend[2 * nb[q]];
 		}
-		// collapse_remap as rank k sees it: a move committed by a higher rank (possible once
-		// flip tests are decided early) reads as "not moved"
 		uint32_t seen[2 * kChunk];
 		uint32_t pend_mask = 0;
 #pragma unroll
 		for (int q = 0; q < 2 * kChunk; ++q)
 		{
-			seen[q] = (cm[q] != nb[q] && lr[q] > k) ? nb[q] : cm[q];
+			seen[q] = seen_by(k, nb[q], cm[q], lr[q]);
 			const bool moving = (uint32_t)(q / 2) < n && (uint32_t)(ps[q] >> 32) == prev_tag && (uint32_t)ps[q] < k;
 			pend_mask |= moving ? 1u << q : 0u;
 		}
-		pending += __builtin_popcount(pend_mask);
-		if (kDeep && pending > kMaxPendingSlots)
-			return 0;
 		// entries without a moving corner have one scenario: the positions they need, all at once
 		V3 pa[kChunk], pb[kChunk];
 		uint32_t test_mask = 0;
@@ -937,26 +938,67 @@ __device__ int flip_outcome(const RoundState& a, uint32_t i1, uint32_t k, uint32
 		for (int j = 0; j < kChunk; ++j)
 			if (((test_mask >> j) & 1u) && triangle_flips(pa[j], pb[j], v0, v1))
 				return 2;
-		if (!kDeep)
+		all_pass &= pend_mask == 0;
+	}
+	return all_pass ? 1 : 0;
+}
+
+// whether any lane of this lane's kDeepLanes has the bit set in a wavefront's mask
+__device__ __forceinline__ bool any_of_group(uint64_t mask)
+{
+	return (mask >> (__lane_id() & ~(kDeepLanes - 1)) & ((1u << kDeepLanes) - 1)) != 0;
+}
+
+// the deep test, called by the rank's kDeepLanes lanes together: each takes an entry and every
+// combination of its moving corners' alternatives.  What an entry may need is gathered with its
+// state: the unmoved corners' positions and the bounds of their source lists
+__device__ __forceinline__ int flip_outcome_deep(const RoundState& a, uint32_t i1, uint32_t k, uint32_t epoch, uint32_t begin, uint32_t end, const V3& v0,
+                                                 const V3& v1)
+{
+	const uint64_t* prev_pend = a.pend[(epoch - 1) & 1];
+	const uint32_t prev_tag = ~(epoch - 1);
+	bool all_pass = true;
+	for (uint32_t p0 = begin; p0 < end; p0 += kDeepLanes)
+	{
+		const uint32_t p = p0 + (__lane_id() & (kDeepLanes - 1));
+		int outcome = 1;
+		if (p < end)
 		{
-			all_pass &= pending == 0;
-			continue;
+			const uint2 e = a.adj[p];
+			const uint32_t nb[2] = {e.x, e.y};
+			uint32_t cm[2], lr[2], tb[2], te[2], seen[2], pend2 = 0;
+			uint64_t ps[2];
+			V3 at[2];
+#pragma unroll
+			for (int q = 0; q < 2; ++q)
+			{
+				cm[q] = a.cremap[nb[q]];
+				lr[q] = a.lock_rank[nb[q]];
+				ps[q] = prev_pend[2 * (size_t)nb[q]];
+				at[q] = load_pos(a.pos, nb[q]);
+				tb[q] = a.src_off[nb[q]];
+				te[q] = a.src_off[nb[q] + 1];
+			}
+#pragma unroll
+			for (int q = 0; q < 2; ++q)
+			{
+				seen[q] = seen_by(k, nb[q], cm[q], lr[q]);
+				pend2 |= (uint32_t)(ps[q] >> 32) == prev_tag && (uint32_t)ps[q] < k ? 1u << q : 0u;
+			}
+			if (pend2)
+				outcome = flip_entry_pending(a, k, nb, seen, pend2, tb, te, v0, v1, i1);
+			else if (seen[0] != i1 && seen[1] != i1 && seen[0] != seen[1])
+			{
+#pragma unroll
+				for (int q = 0; q < 2; ++q)
+					if (seen[q] != nb[q])
+						at[q] = load_pos(a.pos, seen[q]);
+				outcome = triangle_flips(at[0], at[1], v0, v1) ? 2 : 1;
+			}
 		}
-		// entries with a moving corner: every combination of the alternatives
-		for (int j = 0; j < kChunk; ++j)
-		{
-			if ((uint32_t)j >= n || !((pend_mask >> (2 * j)) & 3u))
-				continue;
-			const uint32_t nbj[2] = {nb[2 * j], nb[2 * j + 1]};
-			const uint32_t seenj[2] = {seen[2 * j], seen[2 * j + 1]};
-			const int o = flip_entry_pending(a, k, nbj, seenj, (pend_mask >> (2 * j)) & 3u, v0, v1, i1);
-			if (o == 3)
-				return 0;
-			if (o == 2)
-				return 2;
-			if (o == 0)
-				all_pass = false;
-		}
+		if (any_of_group(__ballot(outcome == 2)))
+			return 2;
+		all_pass &= !any_of_group(__ballot(outcome == 0));
 	}
 	return all_pass ? 1 : 0;
 }
@@ -975,40 +1017,74 @@ __device__ int flip_outcome(const RoundState& a, uint32_t i1, uint32_t k, uint32
 // that commits in this round published its source then, so no test reads a move still in
 // flight.  A lock written in this round may be missed by a rank sharing that endpoint: that rank
 // publishes once more and is skipped in the next round, before it can commit.
+//
+// kDeep: the whole wavefront calls, and its ranks that need the test get it eight at a time.
 template <bool kDeep>
-__device__ __forceinline__ bool round_x(const RoundState& a, uint4 w, uint32_t epoch)
+__device__ __forceinline__ bool round_x(const RoundState& a, uint4 w, bool valid, uint32_t epoch)
 {
 	const uint32_t k = w.x, r0 = w.y, r1 = w.z;
 	const ulonglong2* prev = reinterpret_cast<const ulonglong2*>(a.pend[(epoch - 1) & 1]);
+	if (!kDeep && !valid)
+		return false;
+	// (a lane without a rank reads the entries of rank and class 0)
 	const uint8_t st = a.status[k];
 	const uint32_t l0 = a.lock_rank[r0], l1 = a.lock_rank[r1];
 	const ulonglong2 q0 = prev[r0], q1 = prev[r1];
 	const uint64_t p0 = q0.x < q0.y ? q0.x : q0.y, p1 = q1.x < q1.y ? q1.x : q1.y;
 	const uint2 range = a.adj_range[r0];
 	const V3 v0 = load_pos(a.pos, r0), v1 = load_pos(a.pos, r1);
-	if (st != kUndecided && st != kFlipPass)
+	bool live = valid && (st == kUndecided || st == kFlipPass);
+	if (!kDeep && !live)
 		return false;
-	if (l0 != kNone || l1 != kNone)
+	if (live && (l0 != kNone || l1 != kNone))
 	{
 		a.status[k] = kSkipped;
-		return false;
+		live = false;
 	}
+	if (!kDeep && !live)
+		return false;
 	// the flip test is only worth evaluating for a rank that was the lowest published at one of
 	// its endpoints in the previous round (others cannot commit yet)
 	const uint64_t was = round_key(epoch - 1, k);
 	const bool low0 = p0 == was, low1 = p1 == was;
-	uint8_t now = st;
-	if (st == kUndecided && (low0 || low1))
+	const bool test = live && st == kUndecided && (low0 || low1);
+	int o = 0;
+	if (kDeep)
 	{
-		int o = flip_outcome<kDeep>(a, r1, k, epoch, range.x, range.y, v0, v1);
-		if (o == 2)
+		const uint32_t lane = __lane_id();
+		const uint64_t below = (1ull << lane) - 1ull;
+		for (uint64_t todo = __ballot(test); todo;)
 		{
-			a.status[k] = kFlipFail;
-			return false;
+			// the next eight of them, one to each kDeepLanes lanes
+			uint64_t left = todo, mine = 0;
+#pragma unroll
+			for (uint32_t g = 0; g < 64 / kDeepLanes; ++g)
+			{
+				mine = lane / kDeepLanes == g ? left : mine;
+				left &= left - 1;
+			}
+			const int src = mine ? __ffsll((long long)mine) - 1 : 0;
+			const uint32_t tk = __shfl(k, src, 64), t1 = __shfl(r1, src, 64), begin = __shfl(range.x, src, 64), end = __shfl(range.y, src, 64);
+			const V3 t_v0 = {__shfl(v0.x, src, 64), __shfl(v0.y, src, 64), __shfl(v0.z, src, 64)};
+			const V3 t_v1 = {__shfl(v1.x, src, 64), __shfl(v1.y, src, 64), __shfl(v1.z, src, 64)};
+			const int outcome = mine ? flip_outcome_deep(a, t1, tk, epoch, begin, end, t_v0, t_v1) : 0;
+			const uint32_t place = (uint32_t)__popcll(todo & below);
+			const int got = __shfl(outcome, (int)(place * kDeepLanes) & 63, 64);
+			if ((todo >> lane & 1) && place < 64 / kDeepLanes)
+				o = got;
+			todo = left;
 		}
-		if (o == 1)
-			now = kFlipPass;
 	}
+	else if (test)
+		o = flip_outcome_cheap(a, r1, k, epoch, range.x, range.y, v0, v1);
+	if (!live)
+		return false;
+	if (o == 2)
+	{
+		a.status[k] = kFlipFail;
+		return false;
+	}
+	const uint8_t now = o == 1 ? (uint8_t)kFlipPass : st;
 	if (now == kFlipPass && low0 && low1)
 	{
 		const uint2 v = a.r_v[k];
@@ -1043,6 +1119,18 @@ __device__ __forceinline__ void append_wave(bool keep, uint4 w, uint4* out_list,
 	}
 }
 
+// wavefronts of the deep round kernel that one XCD's 32 CUs hold at once (4 to each SIMD)
+constexpr uint32_t kDeepSegmentWaves = 32 * 4 * 4;
+
+// ranks a wavefront takes of n in a deep round: as few as `waves` of them get through at once
+__device__ __forceinline__ uint32_t deep_ranks(uint32_t n, uint32_t waves)
+{
+	uint32_t ranks = 64 / kDeepLanes;
+	while (ranks < 64 && n > ranks * waves)
+		ranks *= 2;
+	return ranks;
+}
+
 // head round.  Round r reads list (r & 1) / counters (r % 3), appends the survivors to list
 // ((r + 1) & 1) / counters ((r + 1) % 3) and clears counters ((r + 2) % 3).  A rank stays in its
 // segment, at the segment's offset in both lists.  Workgroups are dealt to the XCDs in turn, so
@@ -1050,8 +1138,9 @@ __device__ __forceinline__ void append_wave(bool keep, uint4 w, uint4* out_list,
 // one segment's ranks rather than of all of them.  The grid is a multiple of kListSegments; one
 // rank per thread when it is large enough, and the grid-stride loop covers any segment length.
 // kDeep: this round examines the alternatives of moving corners (the window's per-source lists
-// are built).  Two kernels rather than a flag, so that the cheap rounds are not held to the deep
-// test's register count.
+// are built); a wavefront takes as few ranks as keep the list within the wavefronts that are
+// resident at once, so that few of its ranks' tests come one after the other.  Two kernels rather
+// than a flag, so that the cheap rounds are not held to the deep test's register count.
 template <bool kDeep>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kDeep ? 4 : kCheapWaves))) k_round_x(RoundState a, uint32_t head_index, uint32_t rel)
 {
@@ -1081,12 +1170,15 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(k
 	const uint4* in_list = a.list[round & 1] + off;
 	uint4* out_list = a.list[(round + 1) & 1] + off;
 	uint32_t* out_count = &sc->list_count[(round + 1) % 3][seg];
-	const uint32_t stride = (gridDim.x / kListSegments) * kThreads;
-	for (uint32_t base = (blockIdx.x / kListSegments) * kThreads; base < n; base += stride)
+	const uint32_t lane = threadIdx.x & 63;
+	const uint32_t waves = gridDim.x / kListSegments * (kThreads / 64);
+	const uint32_t ranks = kDeep ? deep_ranks(n, kDeepSegmentWaves < waves ? kDeepSegmentWaves : waves) : 64;
+	for (uint32_t base = (blockIdx.x / kListSegments * (kThreads / 64) + threadIdx.x / 64) * ranks; base < n; base += waves * ranks)
 	{
-		uint32_t idx = base + threadIdx.x;
-		uint4 w = idx < n ? in_list[idx] : make_uint4(0, 0, 0, 0);
-		bool keep = idx < n && round_x<kDeep>(a, w, epoch);
+		const uint32_t idx = base + lane;
+		const bool valid = lane < ranks && idx < n;
+		const uint4 w = valid ? in_list[idx] : make_uint4(0, 0, 0, 0);
+		const bool keep = round_x<kDeep>(a, w, valid, epoch);
 		append_wave(keep, w, out_list, out_count);
 	}
 }
@@ -1128,18 +1220,21 @@ __global__ void __launch_bounds__(kTailThreads) k_round_tail(RoundState a, uint3
 			break;
 		const uint4* in_list = a.list[round & 1];
 		uint4* out_list = a.list[(round + 1) & 1];
-		for (uint32_t base = 0; base < n; base += kTailThreads)
+		const uint32_t lane = threadIdx.x & 63;
+		const uint32_t ranks = deep ? deep_ranks(n, kTailThreads / 64) : 64;
+		for (uint32_t base = threadIdx.x / 64 * ranks; base < n; base += kTailThreads / 64 * ranks)
 		{
-			uint32_t idx = base + threadIdx.x;
+			const uint32_t idx = base + lane;
+			const bool valid = lane < ranks && idx < n;
 			uint4 w = make_uint4(0, 0, 0, 0);
-			if (idx < n)
+			if (valid)
 			{
 				int q = 0;
 				while (idx >= s_pre[q + 1]) // stops below kListSegments: idx < s_pre[kListSegments] = n
 					++q;
 				w = in_list[s_off[q] + (idx - s_pre[q])];
 			}
-			bool keep = idx < n && (deep ? round_x<true>(a, w, epoch) : round_x<false>(a, w, epoch));
+			const bool keep = deep ? round_x<true>(a, w, valid, epoch) : round_x<false>(a, w, valid, epoch);
 			append_wave(keep, w, out_list, &s_out);
 		}
 		__syncthreads();
@@ -1226,8 +1321,9 @@ static RoundState round_state(Mesh& m)
 	return a;
 }
 
-// the per-source candidate lists deep rounds read (they depend on the ranks alone, so they may
-// also be built between the rounds of a window)
+// the per-source candidate lists deep rounds read, of the ranks below cand_count: a test looks at
+// ranks lower than its own, so the window's end is enough (they depend on the ranks alone, so they
+// may also be built between the rounds of a window)
 void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count)
 {
 	size_t n = m.vertex_count;

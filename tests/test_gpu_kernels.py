@@ -115,6 +115,30 @@ def test_candidate_tiles(side):
         assert same_bits(eg, eo), (eg, eo)
 
 
+@pytest.mark.parametrize("mesh", ["grid3", "grid20", "grid110", "grid220", "grid330", "fan8", "fan9", "fan17", "fan200"])
+def test_deep_rounds(mesh):
+    """Rounds that examine moving corners from the first on: lists that leave a wavefront 8, 16, 32 and
+    64 ranks, and sources of more triangles than the lanes that test them."""
+    from meshoptimizer_amd import workloads as W
+    size = int("".join(c for c in mesh if c.isdigit()))
+    if mesh.startswith("grid"):
+        m = W.grid(size, seed=size)
+        ib, v = m.indices, m.vertices
+    else:
+        ib, v = fan(np.random.default_rng(size), size, True, False)
+    M.set_round_policy(-1, 0)
+    try:
+        for den, err, opts in ((10, 1.0, 0), (2, 1e-2, M.SimplifyPermissive)):
+            target = W.target_count(ib.size, 1, den)
+            announce(f"deep {mesh} target 1/{den} err {err}")
+            rg, eg = M.simplify(ib, v, target, err, opts)
+            ro, eo = O.simplify(ib, v, target, err, opts)
+            assert np.array_equal(rg, ro)
+            assert same_bits(eg, eo), (eg, eo)
+    finally:
+        M.set_round_policy()
+
+
 @pytest.mark.parametrize("side,grid", [(2, 2), (17, 3), (27, 3), (27, 26), (64, 4), (64, 20), (300, 6), (300, 150), (516, 40)])
 def test_sloppy_cells(side, grid):
     """Cells of few and of many triangles (both forms of the cell sums) and entry counts around the
