@@ -111,6 +111,7 @@ struct CallScalars
 	uint32_t dual_count;  // boundEdgeCollapses reduction
 	uint32_t kind_counts[6]; // primaries per kind, and all of them
 	uint32_t secondary_count; // vertices that are not their class's primary
+	uint32_t long_lists;  // whether some vertex, or class, has too many corners for the all-pairs order (setup.hip)
 	uint32_t box_done;    // workgroups of the position gather that are done
 	uint32_t unique_count; // sparse remap: number of referenced vertices
 	uint32_t tail_rounds;   // rounds run by the single-workgroup tail of the commit

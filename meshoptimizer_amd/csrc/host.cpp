@@ -427,6 +427,7 @@ struct Plan
 	uint32_t* v_b;
 	uint32_t* v_c;
 	uint32_t* v_d;
+	size_t off_words;
 	uint32_t* raw_off;
 	uint32_t* raw_keys;
 	uint32_t* raw_corners;
@@ -509,8 +510,8 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	m.src_rank = a.take<uint32_t>(cap);
 	m.src_val = a.take<uint32_t>(cap);
 	m.status = a.take<uint8_t>(cap);
-	m.list[0] = a.take<uint4>(cap);
-	m.list[1] = a.take<uint4>(cap);
+	m.list[0] = a.take<uint4>(2 * cap);
+	m.list[1] = m.list[0] + cap;
 	m.stop_tile = a.take<uint32_t>(stop_scan_words(cap));
 
 	// setup-only buffers alias the candidate arrays (not live at the same time)
@@ -521,10 +522,12 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	p.v_b = a.take<uint32_t>(Vp);
 	p.v_c = a.take<uint32_t>(Vp);
 	p.v_d = a.take<uint32_t>(Vp);
-	p.raw_off = a.take<uint32_t>(Vp + 1);
+	// cleared together: the corner counts and the classes' counts of their secondaries' corners
+	p.off_words = (Vp + 1 + 63) & ~size_t(63);
+	p.raw_off = a.take<uint32_t>(2 * p.off_words);
+	p.w_off = p.raw_off + p.off_words;
 	p.raw_keys = reinterpret_cast<uint32_t*>(m.r_v);
 	p.raw_corners = p.raw_keys + cap;
-	p.w_off = a.take<uint32_t>(Vp + 1);
 	p.w_keys = reinterpret_cast<uint32_t*>(m.r_class);
 	p.w_corners = p.w_keys + cap;
 	p.i_alt0 = m.keys_alt;
@@ -682,8 +685,9 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 
 	t_read_backs = 0;
 	// one read-back after the checks and the position remap: the index check, the sparse remap's
-	// vertex count (which its own read-back brings earlier) and the number of secondary vertices
-	launch_call_init(s, m.sc, plan.raw_off, V_alloc + 1);
+	// vertex count (which its own read-back brings earlier), the number of secondary vertices and
+	// whether there are long corner lists
+	launch_call_init(s, m.sc, plan.raw_off, 2 * plan.off_words);
 	launch_load_indices(s, c.indices, m.ib[0], I, V_in, sparse ? nullptr : plan.raw_off, plan.i_alt0, &m.sc->work[2]);
 	auto check_indices = [&]() {
 		if (ctx.sc_host->work[2])
@@ -706,14 +710,17 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 
 	const size_t table_size = pow2_at_least(2 * V + 2);
 	launch_gather_positions(s, m, c.positions, c.position_stride / sizeof(float), sparse_remap, plan.table, table_size);
-	launch_position_remap(s, m, plan.table, table_size);
+	if (sparse)
+		launch_corner_count(s, m, nullptr, plan.raw_off, plan.i_alt0);
+	launch_position_remap(s, m, plan.table, table_size, plan.raw_off, plan.w_off);
 	sync_scalars(ctx, m);
 	check_indices();
 	const size_t secondaries = ctx.sc_host->secondary_count;
+	const uint32_t long_lists = ctx.sc_host->long_lists;
 	launch_wedges(s, m, secondaries, plan.v_flags, plan.v_a, plan.v_b, plan.v_c, plan.v_d);
 
 	const bool permissive = (c.options & kOptPermissive) != 0;
-	launch_corner_lists(s, m, !sparse, permissive, plan.raw_off, plan.i_alt0, plan.raw_keys, plan.raw_corners);
+	launch_corner_lists(s, m, long_lists, permissive, plan.raw_off, plan.i_alt0, plan.raw_keys, plan.raw_corners);
 	launch_classify(s, m, plan.raw_off, secondaries != 0, c.lock, sparse_remap, c.options);
 
 	if (A)
@@ -730,7 +737,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	const uint32_t *w_off = plan.raw_off, *w_corners = plan.raw_corners;
 	if (secondaries)
 	{
-		launch_welded_corner_lists(s, m, plan.w_off, plan.i_alt0, plan.w_keys, plan.w_corners);
+		launch_welded_corner_lists(s, m, long_lists, plan.w_off, plan.i_alt0, plan.w_keys, plan.w_corners);
 		w_off = plan.w_off;
 		w_corners = plan.w_corners;
 	}

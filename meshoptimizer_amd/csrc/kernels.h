@@ -73,7 +73,8 @@ struct Mesh
 	uint2* r_class;          // their source and target classes (remap of r_v)
 	float* r_err;
 	uint8_t* status;
-	uint4* list[2];          // undecided work lists: (rank, source class, target class, 0)
+	uint4* list[2];          // undecided work lists: (rank, source class, target class, 0); one block of
+	                         // 2 * (I + 4) entries, scratch of the set-up
 	uint32_t* stop_tile;     // per-tile sums and records of the stop scan
 
 	uint32_t* temp;          // scan / sort temporaries
@@ -93,16 +94,20 @@ void launch_load_indices(hipStream_t s, const uint32_t* in, uint32_t* out, size_
 // m.praw, the box and the extent (m.sc as launch_call_init leaves it), and an empty hash table
 void launch_gather_positions(hipStream_t s, Mesh& m, const float* positions, size_t stride_floats, const uint32_t* sparse_remap, uint32_t* table,
                              size_t table_size);
-// m.remap, m.pos, sc->secondary_count; wedge rings of one vertex each and empty round minima
-void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size);
+// adds the corners of each vertex (remap null) or class to its count, and says which of them each is
+void launch_corner_count(hipStream_t s, Mesh& m, const uint32_t* remap, uint32_t* counts, uint32_t* slot);
+// m.remap, m.pos, sc->secondary_count; wedge rings of one vertex each and empty round minima.
+// sc->long_lists from the corners per vertex (counts); class_extra: V zero words
+void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size, const uint32_t* counts, uint32_t* class_extra);
 // the wedge rings of the classes with secondaries (their count as read back)
 void launch_wedges(hipStream_t s, Mesh& m, size_t secondaries, uint32_t* flags, uint32_t* scratch_a, uint32_t* scratch_b, uint32_t* scratch_c, uint32_t* scratch_d);
-// each vertex's corners in corner order (offsets: V + 1 words) and its open edges (m.loop[0],
-// m.loopback[0]); `counted`: offsets and slot as launch_load_indices left them, else offsets zero.
+// each vertex's corners in corner order (offsets: V + 1 words, the counts on entry, with the slots
+// that go with them) and its open edges (m.loop[0], m.loopback[0]); long_lists as read back.
 // with_adjacency: (next, prev) per listed corner in m.adj[1], for launch_classify under Permissive
-void launch_corner_lists(hipStream_t s, Mesh& m, bool counted, bool with_adjacency, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners);
+void launch_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, bool with_adjacency, uint32_t* offsets, const uint32_t* slot, uint32_t* placed,
+                         uint32_t* corners);
 // the same lists by class (no open edges); without secondaries they are the vertices' own
-void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners);
+void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners);
 // m.kind, sc->kind_counts and sc->dual_count
 void launch_classify(hipStream_t s, Mesh& m, const uint32_t* raw_off, bool secondaries, const uint8_t* vertex_lock, const uint32_t* sparse_remap,
                      uint32_t options);

@@ -273,6 +273,15 @@ void launch_rescale(hipStream_t s, Mesh& m)
 }
 
 // ------------------------------------------------------------------------------------------
+// Corner lists of more than kAllPairs corners are long.  Up to it a wavefront compares every corner of a
+// list with every other (k_corner_order); beyond it the lists of the mesh are made by sorts, and the
+// open edges of the long ones by a table, linear in the corners.  The two meet at 250-300 corners
+// (calls on a hub of 400 beside 200 triangles 835 us by pairs, 699 sorted; beside 320 thousand 2657 and
+// 2533; of 200 corners 565 and 570, 2483 and 2551); by pairs, the 300 thousand corners that padding
+// with (0,0,0) triangles gives a vertex would take half a minute.
+constexpr uint32_t kAllPairs = 256;
+constexpr uint32_t kLongVertexList = 1, kLongClassList = 2; // of CallScalars::long_lists
+
 // position remap (src/simplifier.cpp:111-240).  remap[i] = lowest index whose xyz compare
 // equal as floats (+0 == -0; NaN equals nothing).  Linear-probing table keyed by the
 // canonical bits; a slot holds one equality class, and atomicMin leaves its lowest index.
@@ -326,9 +335,12 @@ __global__ void k_hash_insert(const float4* pos, size_t n, uint32_t* table, uint
 }
 
 // each vertex's primary, its rescaled position, a wedge ring of its own and no pending ranks; sc
-// counts the secondaries
+// counts the secondaries and says whether any corner list is long (kAllPairs): a vertex's own from
+// its corner count, a class's from its primary's count and the sum over its secondaries, so a class
+// that is not reported has at most 2 * kAllPairs corners
 __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, size_t n, const uint32_t* table, uint32_t mask, uint32_t* remap,
-                                                          uint32_t* wedge, float4* pos, ulonglong2* pend0, ulonglong2* pend1, CallScalars* sc)
+                                                          uint32_t* wedge, float4* pos, ulonglong2* pend0, ulonglong2* pend1, const uint32_t* counts,
+                                                          uint32_t* class_extra, CallScalars* sc)
 {
 	__shared__ uint32_t secondaries;
 	if (threadIdx.x == 0)
@@ -336,8 +348,10 @@ __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, si
 	__syncthreads();
 	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	uint32_t result = (uint32_t)i;
+	uint32_t corners = 0, in_class = 0;
 	if (i < n)
 	{
+		corners = counts[i];
 		const float4 p = praw[i];
 		if (!has_nan(p))
 		{
@@ -361,7 +375,13 @@ __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, si
 		// round minima start as "no entry" (tag of epoch 0, rank all-ones)
 		pend0[i] = make_ulonglong2(~0ull, ~0ull);
 		pend1[i] = make_ulonglong2(~0ull, ~0ull);
+		in_class = corners;
+		if (result != (uint32_t)i && corners)
+			in_class += atomicAdd(&class_extra[result], corners);
 	}
+	const uint64_t long_vertex = __ballot(corners > kAllPairs), long_class = __ballot(in_class > kAllPairs);
+	if (long_class && __lane_id() == 0)
+		atomicOr(&sc->long_lists, (long_vertex ? kLongVertexList : 0u) | kLongClassList);
 	const uint64_t second = __ballot(result != (uint32_t)i);
 	if (second && __lane_id() == 0)
 		atomicAdd(&secondaries, (uint32_t)__popcll(second));
@@ -370,14 +390,15 @@ __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, si
 		atomicAdd(&sc->secondary_count, secondaries);
 }
 
-void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size)
+void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size, const uint32_t* counts, uint32_t* class_extra)
 {
 	size_t n = m.vertex_count;
 	if (!n)
 		return;
 	k_hash_insert<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1));
 	k_hash_lookup<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1), m.remap, m.wedge, m.pos,
-	                                               reinterpret_cast<ulonglong2*>(m.pend[0]), reinterpret_cast<ulonglong2*>(m.pend[1]), m.sc);
+	                                               reinterpret_cast<ulonglong2*>(m.pend[0]), reinterpret_cast<ulonglong2*>(m.pend[1]), counts, class_extra,
+	                                               m.sc);
 }
 
 // wedge rings: for a class r < a_1 < ... < a_m, wedge[r] = a_m, wedge[a_k] = a_{k-1}, wedge[a_1] = r
@@ -434,7 +455,8 @@ void launch_wedges(hipStream_t s, Mesh& m, size_t secondaries, uint32_t* flags, 
 // eight corners by a sorting network in registers, more by the wavefront, every corner's place the
 // number of smaller ones.  (Sorting all corners by vertex with three radix digits took 370 us for
 // the 3.9 M of icosphere L8 and the open edges 140; lists and open edges now take 300 with the index
-// copy and check, 250 of it the count's and the placement's scattered words.)
+// copy and check, 250 of it the count's and the placement's scattered words.)  Meshes with a long list
+// (kAllPairs) do take that sort, and a table of edges answers for the long lists' open ones.
 
 __global__ void k_corner_count(const uint32_t* ib, size_t n, const uint32_t* remap, uint32_t* counts, uint32_t* slot)
 {
@@ -468,6 +490,7 @@ struct CornerArgs
 	uint32_t* openinc;
 	uint2* adj; // (next, prev) per listed corner, or null
 	size_t n;
+	uint32_t longest; // longer lists are sorted already
 };
 
 // the vertices after and before corner j in its triangle
@@ -557,7 +580,13 @@ __global__ void __launch_bounds__(kThreads) k_corner_order(CornerArgs a)
 			a.openinc[v] = open_end(v, self, ins, in_last);
 		}
 	}
-	for (uint64_t left = __ballot(len > kNet); left; left &= left - 1)
+	if (kOpen && len > a.longest)
+	{
+		// a sorted list; k_long_edges finds its open edges, starting from none
+		a.openout[v] = kNone;
+		a.openinc[v] = kNone;
+	}
+	for (uint64_t left = __ballot(len > kNet && len <= a.longest); left; left &= left - 1)
 	{
 		const int from = __builtin_ctzll(left);
 		const uint32_t w = __builtin_amdgcn_readlane(v, from), wb = __builtin_amdgcn_readlane(b, from), we = __builtin_amdgcn_readlane(e, from);
@@ -612,33 +641,181 @@ __global__ void __launch_bounds__(kThreads) k_corner_order(CornerArgs a)
 	}
 }
 
-// offsets (n + 1 words) hold the counts when `counted` (the slots are then given), else zeros
-static void corner_lists(hipStream_t s, Mesh& m, const uint32_t* remap, bool counted, uint32_t* offsets, uint32_t* slot, uint32_t* placed)
+// Lists by sorting, for meshes with a long one: every corner's vertex as the key, its place as the
+// value, both arrays in `corners` and `keys` and the sort's other halves in the candidate lists.
+// The time is linear in the corners (a sweep per byte of the vertex ids).
+
+__global__ void k_corner_keys(const uint32_t* ib, size_t n, const uint32_t* remap, uint32_t* keys)
 {
-	const size_t n = m.index_count;
-	if (!counted && n)
-		k_corner_count<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], n, remap, offsets, slot);
-	scan_exclusive(s, offsets, offsets, m.vertex_count, nullptr, offsets + m.vertex_count, m.temp);
-	if (n)
-		k_corner_place<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], n, remap, offsets, slot, placed);
+	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (j >= n)
+		return;
+	const uint32_t v = ib[j];
+	keys[j] = remap ? remap[v] : v;
 }
 
-void launch_corner_lists(hipStream_t s, Mesh& m, bool counted, bool with_adjacency, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners)
+static void sort_corners(hipStream_t s, Mesh& m, const uint32_t* remap, uint32_t* keys, uint32_t* corners)
+{
+	const size_t n = m.index_count;
+	uint32_t* keys_alt = reinterpret_cast<uint32_t*>(m.list[0]);
+	uint32_t* vals_alt = keys_alt + n;
+	k_corner_keys<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], n, remap, keys);
+	radix_sort_pairs(s, keys, corners, keys_alt, vals_alt, n, nullptr, std::max(1, key_bits(m.vertex_count)), m.temp, true);
+}
+
+// Open edges of the long lists, the rule of k_corner_order: a table holds the directed edges at
+// their vertices, two per corner, and each corner looks for the opposites of its own two.  The
+// candidate lists hold the table: 4 * (I + 4) slots, rounded down to a power of two, for at most I
+// different edges, so that every search ends at an empty slot soon.
+
+struct EdgeTable
+{
+	unsigned long long* slots; // from << 32 | to; ~0: empty
+	uint32_t mask;
+};
+
+__device__ __forceinline__ uint32_t edge_hash(uint64_t edge)
+{
+	edge *= 0x9E3779B97F4A7C15ull;
+	return (uint32_t)(edge >> 32) ^ (uint32_t)edge;
+}
+
+__device__ __forceinline__ void edge_insert(const EdgeTable& t, uint32_t from, uint32_t to)
+{
+	const unsigned long long edge = (unsigned long long)from << 32 | to;
+	uint32_t slot = edge_hash(edge) & t.mask;
+	for (uint32_t probe = 0; probe <= t.mask; ++probe)
+	{
+		// read before it is written: the corners of a padded list all bring the same edge
+		unsigned long long old = __hip_atomic_load(&t.slots[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		if (old == ~0ull)
+			old = atomicCAS(&t.slots[slot], ~0ull, edge);
+		if (old == ~0ull || old == edge)
+			return;
+		slot = (slot + 1) & t.mask;
+	}
+}
+
+__device__ __forceinline__ bool edge_known(const EdgeTable& t, uint32_t from, uint32_t to)
+{
+	const unsigned long long edge = (unsigned long long)from << 32 | to;
+	uint32_t slot = edge_hash(edge) & t.mask;
+	for (uint32_t probe = 0; probe <= t.mask; ++probe)
+	{
+		const unsigned long long at = t.slots[slot];
+		if (at == edge)
+			return true;
+		if (at == ~0ull)
+			return false;
+		slot = (slot + 1) & t.mask;
+	}
+	return false;
+}
+
+// one more open edge of a vertex: the first is named, any other makes it the vertex itself
+__device__ __forceinline__ void open_add(uint32_t* open, uint32_t v, uint32_t end)
+{
+	if (__hip_atomic_load(&open[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == v)
+		return;
+	if (end == v || atomicCAS(&open[v], kNone, end) != kNone)
+		(void)__hip_atomic_exchange(&open[v], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <bool kInsert>
+__global__ void k_long_edges(CornerArgs a, size_t n, EdgeTable t)
+{
+	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (j >= n)
+		return;
+	const uint32_t v = a.ib[j];
+	if (a.off[v + 1] - a.off[v] <= a.longest)
+		return;
+	const uint2 nb = corner_neighbours(a.ib, (uint32_t)j);
+	if (kInsert)
+	{
+		if (nb.x != v)
+			edge_insert(t, v, nb.x);
+		if (nb.y != v)
+			edge_insert(t, nb.y, v);
+		return;
+	}
+	if (nb.x == v || nb.y == v)
+	{
+		open_add(a.openout, v, v);
+		open_add(a.openinc, v, v);
+	}
+	if (nb.x != v && !edge_known(t, nb.x, v))
+		open_add(a.openout, v, nb.x);
+	if (nb.y != v && !edge_known(t, v, nb.y))
+		open_add(a.openinc, v, nb.y);
+}
+
+__global__ void k_list_neighbours(const uint32_t* ib, const uint32_t* corners, size_t n, uint2* adj)
+{
+	size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+	if (p < n)
+		adj[p] = corner_neighbours(ib, corners[p]);
+}
+
+static void long_open_edges(hipStream_t s, Mesh& m, const CornerArgs& a)
+{
+	const size_t n = m.index_count;
+	size_t slots = 1;
+	while (slots * 2 <= 4 * (n + 4) && slots < (size_t)1 << 32)
+		slots *= 2;
+	const EdgeTable t{reinterpret_cast<unsigned long long*>(m.list[0]), (uint32_t)(slots - 1)};
+	fill_u32(s, reinterpret_cast<uint32_t*>(t.slots), kNone, 2 * slots);
+	k_long_edges<true><<<grid_for(n), kThreads, 0, s>>>(a, n, t);
+	k_long_edges<false><<<grid_for(n), kThreads, 0, s>>>(a, n, t);
+	if (a.adj)
+		k_list_neighbours<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], a.corners, n, a.adj);
+}
+
+// the counts (one word per list) become offsets (one more)
+static void corner_offsets(hipStream_t s, Mesh& m, uint32_t* offsets)
+{
+	scan_exclusive(s, offsets, offsets, m.vertex_count, nullptr, offsets + m.vertex_count, m.temp);
+}
+
+void launch_corner_count(hipStream_t s, Mesh& m, const uint32_t* remap, uint32_t* counts, uint32_t* slot)
+{
+	if (m.index_count)
+		k_corner_count<<<grid_for(m.index_count), kThreads, 0, s>>>(m.ib[0], m.index_count, remap, counts, slot);
+}
+
+void launch_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, bool with_adjacency, uint32_t* offsets, const uint32_t* slot, uint32_t* placed,
+                         uint32_t* corners)
 {
 	if (!m.vertex_count)
 		return;
-	corner_lists(s, m, nullptr, counted, offsets, slot, placed);
-	const CornerArgs a{m.ib[0], offsets, placed, corners, m.loop[0], m.loopback[0], with_adjacency ? m.adj[1] : nullptr, m.vertex_count};
+	const bool sorted = (long_lists & kLongVertexList) != 0;
+	corner_offsets(s, m, offsets);
+	if (sorted)
+		sort_corners(s, m, nullptr, placed, corners);
+	else if (m.index_count)
+		k_corner_place<<<grid_for(m.index_count), kThreads, 0, s>>>(m.ib[0], m.index_count, nullptr, offsets, slot, placed);
+	const CornerArgs a{m.ib[0],   offsets, sorted ? corners : placed, corners, m.loop[0], m.loopback[0], with_adjacency ? m.adj[1] : nullptr,
+	                   m.vertex_count, sorted ? kAllPairs : kNone};
 	k_corner_order<true><<<grid_for(m.vertex_count), kThreads, 0, s>>>(a);
+	if (sorted)
+		long_open_edges(s, m, a);
 }
 
-void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners)
+void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners)
 {
 	if (!m.vertex_count)
 		return;
 	fill_u32(s, offsets, 0, (size_t)m.vertex_count + 1);
-	corner_lists(s, m, m.remap, false, offsets, slot, placed);
-	const CornerArgs a{m.ib[0], offsets, placed, corners, nullptr, nullptr, nullptr, m.vertex_count};
+	launch_corner_count(s, m, m.remap, offsets, slot);
+	corner_offsets(s, m, offsets);
+	if (long_lists & kLongClassList)
+	{
+		sort_corners(s, m, m.remap, placed, corners);
+		return;
+	}
+	if (m.index_count)
+		k_corner_place<<<grid_for(m.index_count), kThreads, 0, s>>>(m.ib[0], m.index_count, m.remap, offsets, slot, placed);
+	const CornerArgs a{m.ib[0], offsets, placed, corners, nullptr, nullptr, nullptr, m.vertex_count, kNone};
 	k_corner_order<false><<<grid_for(m.vertex_count), kThreads, 0, s>>>(a);
 }
 
