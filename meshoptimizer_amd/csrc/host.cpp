@@ -50,7 +50,8 @@ void fatal_hip(hipError_t err, const char* expr, const char* file, int line)
 }
 
 // ------------------------------------------------------------------------------------------
-// arena: bump allocation of 256-byte aligned sub-buffers; a dry run measures the footprint
+// arena: bump allocation of sub-buffers aligned to the 128 bytes of a cache line; a dry run measures
+// the footprint
 
 struct Arena
 {
@@ -61,7 +62,7 @@ struct Arena
 	template <typename T>
 	T* take(size_t count)
 	{
-		size_t off = (used + 255) & ~size_t(255);
+		size_t off = (used + 127) & ~size_t(127);
 		used = off + count * sizeof(T) + 16;
 		return base ? reinterpret_cast<T*>(base + off) : nullptr;
 	}
@@ -434,8 +435,7 @@ struct Plan
 	uint32_t* w_off;
 	uint32_t* w_keys;
 	uint32_t* w_corners;
-	uint32_t* i_alt0;
-	uint32_t* i_alt1;
+	uint32_t* slot; // a corner's place in its list
 	uint32_t* comp; // Prune: component per vertex
 	float* cerr;    // Prune: error per component
 	SolveBuffers solve; // meshopt_simplifyWithUpdate only
@@ -449,6 +449,9 @@ static size_t pow2_at_least(size_t n)
 	return p;
 }
 
+// Arrays of the set-up lie in those that only the passes use, and the other way round, and so do a
+// pass's early arrays in its late ones; each alias says what makes the two lifetimes disjoint.  The
+// size is what a server admits a request by (request_device_bytes).
 static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, bool sparse, bool prune, bool solve)
 {
 	Mesh& m = p.m;
@@ -491,37 +494,34 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 		m.adj[k] = a.take<uint2>(I + 4);
 	}
 	m.new_class = a.take<uint32_t>(Vp);
-	m.adj_off = a.take<uint32_t>(Vp + 1);
+	m.adj_off = m.src_off; // between the passes and after them; the source lists are a pass's
 
-	m.tile_sums = a.take<uint2>(2 * tile_sum_words(std::max(V, T)));
+	m.tri_sums = a.take<uint2>(compaction_tiles(T));
+	m.vertex_sums = a.take<uint2>(compaction_tiles(V));
 	m.tri_cnt = prune ? a.take<uint32_t>(T) : nullptr;
 	m.tri_off = prune ? a.take<uint32_t>(T) : nullptr;
 
 	m.c_v = a.take<uint2>(cap);
 	m.c_err = a.take<float>(cap);
-	m.rank_counts = a.take<uint32_t>(rank_sort_words(cap));
-	m.keys = a.take<uint32_t>(cap);
-	m.vals = a.take<uint32_t>(cap);
-	m.keys_alt = a.take<uint32_t>(cap);
-	m.vals_alt = a.take<uint32_t>(cap);
 	m.r_v = a.take<uint2>(cap);
 	m.r_class = a.take<uint2>(cap);
 	m.r_err = a.take<float>(cap);
 	m.src_rank = a.take<uint32_t>(cap);
 	m.src_val = a.take<uint32_t>(cap);
 	m.status = a.take<uint8_t>(cap);
-	m.list[0] = a.take<uint4>(2 * cap);
+	m.list[0] = a.take<uint4>(std::max(2 * cap, rank_sort_words(cap) / 4));
 	m.list[1] = m.list[0] + cap;
+	m.rank_counts = reinterpret_cast<uint32_t*>(m.list[0]); // read for the last time before the window opens
 	m.stop_tile = a.take<uint32_t>(stop_scan_words(cap));
 
-	// setup-only buffers alias the candidate arrays (not live at the same time)
+	// of the set-up only, in arrays that the first pass writes before it reads them
 	p.table_size = pow2_at_least(2 * V + 2);
 	p.table = a.take<uint32_t>(p.table_size);
-	p.v_flags = a.take<uint32_t>(Vp);
-	p.v_a = a.take<uint32_t>(Vp);
-	p.v_b = a.take<uint32_t>(Vp);
-	p.v_c = a.take<uint32_t>(Vp);
-	p.v_d = a.take<uint32_t>(Vp);
+	p.v_flags = m.new_class;
+	p.v_a = reinterpret_cast<uint32_t*>(m.adj_range[1]);
+	p.v_b = p.v_a + Vp;
+	p.v_c = m.lock_rank;
+	p.v_d = m.cremap;
 	// cleared together: the corner counts and the classes' counts of their secondaries' corners
 	p.off_words = (Vp + 1 + 63) & ~size_t(63);
 	p.raw_off = a.take<uint32_t>(2 * p.off_words);
@@ -530,8 +530,7 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	p.raw_corners = p.raw_keys + cap;
 	p.w_keys = reinterpret_cast<uint32_t*>(m.r_class);
 	p.w_corners = p.w_keys + cap;
-	p.i_alt0 = m.keys_alt;
-	p.i_alt1 = m.vals_alt;
+	p.slot = m.src_rank;
 	p.comp = prune ? a.take<uint32_t>(Vp) : nullptr;
 	p.cerr = prune ? a.take<float>(Vp) : nullptr;
 	p.solve.update = solve ? a.take<uint8_t>(Vp + 8) : nullptr;
@@ -647,7 +646,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	Arena dry;
 	Plan plan;
 	carve(dry, plan, V_in, V_alloc, I, A, sparse, prune, solve);
-	ctx.ensure_arena(dry.used + 4096);
+	ctx.ensure_arena(dry.used);
 	Arena arena;
 	arena.base = ctx.arena;
 	arena.size = ctx.arena_size;
@@ -681,14 +680,13 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	m.ib_cur = 0;
 	m.loop_cur = 0;
 	m.adj_cur = 0;
-	m.epoch = 0;
 
 	t_read_backs = 0;
 	// one read-back after the checks and the position remap: the index check, the sparse remap's
 	// vertex count (which its own read-back brings earlier), the number of secondary vertices and
 	// whether there are long corner lists
 	launch_call_init(s, m.sc, plan.raw_off, 2 * plan.off_words);
-	launch_load_indices(s, c.indices, m.ib[0], I, V_in, sparse ? nullptr : plan.raw_off, plan.i_alt0, &m.sc->work[2]);
+	launch_load_indices(s, c.indices, m.ib[0], I, V_in, sparse ? nullptr : plan.raw_off, plan.slot, &m.sc->work[2]);
 	auto check_indices = [&]() {
 		if (ctx.sc_host->work[2])
 			throw std::invalid_argument("index buffer references a vertex >= vertex_count");
@@ -711,7 +709,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	const size_t table_size = pow2_at_least(2 * V + 2);
 	launch_gather_positions(s, m, c.positions, c.position_stride / sizeof(float), sparse_remap, plan.table, table_size);
 	if (sparse)
-		launch_corner_count(s, m, nullptr, plan.raw_off, plan.i_alt0);
+		launch_corner_count(s, m, nullptr, plan.raw_off, plan.slot);
 	launch_position_remap(s, m, plan.table, table_size, plan.raw_off, plan.w_off);
 	sync_scalars(ctx, m);
 	check_indices();
@@ -720,7 +718,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	launch_wedges(s, m, secondaries, plan.v_flags, plan.v_a, plan.v_b, plan.v_c, plan.v_d);
 
 	const bool permissive = (c.options & kOptPermissive) != 0;
-	launch_corner_lists(s, m, long_lists, permissive, plan.raw_off, plan.i_alt0, plan.raw_keys, plan.raw_corners);
+	launch_corner_lists(s, m, long_lists, permissive, plan.raw_off, plan.slot, plan.raw_keys, plan.raw_corners);
 	launch_classify(s, m, plan.raw_off, secondaries != 0, c.lock, sparse_remap, c.options);
 
 	if (A)
@@ -737,7 +735,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	const uint32_t *w_off = plan.raw_off, *w_corners = plan.raw_corners;
 	if (secondaries)
 	{
-		launch_welded_corner_lists(s, m, long_lists, plan.w_off, plan.i_alt0, plan.w_keys, plan.w_corners);
+		launch_welded_corner_lists(s, m, long_lists, plan.w_off, plan.slot, plan.w_keys, plan.w_corners);
 		w_off = plan.w_off;
 		w_corners = plan.w_corners;
 	}
@@ -2790,8 +2788,7 @@ static size_t request_device_bytes(const meshopt_hip_request& r)
 	Plan plan;
 	carve(dry, plan, r.vertex_count, sparse ? std::min(r.vertex_count, r.index_count) : r.vertex_count, r.index_count, A, sparse,
 	      (r.options & kOptPrune) != 0, false);
-	size_t arena = dry.used + 4096;
-	arena += arena / 4;
+	const size_t arena = dry.used + dry.used / 4;
 	const HostStaging h = plan_staging(r.index_count, r.vertex_positions, r.vertex_count, r.vertex_positions_stride, r.vertex_attributes,
 	                                   r.vertex_attributes_stride, r.attribute_count, r.vertex_lock);
 	return arena + h.total + h.total / 4 + 256;

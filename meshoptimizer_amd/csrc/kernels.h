@@ -46,35 +46,31 @@ struct Mesh
 	uint32_t* lock_rank;     // rank of the commit that locked a class (collapse_locked)
 	uint64_t* pend[2];       // per-class round minima of the commit rounds, two per class (16 B):
 	                         // over ranks whose source is the class, and whose target is
-	uint32_t epoch;
 
 	uint2* adj_range[2];     // V: a class's entries (begin, end) of adj, of the current pass and the next
 	uint2* adj[2];           // I: (next, prev) classes per corner
 	int adj_cur;
 	uint32_t* new_class;     // V: the class a primary's class belongs to after the pass
-	uint32_t* adj_off;       // V + 1: offsets of an adjacency built from scratch
+	uint32_t* adj_off;       // V + 1: offsets of an adjacency built from scratch (the space of src_off)
 
 	uint32_t* ib[2];         // index buffer ping-pong
 	int ib_cur;
 
-	uint2* tile_sums;        // per-tile sums of the blocked compactions
+	uint2* tri_sums;         // per-tile sums of the blocked compactions: triangles, vertices
+	uint2* vertex_sums;
 	uint32_t* tri_cnt;       // per-triangle flags and offsets (Prune only)
 	uint32_t* tri_off;
 
 	uint2* c_v;              // candidates in pick order
 	float* c_err;
-	uint32_t* rank_counts;   // candidates per key value and tile (rank_sort_words)
-	uint32_t* keys;          // sort buffers of the set-up and the prune; rank slots of the source lists
-	uint32_t* vals;
-	uint32_t* keys_alt;
-	uint32_t* vals_alt;
+	uint32_t* rank_counts;   // candidates per key value and tile (rank_sort_words), in the space of the lists
 
 	uint2* r_v;              // candidates in rank order
 	uint2* r_class;          // their source and target classes (remap of r_v)
 	float* r_err;
 	uint8_t* status;
 	uint4* list[2];          // undecided work lists: (rank, source class, target class, 0); one block of
-	                         // 2 * (I + 4) entries, scratch of the set-up
+	                         // 2 * (I + 4) entries or more, scratch of the set-up
 	uint32_t* stop_tile;     // per-tile sums and records of the stop scan
 
 	uint32_t* temp;          // scan / sort temporaries
@@ -126,7 +122,7 @@ void launch_pick(hipStream_t s, Mesh& m, size_t tri_count, const uint32_t* live 
 // and as the ranges the passes read
 void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count);
 void launch_adjacency_ranges(hipStream_t s, Mesh& m, size_t tri_count);
-size_t tile_sum_words(size_t n); // entries of one m.tile_sums array (there are two)
+size_t compaction_tiles(size_t n); // tiles of a blocked compaction of up to n items
 // errors and rank order of the candidates, the commit state of the pass, and the work-list counts of
 // the ranks below `window`
 void launch_rank_sort(hipStream_t s, Mesh& m, size_t cand_count, size_t window);

@@ -65,16 +65,16 @@ __global__ void k_adj_ranges(const uint32_t* off, size_t n, uint2* range)
 		range[v] = make_uint2(off[v], off[v + 1]);
 }
 
-// the corner slots go to m.keys, free between the passes and after them
+// the corner slots go to the space of the source lists, which a pass makes for itself
 void launch_adjacency(hipStream_t s, Mesh& m, size_t tri_count)
 {
 	size_t n = m.vertex_count;
 	fill_u32(s, m.adj_off, 0, n + 1);
 	if (tri_count)
-		k_adj_count<<<grid_for(tri_count * 3), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count * 3, m.remap, m.adj_off, m.keys);
+		k_adj_count<<<grid_for(tri_count * 3), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count * 3, m.remap, m.adj_off, m.src_rank);
 	scan_exclusive(s, m.adj_off, m.adj_off, n, nullptr, m.adj_off + n, m.temp);
 	if (tri_count)
-		k_adj_fill<<<grid_for(tri_count), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, m.remap, m.adj_off, m.keys, m.adj[m.adj_cur]);
+		k_adj_fill<<<grid_for(tri_count), kThreads, 0, s>>>(m.ib[m.ib_cur], tri_count, m.remap, m.adj_off, m.src_rank, m.adj[m.adj_cur]);
 }
 
 void launch_adjacency_ranges(hipStream_t s, Mesh& m, size_t tri_count)
@@ -96,9 +96,9 @@ static inline uint32_t tile_items(size_t n)
 	return div_up(n ? n : 1, (size_t)kThreads * kMaxTiles);
 }
 
-size_t tile_sum_words(size_t)
+size_t compaction_tiles(size_t n)
 {
-	return kMaxTiles + 1;
+	return std::min((size_t)div_up(n ? n : 1, kThreads), kMaxTiles);
 }
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
@@ -358,7 +358,7 @@ static TriArgs tri_args(Mesh& m, size_t tri_count, const uint32_t* live, int loo
 	a.kind = m.kind;
 	a.loop = m.loop[loop_set];
 	a.loopback = m.loopback[loop_set];
-	a.sums = m.tile_sums;
+	a.sums = m.tri_sums;
 	a.c_v = m.c_v;
 	a.c_err = m.c_err;
 	a.sc = m.sc;
@@ -1328,12 +1328,14 @@ void launch_source_lists(hipStream_t s, Mesh& m, size_t cand_count)
 {
 	size_t n = m.vertex_count;
 	fill_u32(s, m.src_off, 0, n + 1);
-	// the rank slots go to m.keys, free once the ranked copies are gathered
+	// the rank slots go to the candidates' errors: the ranked copies are made, the next pass's
+	// candidates are not
+	uint32_t* slot = reinterpret_cast<uint32_t*>(m.c_err);
 	if (cand_count)
-		k_src_count<<<grid_for(cand_count), kThreads, 0, s>>>(m.r_class, cand_count, m.src_off, m.keys);
+		k_src_count<<<grid_for(cand_count), kThreads, 0, s>>>(m.r_class, cand_count, m.src_off, slot);
 	scan_exclusive(s, m.src_off, m.src_off, n, nullptr, m.src_off + n, m.temp);
 	if (cand_count)
-		k_src_fill<<<grid_for(cand_count), kThreads, 0, s>>>(round_state(m), m.r_class, cand_count, m.keys, m.src_rank, m.src_val);
+		k_src_fill<<<grid_for(cand_count), kThreads, 0, s>>>(round_state(m), m.r_class, cand_count, slot, m.src_rank, m.src_val);
 }
 
 // Ranks [lo, hi) become a work list, in segments by source class, and publish: the first round of a
@@ -1799,8 +1801,9 @@ void launch_stop_scan(hipStream_t s, Mesh& m, size_t window, size_t cand_count, 
 
 size_t stop_scan_words(size_t cand_count)
 {
-	// at most 1024 tiles of four ranks a thread, or tiles of sixteen
-	return (kStopWords + kRecWords) * ((size_t)div_up(cand_count, kThreads * 16) + 1026);
+	// up to 1024 tiles of four ranks a thread, then tiles of sixteen
+	const size_t short_tiles = std::min((size_t)div_up(cand_count, kThreads * 4), (size_t)1024);
+	return (kStopWords + kRecWords) * std::max(short_tiles, (size_t)div_up(cand_count, kThreads * 16));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1917,7 +1920,6 @@ struct ApplyArgs
 	uint2* sums;
 	CallScalars* sc;
 	int attr_count;
-	uint32_t ranks;
 	uint32_t rank_blocks;
 	uint32_t vertices;
 	uint32_t items;
@@ -2134,10 +2136,9 @@ void launch_apply(hipStream_t s, Mesh& m, size_t window, size_t tri_count)
 	a.range_out = m.adj_range[m.adj_cur ^ 1];
 	a.adj_out = m.adj[m.adj_cur ^ 1];
 	a.new_class = m.new_class;
-	a.sums = m.tile_sums + tile_sum_words(0);
+	a.sums = m.vertex_sums;
 	a.sc = m.sc;
 	a.attr_count = (int)m.attr_count;
-	a.ranks = (uint32_t)window;
 	a.rank_blocks = grid_for(window);
 	a.vertices = m.vertex_count;
 	a.items = tile_items(m.vertex_count);

@@ -60,6 +60,25 @@ def submit(srv, r):
                       lock=r.get("lock"))
 
 
+@pytest.mark.parametrize("V,T,A,opts,budget", [
+    (4, 2, 0, 0, 25696), (4, 2, 3, 8, 27296), (100, 200, 0, 0, 130976), (1000, 20, 0, 0, 280736), (1000, 20, 0, 2, 69216),
+    (1000, 20, 3, 8, 441376), (1000, 2000, 0, 0, 1136416), (1000, 2000, 3, 2, 1382176), (11000, 22000, 0, 8, 12508256),
+    (100000, 3000, 0, 0, 26785696), (100000, 3000, 0, 2, 5656096), (30000, 58000, 3, 0, 37294496), (120000, 174900, 0, 0, 106311456),
+    (300000, 620000, 0, 8, 350150496), (400000, 800000, 0, 0, 449525216), (1500000, 100, 3, 8, 623377696)])
+def test_budgets_that_were_enough(V, T, A, opts, budget):
+    """Requests of many vertices, many triangles, attributes, Sparse and Prune, each with the budget that
+    a single adjacency and separate set-up arrays needed: they are still admitted, and run."""
+    rng = np.random.default_rng(V + T)
+    ib = rng.integers(0, V, 3 * T).astype(np.uint32)
+    v = rng.random((V, 3 + A)).astype(np.float32)
+    announce(f"budget V={V} T={T} A={A} opts={opts}")
+    with M.Server(budget_bytes=budget, slots=1) as srv:
+        ri, _, info = srv.wait(srv.submit(ib, v, ib.size, 1e-2, opts, attributes=v[:, 3:] if A else None,
+                                          weights=np.ones(A, np.float32) if A else None))
+    assert info["device_bytes"] <= budget
+    assert np.array_equal(ri, ib)
+
+
 def test_mix_equals_alone_and_oracle():
     reqs = mixed_requests()
     announce(f"serving mix of {len(reqs)} requests on 4 slots")
