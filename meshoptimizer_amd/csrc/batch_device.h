@@ -136,10 +136,12 @@ inline PatchLayout patch_layout(uint32_t vmax, uint32_t imax, uint32_t cmax)
 	L.lock = take(vmax);
 	L.off = take((vmax + 2) * 2);
 	L.adj = take(imax * 4);
-	// the sort's ping-pong half and digit counts (64 offsets + 64 counts per wavefront)
-	// (commit keeps a 64-bit lane mask per vertex there; the sort needs as much in nearly every layout)
-	const uint32_t sort_bytes = align16(cmax * 2) + (1 + kBatchWaves) * 64 * 4;
-	L.sortbuf = take(sort_bytes > vmax * 8 ? sort_bytes : vmax * 8);
+	// the sort's ping-pong half and its digit counts (64 per wavefront), and in the same space the
+	// commit's lane masks, a 64-bit word per vertex, for meshes whose vertices are no more than the
+	// words (layout_has_masks; space of their own would take up to 100 indices from the classes of
+	// large meshes).  The 64 words more than the sort needs are the masks'; the shape table's caps rest
+	// on the size
+	L.sortbuf = take(align16(cmax * 2) + (1 + kBatchWaves) * 64 * 4);
 	// one region for uses whose lifetimes do not overlap: the candidate arrays (pick to commit)
 	// and the scratch of setup (position hash, wedge maxima), of build_adjacency (cursor, corner
 	// ids; the ordered welded corners live on through the quadrics) and of the edge-loop update
@@ -158,6 +160,12 @@ inline PatchLayout patch_layout(uint32_t vmax, uint32_t imax, uint32_t cmax)
 	L.cerr = L.order + align16(cmax * 2);
 	L.total = o;
 	return L;
+}
+
+// whether the commit has a mask word for every vertex that the layout holds
+inline bool layout_has_masks(const PatchLayout& L)
+{
+	return L.vmax <= (L.region - L.sortbuf) / 8;
 }
 
 struct PatchSmem
@@ -436,7 +444,10 @@ __device__ __forceinline__ uint32_t lds_next_wedge_above(const PatchSmem& s, uin
 // The whole simplify of one mesh by the calling workgroup; every return is workgroup-uniform.
 // sh[0..4] and shf[] are scratch words of this function.  kAttr: the batch has attributes
 // (a.attribute_count > 0), which only that build of the function reads.
-template <bool kAttr = false>
+// kMasks: the layout has a mask word for every vertex; otherwise the commit of a mesh that has more
+// vertices than words compares its lanes with each other.  Two builds, since the test alone costs the
+// first 1% (4096 patches 418 us, 422 with it; 1156 groups of 1810 triangles 1343 and 1360)
+template <bool kAttr, bool kMasks>
 __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLayout& L, uint32_t patch, uint8_t* smem, uint32_t* part,
                                                uint32_t* sh, uint64_t* box, float* shf)
 {
@@ -1227,12 +1238,16 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 		// Bound by the latency of one wavefront's LDS and ballot chains; a chunk takes 4-8 rounds
 		// where one rank at a time took 15-20 decisions.  4096 patches of 64-512 triangles:
 		// 541 to 466 us a call; 1156 groups of 1810 triangles: 2.58 to 1.43 ms.
-		uint64_t* const tab = (uint64_t*)s.sortbuf; // the sort's half: one word per vertex, zero between chunks
+		//
+		// Without a word for every vertex (kMasks), the lanes are compared with each other instead.
+		uint64_t* const tab = (uint64_t*)s.sortbuf; // zero between chunks
+		const bool masks = kMasks || V <= (L.region - L.sortbuf) / 8;
 		for (uint32_t v = tid; v < V; v += kBatchThreads)
 		{
 			s.cremap[v] = (uint16_t)v;
 			s.lock[v] = 0;
-			tab[v] = 0;
+			if (masks)
+				tab[v] = 0;
 		}
 		__syncthreads();
 		if (tid < 64)
@@ -1277,35 +1292,52 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 				// flip: the lower lanes whose source the flip test reads; share: those that share an
 				// endpoint class
 				uint64_t flip = 0, share = 0;
-				if (open)
-					atomicOr((unsigned long long*)&tab[r0], (unsigned long long)bit);
-				wave_fence();
-				if (open)
+				if (!masks)
 				{
+					for (uint64_t left = __ballot(open); left; left &= left - 1)
+					{
+						const int j = __builtin_ctzll(left);
+						const uint32_t j0 = __builtin_amdgcn_readlane(r0, j), j1 = __builtin_amdgcn_readlane(r1, j);
+						share |= r0 == j0 || r0 == j1 || r1 == j0 || r1 == j1 ? 1ull << j : 0;
+						bool reads = false;
+						for (uint32_t p = ab; p < ae; ++p)
+							reads |= (s.adj[p] & 0xffffu) == j0 || s.adj[p] >> 16 == j0;
+						flip |= reads ? 1ull << j : 0;
+					}
+					share &= below;
+				}
+				else
+				{
+					if (open)
+						atomicOr((unsigned long long*)&tab[r0], (unsigned long long)bit);
+					wave_fence();
+					if (open)
+					{
 #pragma unroll
-					for (int q = 0; q < kNearSlots; ++q)
-						if (ab + q < ae)
+						for (int q = 0; q < kNearSlots; ++q)
+							if (ab + q < ae)
+							{
+								const uint32_t ad = s.adj[ab + q];
+								flip |= tab[ad & 0xffffu] | tab[ad >> 16];
+							}
+						for (uint32_t p = ab + kNearSlots; p < ae; ++p)
 						{
-							const uint32_t ad = s.adj[ab + q];
+							const uint32_t ad = s.adj[p];
 							flip |= tab[ad & 0xffffu] | tab[ad >> 16];
 						}
-					for (uint32_t p = ab + kNearSlots; p < ae; ++p)
-					{
-						const uint32_t ad = s.adj[p];
-						flip |= tab[ad & 0xffffu] | tab[ad >> 16];
 					}
-				}
-				wave_fence();
-				if (open)
-					atomicOr((unsigned long long*)&tab[r1], (unsigned long long)bit);
-				wave_fence();
-				if (open)
-					share = (tab[r0] | tab[r1]) & below;
-				wave_fence();
-				if (open)
-				{
-					tab[r0] = 0;
-					tab[r1] = 0;
+					wave_fence();
+					if (open)
+						atomicOr((unsigned long long*)&tab[r1], (unsigned long long)bit);
+					wave_fence();
+					if (open)
+						share = (tab[r0] | tab[r1]) & below;
+					wave_fence();
+					if (open)
+					{
+						tab[r0] = 0;
+						tab[r1] = 0;
+					}
 				}
 				const uint64_t deps = (flip & below) | share;
 				const uint32_t ends = r0 | (r1 << 16), span = ab | (ae << 16);
@@ -1628,7 +1660,7 @@ __device__ __forceinline__ void simplify_patch(const BatchArgs& a, const PatchLa
 // read back is made wave-uniform (every thread reads the same word after the barrier, so the
 // first lane's value is every lane's): the loop exit and every barrier loop inside simplify_patch
 // then sit in uniform control flow, as in the one-mesh-per-workgroup form.
-template <bool kAttr = false>
+template <bool kAttr, bool kMasks>
 __device__ __forceinline__ void simplify_from_cursor(const BatchArgs& a, const PatchLayout& L, const uint32_t* ids, uint32_t n, uint32_t* cursor,
                                                      uint8_t* smem, uint32_t* part, uint32_t* sh, uint64_t* box, float* shf, uint32_t* next)
 {
@@ -1640,7 +1672,7 @@ __device__ __forceinline__ void simplify_from_cursor(const BatchArgs& a, const P
 		const uint32_t i = __builtin_amdgcn_readfirstlane(*next);
 		if (i >= n)
 			break;
-		simplify_patch<kAttr>(a, L, ids[i], smem, part, sh, box, shf);
+		simplify_patch<kAttr, kMasks>(a, L, ids[i], smem, part, sh, box, shf);
 		__syncthreads();
 	}
 }

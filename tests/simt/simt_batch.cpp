@@ -141,21 +141,21 @@ struct Task
 
 static Task g_tasks[kMaxGroups];
 
+template <bool kAttr, bool kMasks>
+static void run_task(const Task& t)
+{
+	if (t.ids)
+		mhip::simplify_from_cursor<kAttr, kMasks>(*t.a, *t.L, t.ids, t.n, t.cursor, t.smem, t.part, t.sh, t.box, t.shf, t.next);
+	else
+		mhip::simplify_patch<kAttr, kMasks>(*t.a, *t.L, t.patch, t.smem, t.part, t.sh, t.box, t.shf);
+}
+
 static void fiber_main()
 {
 	const Task& t = g_tasks[g.id];
-	const bool attr = t.a->attribute_count != 0;
-	if (t.ids)
-	{
-		if (attr)
-			mhip::simplify_from_cursor<true>(*t.a, *t.L, t.ids, t.n, t.cursor, t.smem, t.part, t.sh, t.box, t.shf, t.next);
-		else
-			mhip::simplify_from_cursor<false>(*t.a, *t.L, t.ids, t.n, t.cursor, t.smem, t.part, t.sh, t.box, t.shf, t.next);
-	}
-	else if (attr)
-		mhip::simplify_patch<true>(*t.a, *t.L, t.patch, t.smem, t.part, t.sh, t.box, t.shf);
-	else
-		mhip::simplify_patch<false>(*t.a, *t.L, t.patch, t.smem, t.part, t.sh, t.box, t.shf);
+	// the build that the library launches for the layout
+	const bool attr = t.a->attribute_count != 0, masks = mhip::layout_has_masks(*t.L);
+	(attr ? masks ? run_task<true, true> : run_task<true, false> : masks ? run_task<false, true> : run_task<false, false>)(t);
 	g.fibers[g.current].state = kDone;
 	swapcontext(&g.fibers[g.current].ctx, &g.scheduler);
 }

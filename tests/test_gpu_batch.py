@@ -310,6 +310,30 @@ def test_batch_shapes(shape):
         check_batch_device(meshes, targets, 1e-2, M.SimplifyLockBorder)
 
 
+@pytest.mark.parametrize("threads,cap", [(128, (2016, 6048)), (256, (2016, 6048)), (512, (1984, 5952)), (1024, (1984, 5952))])
+def test_last_class_holds(threads, cap):
+    """The largest meshes of the last class at every width, of few vertices and of as many as it takes
+    (more than the commit has mask words in the narrow ones)."""
+    with launch_shape([2, 2, 2, 1], [128, 128, 128, threads], [0, 0, 0, 1]) as shape:
+        assert (shape["vertex_caps"][3], shape["index_caps"][3]) == cap
+        meshes, targets = [], []
+        for n, own in ((32, 0), (31, 700), (32, cap[0] // 3), (2, 0)):
+            m = W.grid(n, seed=n + threads)
+            tri = m.indices.reshape(-1, 3)[:cap[1] // 3].copy()
+            v = m.vertices[:, :3]
+            # the last triangles get vertices of their own, as far as the vertex cap goes
+            k = min(own, (cap[0] - v.shape[0]) // 3)
+            if k:
+                extra = v[tri[-k:].reshape(-1)]
+                tri[-k:] = np.arange(v.shape[0], v.shape[0] + 3 * k).reshape(-1, 3)
+                v = np.concatenate([v, extra])
+            meshes.append((tri.reshape(-1).astype(np.uint32), np.ascontiguousarray(v)))
+            targets.append(len(tri) // 3 * 3)
+        announce(f"last class of {threads} threads: {[(ib.size, v.shape[0]) for ib, v in meshes]}")
+        for opts in (0, M.SimplifyPermissive):
+            check_batch_device(meshes, targets, 5e-2, opts)
+
+
 def check_batch_attributes(meshes, attrs, weights, targets, err, opts, locks=None, entry="host"):
     """The batched entries with attributes against the oracle's simplifyWithAttributes per mesh."""
     if entry == "host":

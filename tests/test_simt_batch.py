@@ -161,6 +161,48 @@ def test_candidate_overflow_runs_again(simt):
     assert simt.simt_retries() >= 1
 
 
+@pytest.mark.parametrize("width,vmax,imax,share", [("simt_narrow", 2016, 6048, 1), ("simt", 2016, 6048, 1), ("simt_mid", 1984, 5952, 1),
+                                                   ("simt_wide", 1984, 5952, 1), ("simt", 992, 3936, 2), ("simt_mid", 992, 3936, 2),
+                                                   ("simt", 672, 2592, 3), ("simt", 384, 1536, 5), ("simt", 320, 1248, 6),
+                                                   ("simt_narrow", 288, 1056, 7), ("simt_narrow", 192, 672, 10)])
+def test_layout_sizes(request, width, vmax, imax, share):
+    """The largest meshes that each width takes at 1 to 10 workgroups per CU (160 KB in granules of 512
+    bytes, 256 of them static): the commit's lane masks take no LDS of their own, which would cost
+    these classes up to 100 indices.  One workgroup per CU holds the full candidate bound."""
+    lib = request.getfixturevalue(width)
+    cmax = imax + 4 if share == 1 else imax * 5 // 8 + 8
+    assert lib.simt_layout_bytes(vmax, imax, cmax) <= 160 * 1024 // share // 512 * 512 - 256
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_shared_mask_words(simt, simt_narrow, seed):
+    """Meshes of more vertices than the commit has mask words, so that two vertices share one: grids cut
+    along every column, loose strips and soups."""
+    rng = np.random.default_rng(900 + seed)
+    meshes, targets = [], []
+    for k in range(6):
+        if k % 3 == 2:
+            ib, v = random_soup(rng, nv=int(rng.integers(500, 800)), ntri=int(rng.integers(420, 500)))
+        else:
+            n = int(rng.integers(18, 26))
+            ib, v = random_grid(rng, n=n, seams=n - 2 if k % 3 else n // 2)
+        v = np.ascontiguousarray(v[:, :3])
+        if k % 3 == 0:
+            # every other triangle with vertices of its own
+            tri = ib.reshape(-1, 3).copy()
+            own = np.arange(0, len(tri), 2)
+            extra = v[tri[own].reshape(-1)]
+            tri[own] = np.arange(v.shape[0], v.shape[0] + extra.shape[0]).reshape(-1, 3)
+            ib, v = tri.reshape(-1).astype(np.uint32), np.ascontiguousarray(np.concatenate([v, extra]))
+        imax = (ib.size + 95) // 96 * 96  # the layout that the mesh has to itself, at 256 threads
+        assert v.shape[0] > (((imax * 5 // 8 + 8) * 2 + 15) // 16 * 16 + 5 * 256) // 8
+        meshes.append((ib, v))
+        targets.append((ib.size // 3 * int(rng.integers(0, 3)) // 4) * 3)
+    for lib in (simt, simt_narrow):
+        for k in range(len(meshes)):
+            check(lib, meshes[k:k + 1], targets[k:k + 1], (1e-1, 1.0)[seed % 2], (0, M.SimplifyPermissive, M.SimplifyLockBorder)[seed % 3], seed=seed + 1)
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_vertex_locks(simt, seed):
     """Per-vertex Lock, Protect and Priority bits (src/simplifier.cpp:498-530, 1095-1098) in the
