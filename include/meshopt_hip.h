@@ -159,6 +159,12 @@ int meshopt_hip_last_call_stats(meshopt_hip_call_stats* call, meshopt_hip_pass_s
  * calls in the process; returns 0, or -1 with meshopt_hip_last_error set. */
 int meshopt_hip_set_round_policy(int deep_heads, int deep_from_head);
 
+/* Nonzero: the plain path builds its adjacency from scratch after every pass, as it does after a pass
+ * that leaves a class's wedges in different classes, instead of carrying it over (no counterpart in
+ * the reference; results never depend on it).  For tests; applies to the calling thread's later
+ * calls; returns 0. */
+int meshopt_hip_set_adjacency_rebuild(int enable);
+
 /* Forgets the head-round counts the library learned per window size (no counterpart in the
  * reference; results never depend on them): later calls start as the process's first did, with
  * a read-back of the list length after each batch of head rounds of a window size not yet seen.

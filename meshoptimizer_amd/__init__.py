@@ -74,7 +74,7 @@ EXPORTED_SYMBOLS = (
     "meshopt_hip_server_destroy",
     "meshopt_hip_last_call_stats",
     "meshopt_hip_set_round_policy",
-    "meshopt_hip_reset_round_counts",
+    "meshopt_hip_set_adjacency_rebuild", "meshopt_hip_reset_round_counts",
     "meshopt_hip_last_error",
     "meshopt_hip_kernel_timing",
     "meshopt_hip_release",
@@ -524,6 +524,12 @@ def set_round_policy(deep_heads=-2, deep_from_head=8):
     lib = library()
     if lib.meshopt_hip_set_round_policy(int(deep_heads), int(deep_from_head)) != 0:
         raise ValueError(lib.meshopt_hip_last_error().decode())
+
+
+def set_adjacency_rebuild(enable):
+    """meshopt_hip_set_adjacency_rebuild: the calling thread's plain calls build their adjacency from
+    scratch after every pass."""
+    library().meshopt_hip_set_adjacency_rebuild(int(bool(enable)))
 
 
 def reset_round_counts():

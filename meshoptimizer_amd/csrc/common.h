@@ -125,7 +125,8 @@ struct CallScalars
 	uint32_t round;         // the commit rounds' base of the pass (list buffers rotate with the round number)
 	uint32_t epoch;         // the round tag before the base round (round minima are tagged, monotonic over the call)
 	uint32_t extend;        // 1 when the pass's first window held no break and the list goes on
-	uint32_t split;         // 1 when a pass took wedges of one class to different classes
+	uint32_t split;         // 1 when a pass took wedges of one class to different classes, or a class elsewhere
+	                        // than to its commit's target
 	uint32_t stop_done;     // workgroups of the stop scan that have left their record (0 between scans)
 	uint32_t pick_capacity; // boundEdgeCollapses (src/simplifier.cpp:1292-1308): pick stops before exceeding it
 	uint32_t work[8];     // small counters of setup kernels

@@ -580,6 +580,9 @@ static std::atomic<int> g_head_rounds[33];
 // the same for the extension window [W, C) of a pass
 static std::atomic<int> g_ext_head_rounds[33];
 
+// meshopt_hip_set_adjacency_rebuild, for the calling thread's calls
+static thread_local bool t_rebuild_adjacency;
+
 static int size_bucket(size_t n)
 {
 	int bucket = 0;
@@ -919,7 +922,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 		m.loop_cur ^= 1;
 		m.adj_cur ^= 1;
 		result_count = (size_t)h.next_triangles * 3;
-		if (h.split)
+		if (h.split || t_rebuild_adjacency)
 			launch_adjacency_ranges(s, m, h.next_triangles);
 
 		// components whose error fell under the pass's error (src/simplifier.cpp:2539-2541)
@@ -2699,6 +2702,13 @@ extern "C" int meshopt_hip_set_round_policy(int deep_heads, int deep_from_head)
 	}
 	g_deep_heads.store(deep_heads < -1 ? kDeepHeads : deep_heads);
 	g_deep_from_head.store(deep_from_head);
+	t_last_error.clear();
+	return 0;
+}
+
+extern "C" int meshopt_hip_set_adjacency_rebuild(int enable)
+{
+	t_rebuild_adjacency = enable != 0;
 	t_last_error.clear();
 	return 0;
 }

@@ -1892,9 +1892,10 @@ __device__ __forceinline__ uint32_t update_one(size_t k, const uint2* r_class, c
 //   - remaps its edge loops (remapEdgeLoops, src/simplifier.cpp:1845-1864): collapse_remap is
 //     idempotent within a pass (targets are locked, never sources), so reading loop[l] before or
 //     after its own update gives the same result and the in-place loop becomes a double-buffered map;
-//   - as a primary, leaves its class's new id and adds the room its adjacency may need to its tile;
-//     as a secondary, checks that its class moves as one (every wedge of a seam or complex class
-//     goes into the target class unless its loops were inconsistent).
+//   - as a primary, leaves its class's new id and adds the room its adjacency may need to its tile,
+//     and checks that a class that moves goes to its commit's target; as a secondary, checks that it
+//     goes where its primary does.  Both hold while a seam class's two loops name neighbours of one
+//     class, as the classification asks; no mesh is known where they stop to.
 struct ApplyArgs
 {
 	const uint8_t* status;
@@ -1948,6 +1949,7 @@ __device__ __forceinline__ uint32_t remap_loop(const ApplyArgs& a, const uint32_
 struct ClassLists
 {
 	uint2 own, other;
+	uint32_t target; // the class it is collapsed into (kNone: none)
 	__device__ __forceinline__ uint32_t room() const
 	{
 		return (own.y - own.x) + (other.y - other.x);
@@ -1959,14 +1961,18 @@ __device__ __forceinline__ ClassLists class_lists(const ApplyArgs& a, uint32_t v
 	ClassLists l;
 	l.own = a.range_in[v];
 	l.other = make_uint2(0, 0);
+	l.target = kNone;
 	const uint32_t k = a.lock_rank[v];
 	if (k < stop)
 	{
-		const uint32_t source = a.r_class[k].x;
-		if (source == v)
+		const uint2 c = a.r_class[k];
+		if (c.x == v)
+		{
 			l.own = make_uint2(0, 0);
+			l.target = c.y;
+		}
 		else
-			l.other = a.range_in[source];
+			l.other = a.range_in[c.x];
 	}
 	return l;
 }
@@ -2008,8 +2014,12 @@ __global__ void __launch_bounds__(kThreads) k_apply(ApplyArgs a)
 		const uint32_t r = a.remap[v];
 		if (r == v)
 		{
-			a.new_class[v] = a.remap[c];
-			room.x += class_lists(a, v, stop).room();
+			const uint32_t to = a.remap[c];
+			const ClassLists l = class_lists(a, v, stop);
+			a.new_class[v] = to;
+			room.x += l.room();
+			if (l.target != kNone && l.target != to)
+				a.sc->split = 1; // its list would go to another class than its vertices
 		}
 		else if (a.remap[c] != a.remap[settled_remap(a, r, stop)])
 			a.sc->split = 1; // this wedge went elsewhere than its primary: the lists by class do not hold
@@ -2044,7 +2054,7 @@ __global__ void __launch_bounds__(kThreads) k_adj_walk(ApplyArgs a)
 	for (uint32_t j = 0; j < a.items; ++j)
 	{
 		const uint32_t v = (blockIdx.x * a.items + j) * kThreads + threadIdx.x;
-		ClassLists l{make_uint2(0, 0), make_uint2(0, 0)};
+		ClassLists l{make_uint2(0, 0), make_uint2(0, 0), kNone};
 		if (v < a.vertices && a.remap[v] == v)
 			l = class_lists(a, v, stop);
 		const uint32_t room = l.room();

@@ -200,6 +200,28 @@ def test_round_policies(policy):
         M.set_round_policy()
 
 
+@pytest.mark.parametrize("seed", range(6))
+def test_adjacency_rebuild(seed):
+    """The adjacency built from scratch after every pass, which a pass does by itself only when a class's
+    wedges go to different classes, gives what the one carried over from pass to pass does: seamed
+    grids with and without attributes, soups with many wedges at a position, and pruned components."""
+    rng = np.random.default_rng(4400 + seed)
+    M.set_adjacency_rebuild(True)
+    try:
+        for k in range(6):
+            ib, v = (random_grid(rng, n=int(rng.integers(12, 48)), seams=int(rng.integers(0, 8))) if k % 3 else
+                     random_soup(rng, nv=int(rng.integers(50, 900)), ntri=int(rng.integers(100, 2000))))
+            target = (ib.size // 3 * int(rng.integers(0, 3)) // 4) * 3
+            announce(f"adjacency rebuild seed={seed} mesh {k} I={ib.size}")
+            assert_parity(ib, v, target, float(rng.choice([1e-2, 1e-1, 1.0])), OPTION_SETS[(6 * seed + k) % len(OPTION_SETS)])
+        ib, v = scattered_components(rng, 12)
+        assert_parity(ib, v, 0, 0.1, M.SimplifyPrune)
+        m = W.seamed_grid(40 + seed, seams=5)
+        assert_parity(m.indices, m.vertices, W.target_count(m.index_count, 1, 8), 1e-1, 0, m.vertices[:, 3:8], W.SEAMED_GRID_WEIGHTS)
+    finally:
+        M.set_adjacency_rebuild(False)
+
+
 @pytest.mark.parametrize("den,err,opts", [(20, 1e-2, 0), (100, 1.0, M.SimplifyLockBorder)])
 def test_window_extension(den, err, opts):
     """A pass whose first rank window holds no break goes on to the rest of the list on the device
