@@ -1819,21 +1819,28 @@ static int simplify_batch_on_device(Context& ctx, const BatchMemory& mem, unsign
 		}
 		ctx.ensure_aux_streams();
 		HIP_CHECK(hipEventRecord(ctx.fork_ev, s));
-		// when the host knows the index counts (host offsets, or the caller's host copy of them)
-		// and one of them lies within class 3's index caps only, class 3 launches at once beside
-		// the others instead; when every mesh is beyond class 2's index cap, classes 0-2 are empty
-		// and not launched
+		// when the host knows the sizes (host offsets, or the caller's host copy of the index offsets
+		// of meshes that have no more vertices than indices) and one of them is class 3's for sure,
+		// class 3 launches at once beside the others; when every mesh is beyond class 2's index cap,
+		// classes 0-2 are empty and not launched.  big_possible: some mesh may be class 3's
 		const int big = kBatchClasses - 1;
 		const unsigned int* known = h_index_offsets ? h_index_offsets : h_size_offsets;
-		bool small_empty = false, big_early = false;
+		bool small_empty = false, big_early = false, big_possible = classes.icap[big] != 0;
 		if (known && classes.icap[big])
 		{
 			small_empty = true;
+			big_possible = false;
 			for (size_t p = 0; p < P; ++p)
 			{
 				const size_t n = known[p + 1] - known[p];
+				const size_t v = h_vertex_offsets ? h_vertex_offsets[p + 1] - h_vertex_offsets[p] : n; // or at most n
 				small_empty &= n > classes.icap[big - 1];
-				big_early |= n > classes.icap[big - 1] && n <= classes.icap[big];
+				bool in_smaller = false;
+				for (int k = 0; k < big; ++k)
+					in_smaller |= n <= classes.icap[k] && v <= classes.vcap[k];
+				const bool index_fits = n <= classes.icap[big], certain = n > classes.icap[big - 1];
+				big_possible |= index_fits && !in_smaller;
+				big_early |= index_fits && (certain || (h_vertex_offsets && !in_smaller && v <= classes.vcap[big]));
 			}
 		}
 		// a class's workgroups: one per mesh slot (those past the class's count leave at once), or
@@ -1879,12 +1886,13 @@ static int simplify_batch_on_device(Context& ctx, const BatchMemory& mem, unsign
 		// class 3 does not wait for the others: its count comes to host memory as soon as the classifier
 		// has ended (about when the launches above are through), and its workgroups take the CUs that
 		// the others leave free.  Launched after the status read-back instead, 777 meshes of 20-1900
-		// triangles took 0.97 ms against 0.90
-		if (!big_early && mem.host_dev && classes.icap[big])
+		// triangles took 0.97 ms against 0.90 (three sets of inputs in turn; sets not seen before take 1.06).
+		// The host waits only where a mesh may be class 3's, and no longer than 200 us for work ahead
+		if (!big_early && mem.host_dev && big_possible)
 		{
 			const auto give_up = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
 			while (*h_large == kNotYet && std::chrono::steady_clock::now() < give_up)
-				;
+				__builtin_ia32_pause();
 			const uint32_t large = *h_large;
 			if (large != kNotYet && large)
 			{

@@ -151,6 +151,26 @@ def test_size_classes(opts, entry):
             check_batch_device(meshes, targets, 1e-2, opts)
 
 
+@pytest.mark.parametrize("entry", ["host", "device"])
+def test_largest_class_by_vertices(entry):
+    """Meshes of few indices that only the last class holds, for their vertices (most of them used by no
+    triangle), among small ones, alone, and with meshes of neither."""
+    with launch_shape() as shape:
+        vcaps = shape["vertex_caps"]
+        small, small_targets = patch_meshes(6, seed=3)
+        wide = []
+        for extra in (vcaps[2] + 1, vcaps[3]):
+            m = W.grid(12, seed=extra)
+            v = np.zeros((extra, 3), np.float32)
+            v[:m.vertices.shape[0]] = m.vertices[:, :3]
+            wide.append((m.indices, v))
+        beyond = (wide[0][0], np.zeros((vcaps[3] + 1, 3), np.float32))
+        for meshes, targets in ((small + wide, small_targets + [300, 0]), (wide, [0, 300]), (small, small_targets),
+                                (small + [beyond], small_targets + [0])):
+            announce(f"classes by vertices: {[(ib.size, v.shape[0]) for ib, v in meshes]}, {entry} entry")
+            (check_batch if entry == "host" else check_batch_device)(meshes, targets, 1e-2, 0)
+
+
 def test_sparse_batch():
     rng = np.random.default_rng(99)
     meshes, targets = [], []
