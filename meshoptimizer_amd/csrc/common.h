@@ -104,7 +104,7 @@ struct CallScalars
 	uint32_t skipped;
 	uint32_t rejected;
 	uint32_t secondary_count; // vertices that are not their class's primary
-	uint32_t long_lists;  // whether some vertex, or class, has too many corners for the all-pairs order (setup.hip)
+	uint32_t long_lists;  // whether the corner lists, by vertex or by class, are too long for the all-pairs order (setup.hip)
 	// The rounds' counters: three of the first row lie in the cache line before the others.  With the
 	// three rows in one line, where the XCDs' atomics meet, rounds took longer (1024 x 1024 seamed grid:
 	// the call 9.20 ms against 8.66).

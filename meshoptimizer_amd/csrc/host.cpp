@@ -428,7 +428,8 @@ struct Plan
 	uint32_t* v_b;
 	uint32_t* v_c;
 	uint32_t* v_d;
-	size_t off_words;
+	size_t off_words, clear_words;
+	uint32_t* class_steps;
 	uint32_t* raw_off;
 	uint32_t* raw_keys;
 	uint32_t* raw_corners;
@@ -522,10 +523,13 @@ static void carve(Arena& a, Plan& p, size_t V_in, size_t V, size_t I, size_t A, 
 	p.v_b = p.v_a + Vp;
 	p.v_c = m.lock_rank;
 	p.v_d = m.cremap;
-	// cleared together: the corner counts and the classes' counts of their secondaries' corners
+	// cleared together: the corner counts, the classes' counts of their secondaries' corners and their
+	// steps (launch_position_remap)
 	p.off_words = (Vp + 1 + 63) & ~size_t(63);
-	p.raw_off = a.take<uint32_t>(2 * p.off_words);
+	p.clear_words = 2 * p.off_words + p.off_words / 64;
+	p.raw_off = a.take<uint32_t>(p.clear_words);
 	p.w_off = p.raw_off + p.off_words;
+	p.class_steps = p.w_off + p.off_words;
 	p.raw_keys = reinterpret_cast<uint32_t*>(m.r_v);
 	p.raw_corners = p.raw_keys + cap;
 	p.w_keys = reinterpret_cast<uint32_t*>(m.r_class);
@@ -687,8 +691,8 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	t_read_backs = 0;
 	// one read-back after the checks and the position remap: the index check, the sparse remap's
 	// vertex count (which its own read-back brings earlier), the number of secondary vertices and
-	// whether there are long corner lists
-	launch_call_init(s, m.sc, plan.raw_off, 2 * plan.off_words);
+	// whether the corner lists are long
+	launch_call_init(s, m.sc, plan.raw_off, plan.clear_words);
 	launch_load_indices(s, c.indices, m.ib[0], I, V_in, sparse ? nullptr : plan.raw_off, plan.slot, &m.sc->work[2]);
 	auto check_indices = [&]() {
 		if (ctx.sc_host->work[2])
@@ -713,7 +717,7 @@ static size_t simplify_on_device(Context& ctx, const CallArgs& c, float* result_
 	launch_gather_positions(s, m, c.positions, c.position_stride / sizeof(float), sparse_remap, plan.table, table_size);
 	if (sparse)
 		launch_corner_count(s, m, nullptr, plan.raw_off, plan.slot);
-	launch_position_remap(s, m, plan.table, table_size, plan.raw_off, plan.w_off);
+	launch_position_remap(s, m, plan.table, table_size, plan.raw_off, plan.w_off, plan.class_steps);
 	sync_scalars(ctx, m);
 	check_indices();
 	const size_t secondaries = ctx.sc_host->secondary_count;

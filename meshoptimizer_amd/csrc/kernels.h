@@ -93,8 +93,10 @@ void launch_gather_positions(hipStream_t s, Mesh& m, const float* positions, siz
 // adds the corners of each vertex (remap null) or class to its count, and says which of them each is
 void launch_corner_count(hipStream_t s, Mesh& m, const uint32_t* remap, uint32_t* counts, uint32_t* slot);
 // m.remap, m.pos, sc->secondary_count; wedge rings of one vertex each and empty round minima.
-// sc->long_lists from the corners per vertex (counts); class_extra: V zero words
-void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size, const uint32_t* counts, uint32_t* class_extra);
+// sc->long_lists from the corners per vertex (counts); class_extra and class_steps: zero words, one a
+// vertex and one for 64 of them
+void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size, const uint32_t* counts, uint32_t* class_extra,
+                           uint32_t* class_steps);
 // the wedge rings of the classes with secondaries (their count as read back)
 void launch_wedges(hipStream_t s, Mesh& m, size_t secondaries, uint32_t* flags, uint32_t* scratch_a, uint32_t* scratch_b, uint32_t* scratch_c, uint32_t* scratch_d);
 // each vertex's corners in corner order (offsets: V + 1 words, the counts on entry, with the slots

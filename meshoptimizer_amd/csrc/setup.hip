@@ -273,14 +273,23 @@ void launch_rescale(hipStream_t s, Mesh& m)
 }
 
 // ------------------------------------------------------------------------------------------
-// Corner lists of more than kAllPairs corners are long.  Up to it a wavefront compares every corner of a
-// list with every other (k_corner_order); beyond it the lists of the mesh are made by sorts, and the
-// open edges of the long ones by a table, linear in the corners.  The two meet at 250-300 corners
-// (calls on a hub of 400 beside 200 triangles 835 us by pairs, 699 sorted; beside 320 thousand 2657 and
-// 2533; of 200 corners 565 and 570, 2483 and 2551); by pairs, the 300 thousand corners that padding
-// with (0,0,0) triangles gives a vertex would take half a minute.
-constexpr uint32_t kAllPairs = 256;
-constexpr uint32_t kLongVertexList = 1, kLongClassList = 2; // of CallScalars::long_lists
+// k_corner_order compares every corner of a list of more than kNet with every other, in the wavefront
+// that has the list: pair_steps of its loop, one list after the other.  Where one wavefront's lists come
+// to more than kPairSteps, the mesh's lists are made by sorts instead, and the open edges of all lists
+// above kNet by a table, linear in the corners.  The two meet at 1000-1400 steps (calls on a hub of 400
+// corners, 2500 steps, beside 200 triangles 835 us by pairs, 699 sorted; beside 320 thousand 2657 and
+// 2533; on a hub of 200, 625 steps, 565 and 570, 2483 and 2551; 64 positions of 140 corners each, whose
+// primaries are neighbours: 1441 us by pairs).  By pairs, the 300 thousand corners that padding with
+// (0,0,0) triangles gives a vertex would take half a minute.
+constexpr int kNet = 8; // corners that the sorting network takes
+constexpr uint32_t kPairSteps = 1280;
+constexpr uint32_t kLongVertexLists = 1, kLongClassLists = 2; // of CallScalars::long_lists
+
+__device__ __forceinline__ uint32_t pair_steps(uint32_t corners)
+{
+	const uint32_t c = corners < 65536 ? corners : 65536; // far beyond kPairSteps
+	return c <= kNet ? 0 : (c <= 64 ? c : (uint32_t)((uint64_t)c * c / 64));
+}
 
 // position remap (src/simplifier.cpp:111-240).  remap[i] = lowest index whose xyz compare
 // equal as floats (+0 == -0; NaN equals nothing).  Linear-probing table keyed by the
@@ -335,12 +344,12 @@ __global__ void k_hash_insert(const float4* pos, size_t n, uint32_t* table, uint
 }
 
 // each vertex's primary, its rescaled position, a wedge ring of its own and no pending ranks; sc
-// counts the secondaries and says whether any corner list is long (kAllPairs): a vertex's own from
-// its corner count, a class's from its primary's count and the sum over its secondaries, so a class
-// that is not reported has at most 2 * kAllPairs corners
+// counts the secondaries and says whether the corner lists are long (kPairSteps).  By vertex, a
+// wavefront here holds the counts of one there; by class, every secondary adds its corners to its
+// class, and what that adds to the steps of the class to those of the wavefront with the primary
 __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, size_t n, const uint32_t* table, uint32_t mask, uint32_t* remap,
                                                           uint32_t* wedge, float4* pos, ulonglong2* pend0, ulonglong2* pend1, const uint32_t* counts,
-                                                          uint32_t* class_extra, CallScalars* sc)
+                                                          uint32_t* class_extra, uint32_t* class_steps, CallScalars* sc)
 {
 	__shared__ uint32_t secondaries;
 	if (threadIdx.x == 0)
@@ -348,7 +357,8 @@ __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, si
 	__syncthreads();
 	const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	uint32_t result = (uint32_t)i;
-	uint32_t corners = 0, in_class = 0;
+	uint32_t corners = 0, own_steps = 0;
+	bool long_class = false;
 	if (i < n)
 	{
 		corners = counts[i];
@@ -375,13 +385,32 @@ __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, si
 		// round minima start as "no entry" (tag of epoch 0, rank all-ones)
 		pend0[i] = make_ulonglong2(~0ull, ~0ull);
 		pend1[i] = make_ulonglong2(~0ull, ~0ull);
-		in_class = corners;
+		own_steps = pair_steps(corners);
 		if (result != (uint32_t)i && corners)
-			in_class += atomicAdd(&class_extra[result], corners);
+		{
+			const uint32_t before = counts[result] + atomicAdd(&class_extra[result], corners);
+			const uint32_t more = pair_steps(before + corners) - pair_steps(before);
+			long_class = more && atomicAdd(&class_steps[result / 64], more) + more > kPairSteps;
+		}
 	}
-	const uint64_t long_vertex = __ballot(corners > kAllPairs), long_class = __ballot(in_class > kAllPairs);
-	if (long_class && __lane_id() == 0)
-		atomicOr(&sc->long_lists, (long_vertex ? kLongVertexList : 0u) | kLongClassList);
+	if (__ballot(own_steps != 0))
+	{
+		// the primaries' own part of the classes' steps, and this wavefront's by vertex
+		uint32_t primary = result == (uint32_t)i ? own_steps : 0;
+		for (int o = 32; o > 0; o >>= 1)
+		{
+			own_steps += __shfl_xor(own_steps, o, 64);
+			primary += __shfl_xor(primary, o, 64);
+		}
+		if (__lane_id() == 0)
+		{
+			long_class |= primary && atomicAdd(&class_steps[i / 64], primary) + primary > kPairSteps;
+			if (own_steps > kPairSteps)
+				atomicOr(&sc->long_lists, kLongVertexLists);
+		}
+	}
+	if (__ballot(long_class) && __lane_id() == 0)
+		atomicOr(&sc->long_lists, kLongClassLists);
 	const uint64_t second = __ballot(result != (uint32_t)i);
 	if (second && __lane_id() == 0)
 		atomicAdd(&secondaries, (uint32_t)__popcll(second));
@@ -390,7 +419,8 @@ __global__ void __launch_bounds__(kThreads) k_hash_lookup(const float4* praw, si
 		atomicAdd(&sc->secondary_count, secondaries);
 }
 
-void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size, const uint32_t* counts, uint32_t* class_extra)
+void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table_size, const uint32_t* counts, uint32_t* class_extra,
+                           uint32_t* class_steps)
 {
 	size_t n = m.vertex_count;
 	if (!n)
@@ -398,7 +428,7 @@ void launch_position_remap(hipStream_t s, Mesh& m, uint32_t* table, size_t table
 	k_hash_insert<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1));
 	k_hash_lookup<<<grid_for(n), kThreads, 0, s>>>(m.praw, n, table, (uint32_t)(table_size - 1), m.remap, m.wedge, m.pos,
 	                                               reinterpret_cast<ulonglong2*>(m.pend[0]), reinterpret_cast<ulonglong2*>(m.pend[1]), counts, class_extra,
-	                                               m.sc);
+	                                               class_steps, m.sc);
 }
 
 // wedge rings: for a class r < a_1 < ... < a_m, wedge[r] = a_m, wedge[a_k] = a_{k-1}, wedge[a_1] = r
@@ -455,8 +485,8 @@ void launch_wedges(hipStream_t s, Mesh& m, size_t secondaries, uint32_t* flags, 
 // eight corners by a sorting network in registers, more by the wavefront, every corner's place the
 // number of smaller ones.  (Sorting all corners by vertex with three radix digits took 370 us for
 // the 3.9 M of icosphere L8 and the open edges 140; lists and open edges now take 300 with the index
-// copy and check, 250 of it the count's and the placement's scattered words.)  Meshes with a long list
-// (kAllPairs) do take that sort, and a table of edges answers for the long lists' open ones.
+// copy and check, 250 of it the count's and the placement's scattered words.)  Meshes with long lists
+// (kPairSteps) do take that sort, and a table of edges answers for the open ones.
 
 __global__ void k_corner_count(const uint32_t* ib, size_t n, const uint32_t* remap, uint32_t* counts, uint32_t* slot)
 {
@@ -520,7 +550,6 @@ __device__ __forceinline__ uint32_t open_end(uint32_t v, bool self, uint32_t cou
 template <bool kOpen>
 __global__ void __launch_bounds__(kThreads) k_corner_order(CornerArgs a)
 {
-	constexpr int kNet = 8;
 	const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
 	const uint32_t v = (uint32_t)i, lane = __lane_id();
 	const uint32_t b = i < a.n ? a.off[i] : 0, e = i < a.n ? a.off[i + 1] : 0, len = e - b;
@@ -582,7 +611,7 @@ __global__ void __launch_bounds__(kThreads) k_corner_order(CornerArgs a)
 	}
 	if (kOpen && len > a.longest)
 	{
-		// a sorted list; k_long_edges finds its open edges, starting from none
+		// a sorted list; k_table_edges finds its open edges, starting from none
 		a.openout[v] = kNone;
 		a.openinc[v] = kNone;
 	}
@@ -641,7 +670,7 @@ __global__ void __launch_bounds__(kThreads) k_corner_order(CornerArgs a)
 	}
 }
 
-// Lists by sorting, for meshes with a long one: every corner's vertex as the key, its place as the
+// Lists by sorting, for meshes with long ones: every corner's vertex as the key, its place as the
 // value, both arrays in `corners` and `keys` and the sort's other halves in the candidate lists.
 // The time is linear in the corners (a sweep per byte of the vertex ids).
 
@@ -663,7 +692,7 @@ static void sort_corners(hipStream_t s, Mesh& m, const uint32_t* remap, uint32_t
 	radix_sort_pairs(s, keys, corners, keys_alt, vals_alt, n, nullptr, std::max(1, key_bits(m.vertex_count)), m.temp, true);
 }
 
-// Open edges of the long lists, the rule of k_corner_order: a table holds the directed edges at
+// Open edges of sorted lists above kNet, the rule of k_corner_order: a table holds the directed edges at
 // their vertices, two per corner, and each corner looks for the opposites of its own two.  The
 // candidate lists hold the table: 4 * (I + 4) slots, rounded down to a power of two, for at most I
 // different edges, so that every search ends at an empty slot soon.
@@ -722,7 +751,7 @@ __device__ __forceinline__ void open_add(uint32_t* open, uint32_t v, uint32_t en
 }
 
 template <bool kInsert>
-__global__ void k_long_edges(CornerArgs a, size_t n, EdgeTable t)
+__global__ void k_table_edges(CornerArgs a, size_t n, EdgeTable t)
 {
 	size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (j >= n)
@@ -757,7 +786,7 @@ __global__ void k_list_neighbours(const uint32_t* ib, const uint32_t* corners, s
 		adj[p] = corner_neighbours(ib, corners[p]);
 }
 
-static void long_open_edges(hipStream_t s, Mesh& m, const CornerArgs& a)
+static void table_open_edges(hipStream_t s, Mesh& m, const CornerArgs& a)
 {
 	const size_t n = m.index_count;
 	size_t slots = 1;
@@ -765,8 +794,8 @@ static void long_open_edges(hipStream_t s, Mesh& m, const CornerArgs& a)
 		slots *= 2;
 	const EdgeTable t{reinterpret_cast<unsigned long long*>(m.list[0]), (uint32_t)(slots - 1)};
 	fill_u32(s, reinterpret_cast<uint32_t*>(t.slots), kNone, 2 * slots);
-	k_long_edges<true><<<grid_for(n), kThreads, 0, s>>>(a, n, t);
-	k_long_edges<false><<<grid_for(n), kThreads, 0, s>>>(a, n, t);
+	k_table_edges<true><<<grid_for(n), kThreads, 0, s>>>(a, n, t);
+	k_table_edges<false><<<grid_for(n), kThreads, 0, s>>>(a, n, t);
 	if (a.adj)
 		k_list_neighbours<<<grid_for(n), kThreads, 0, s>>>(m.ib[0], a.corners, n, a.adj);
 }
@@ -788,17 +817,17 @@ void launch_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, bool with_
 {
 	if (!m.vertex_count)
 		return;
-	const bool sorted = (long_lists & kLongVertexList) != 0;
+	const bool sorted = (long_lists & kLongVertexLists) != 0;
 	corner_offsets(s, m, offsets);
 	if (sorted)
 		sort_corners(s, m, nullptr, placed, corners);
 	else if (m.index_count)
 		k_corner_place<<<grid_for(m.index_count), kThreads, 0, s>>>(m.ib[0], m.index_count, nullptr, offsets, slot, placed);
 	const CornerArgs a{m.ib[0],   offsets, sorted ? corners : placed, corners, m.loop[0], m.loopback[0], with_adjacency ? m.adj[1] : nullptr,
-	                   m.vertex_count, sorted ? kAllPairs : kNone};
+	                   m.vertex_count, sorted ? (uint32_t)kNet : kNone};
 	k_corner_order<true><<<grid_for(m.vertex_count), kThreads, 0, s>>>(a);
 	if (sorted)
-		long_open_edges(s, m, a);
+		table_open_edges(s, m, a);
 }
 
 void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, uint32_t* offsets, uint32_t* slot, uint32_t* placed, uint32_t* corners)
@@ -808,7 +837,7 @@ void launch_welded_corner_lists(hipStream_t s, Mesh& m, uint32_t long_lists, uin
 	fill_u32(s, offsets, 0, (size_t)m.vertex_count + 1);
 	launch_corner_count(s, m, m.remap, offsets, slot);
 	corner_offsets(s, m, offsets);
-	if (long_lists & kLongClassList)
+	if (long_lists & kLongClassLists)
 	{
 		sort_corners(s, m, m.remap, placed, corners);
 		return;

@@ -110,16 +110,25 @@ def long_list_case(name, rng):
         tri = np.concatenate([ib.reshape(-1, 3), tri])
         v = np.concatenate([v, np.full((size, 3), 0.37, np.float32)]).astype(np.float32)
         return tri[rng.permutation(len(tri))].reshape(-1).astype(np.uint32), v
+    if kind == "snapped":
+        # few positions of many vertices, the primaries neighbours in index order
+        v = (np.floor(rng.random((size, 3)) * 4) / 4).astype(np.float32)
+        return rng.integers(0, size, size * 9).astype(np.uint32), v
+    if kind == "strips":
+        # vertices of about 20 corners, all in one wavefront's lists or not
+        return (rng.integers(0, size, (size * 20 // 3, 3)).reshape(-1).astype(np.uint32), rng.random((size, 3)).astype(np.float32))
     # every list long, with edges repeated and self edges
     return rng.integers(0, 37, (size, 3)).reshape(-1).astype(np.uint32), rng.random((37, 3)).astype(np.float32)
 
 
-@pytest.mark.parametrize("name", ["padding84", "padding85", "padding7000", "fan255", "fan256", "fan257", "fan513", "fan4000", "fan4001",
-                                  "soupfan255", "soupfan256", "soupfan257", "soupfan513", "soupfan3000", "soupfan3001", "point255",
-                                  "point257", "point513", "point6000", "dense3100", "dense20000"])
+@pytest.mark.parametrize("name", ["padding84", "padding95", "padding96", "padding7000", "fan255", "fan257", "fan285", "fan288", "fan513", "fan4000", "fan4001",
+                                  "soupfan255", "soupfan257", "soupfan285", "soupfan288", "soupfan513", "soupfan3000", "soupfan3001", "point255",
+                                  "point285", "point287", "point513", "point6000", "dense3100", "dense20000", "snapped300", "snapped1000",
+                                  "snapped4000", "strips40", "strips64", "strips70", "strips500"])
 def test_long_corner_lists(name):
-    """Corner lists and open edges around the length from which lists are sorted and edges come from a
-    table, by vertex and by class, in every option that reads them."""
+    """Corner lists and open edges around the work from which lists are sorted and edges come from a
+    table, in one list and in many of one wavefront, by vertex and by class, in every option that
+    reads them."""
     rng = np.random.default_rng(len(name) + int("".join(c for c in name if c.isdigit())))
     ib, v = long_list_case(name, rng)
     a, w = rng.random((v.shape[0], 2)).astype(np.float32), np.array([0.3, 0.1], np.float32)
