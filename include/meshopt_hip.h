@@ -143,7 +143,8 @@ typedef struct meshopt_hip_call_stats
 	                                outcomes not decided from their neighbours' possible positions) */
 	unsigned int solve_rounds;   /* rounds of the ordered position solve */
 	unsigned int read_backs;     /* host synchronisations with the device during the call */
-	unsigned int device_extensions; /* passes whose rank window was extended to the whole list */
+	unsigned int device_extensions; /* passes whose rank window held no break and was extended to the whole
+	                                list, after a read-back of its own */
 } meshopt_hip_call_stats;
 
 /* Copies up to max_passes pass records of the calling thread's last call; returns the pass count. */

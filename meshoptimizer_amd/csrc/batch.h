@@ -50,9 +50,8 @@ struct BatchArgs
 // The launch shape of the size classes: per class, the workgroups that share one CU (the class's
 // LDS share is the CU's 160 KB over that count), the threads per workgroup (128, 256, 512 or 1024), and
 // whether its workgroups take meshes from a cursor (grid: per_cu workgroups per CU) instead of one
-// workgroup per mesh.  The last class always runs from a cursor and launches after the status
-// read-back (unless the host knows a mesh in its range).  The default comes from the LDS budget;
-// a measured one (meshoptimizer_amd/tune.py) may replace it.
+// workgroup per mesh.  The last class always runs from a cursor and is launched on its own, once the
+// host knows that it has meshes.  The default comes from the LDS budget; a measured one (meshoptimizer_amd/tune.py) may replace it.
 struct BatchShape
 {
 	uint32_t per_cu[kBatchClasses];

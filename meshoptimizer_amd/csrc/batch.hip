@@ -99,7 +99,7 @@ __device__ __forceinline__ int batch_mesh_class(const BatchArgs& a, const BatchC
 	if (cls < 0)
 		status = 1; // too large for the LDS layouts: the plain path
 	else if (cls == kBatchClasses - 1)
-		status = 6; // runs after the other classes (its workgroup takes a whole CU)
+		status = 6; // until it runs: its class is launched on its own (its workgroup takes a whole CU)
 	return cls;
 }
 

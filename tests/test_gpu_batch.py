@@ -125,8 +125,8 @@ def test_size_classes(opts, entry):
     5 workgroups per CU), seamed grids of 2400-2904 indices (2 per CU) and 300 of 4056-5400
     indices (one workgroup per CU with the whole LDS, taking meshes from a cursor: more of them
     than CUs), and one of 6534 indices beyond every class (the plain path).  The host entry knows
-    the sizes and launches the largest class beside the others; the device entry launches it
-    after the status read-back."""
+    the sizes and launches the largest class before the others; the device entry once the
+    classifier's count has arrived, or after the status read-back."""
     rng = np.random.default_rng(4242 + opts)
     meshes, targets = patch_meshes(40, seed=31)
     for k in range(320):

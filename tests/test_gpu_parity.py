@@ -224,9 +224,9 @@ def test_adjacency_rebuild(seed):
 
 @pytest.mark.parametrize("den,err,opts", [(20, 1e-2, 0), (100, 1.0, M.SimplifyLockBorder)])
 def test_window_extension(den, err, opts):
-    """A pass whose first rank window holds no break goes on to the rest of the list on the device
-    (the extension window, with its own head rounds and tail): icosphere L6 at a low target opens
-    one; the result matches the oracle."""
+    """A pass whose first rank window holds no break goes on to the rest of the list (the extension
+    window, opened by the host, with its own head rounds and tail): icosphere L6 at a low target
+    opens one; the result matches the oracle."""
     m = W.icosphere(6)
     target = W.target_count(m.index_count, 1, den)
     announce(f"window extension icosphere6 target 1/{den} err {err} opts {opts}")
