@@ -287,8 +287,9 @@ constexpr uint32_t kLongVertexLists = 1, kLongClassLists = 2; // of CallScalars:
 
 __device__ __forceinline__ uint32_t pair_steps(uint32_t corners)
 {
-	const uint32_t c = corners < 65536 ? corners : 65536; // far beyond kPairSteps
-	return c <= kNet ? 0 : (c <= 64 ? c : (uint32_t)((uint64_t)c * c / 64));
+	// capped far beyond kPairSteps, so that the sum over a wavefront stays in 32 bits
+	const uint32_t c = corners < 4096 ? corners : 4096;
+	return c <= kNet ? 0 : (c <= 64 ? c : c * c / 64);
 }
 
 // position remap (src/simplifier.cpp:111-240).  remap[i] = lowest index whose xyz compare

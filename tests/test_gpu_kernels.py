@@ -117,6 +117,10 @@ def long_list_case(name, rng):
     if kind == "strips":
         # vertices of about 20 corners, all in one wavefront's lists or not
         return (rng.integers(0, size, (size * 20 // 3, 3)).reshape(-1).astype(np.uint32), rng.random((size, 3)).astype(np.float32))
+    if kind == "crowd":
+        # the lists of one wavefront, each of more than `size` corners
+        ib = np.concatenate([np.repeat(np.arange(64), size), rng.integers(0, 64, 64 * size * 2)]).astype(np.uint32)
+        return np.ascontiguousarray(ib.reshape(3, -1).T).reshape(-1), rng.random((64, 3)).astype(np.float32)
     # every list long, with edges repeated and self edges
     return rng.integers(0, 37, (size, 3)).reshape(-1).astype(np.uint32), rng.random((37, 3)).astype(np.float32)
 
@@ -143,11 +147,12 @@ def test_long_corner_lists(name):
         assert same_bits(eg, eo), (eg, eo)
 
 
-@pytest.mark.parametrize("name", ["padding100000", "point100000"])
+@pytest.mark.parametrize("name", ["padding100000", "point100000", "crowd22000"])
 def test_long_corner_lists_time(name):
-    """A list of a hundred thousand corners or more costs time linear in it (its pairs would take many
-    seconds)."""
+    """A list of a hundred thousand corners or more, and 64 such lists, cost time linear in them (their
+    pairs would take many seconds)."""
     ib, v = long_list_case(name, np.random.default_rng(5))
+    assert name[:5] != "crowd" or np.bincount(ib).min() >= 65536
     M.simplify(ib, v, ib.size // 12 * 3, 1e-3, 0)
     announce(f"long lists {name}")
     t = time.perf_counter()
